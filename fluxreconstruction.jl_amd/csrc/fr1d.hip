@@ -5,7 +5,9 @@
 // of T threads owns element first-1+t, so lanes 0 and T-1 are halo elements that only provide
 // their face traces; the T-2 interior lanes produce du.  Traces and interface fluxes go through
 // LDS.  A single problem is a work list of its chunks; an ensemble is the concatenated work list
-// of all members (any degree 1..4 per member) processed by a persistent grid.
+// of all members (any degree 1..8 per member) processed by a persistent grid.  Stepping keeps the
+// elements of a chunk in registers over several steps (fr1d_block_kernel); a launch per stage over
+// the chunks (fr1d_kernel) gives the same bits and serves the residual, Tsit5 and the forced paths.
 #include <algorithm>
 #include <cmath>
 #include <cstring>
@@ -14,21 +16,23 @@
 #include <vector>
 
 #include "fr_common.h"
+#include "fr_ops_table.h"
 #include "fr_tsit5.h"
 
 namespace fr {
 
 constexpr int NSP_MAX = 9;  // degrees 1..8 (example/euler_highlevel.jl runs degree 7)
-// device operator table: entry nsp (2..NSP_MAX) at OPS_STRIDE*(nsp-2):
-// ll lr dhl dhr [NSP_MAX each] dl [NSP_MAX^2] | w/2 [NSP_MAX] (Gauss weights summing to one)
-// V1 iV1 [NSP_MAX^2 each]
-constexpr int OFF_W = 4 * NSP_MAX + NSP_MAX * NSP_MAX;
-constexpr int OFF_V = OFF_W + NSP_MAX, OFF_IV = OFF_V + NSP_MAX * NSP_MAX;
-constexpr int OPS_STRIDE = OFF_IV + NSP_MAX * NSP_MAX;
+// The operators that do not depend on the correction function are compile-time constants
+// (StdOps1D); the device table holds dhl, dhr [NSP_MAX each] of nsp (2..NSP_MAX) at
+// OPS_STRIDE*(nsp-2).  With all operators in the table, or the literals hoisted out of the step
+// loops (Makefile), the register-resident kernel spilled up to 1400 scalar values into lanes of
+// vector registers: 40 against 34 us per step on 512 members of p = 2..4.
+constexpr int OPS_STRIDE = 2 * NSP_MAX;
 struct Prob1D {
   long long off;  // first double of the member in the concatenated state
   int ncell, nsp;
   double iJ;      // 2/dx
+  double cut;     // shock_cut of the member's degree
 };
 
 struct Work1D {
@@ -51,6 +55,78 @@ struct Phys1D {
   double g, gm1, a;
 };
 
+// The arithmetic of one element, shared by the launch-per-stage and the register-resident kernels
+// (the same code in both, so both give the same bits; the sums are written as fma chains, since which
+// of two products the compiler fuses depends on where else a product with the same literal is used).
+
+// discontinuous flux f = F(u) / J, traces of u and f on the element's two faces
+template <int NSP, int EQ, int NV>
+__device__ __forceinline__ void elem_traces(const double (&w)[NSP][NV], double iJ, const Phys1D &ph, double (&f)[NSP][NV],
+                                            double (&uL)[NV], double (&uR)[NV], double (&fL)[NV], double (&fR)[NV]) {
+  constexpr StdOps1D<NSP> o{};
+#pragma unroll
+  for (int p = 0; p < NSP; ++p) {
+    if constexpr (EQ == FR_EQ_EULER) {
+      const double r = 1.0 / w[p][0];
+      const double vel = w[p][1] * r;
+      const double pr = ph.gm1 * (w[p][2] - 0.5 * w[p][1] * vel);
+      f[p][0] = w[p][1] * iJ;
+      f[p][1] = (w[p][1] * vel + pr) * iJ;
+      f[p][2] = ((w[p][2] + pr) * vel) * iJ;
+    } else {
+      f[p][0] = ph.a * w[p][0] * iJ;
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < NV; ++k) {
+    double a = 0, b = 0, c = 0, d = 0;
+#pragma unroll
+    for (int q = 0; q < NSP; ++q) {
+      a = fma(w[q][k], o.ll[q], a);
+      b = fma(w[q][k], o.lr[q], b);
+      c = fma(f[q][k], o.ll[q], c);
+      d = fma(f[q][k], o.lr[q], d);
+    }
+    uL[k] = a;
+    uR[k] = b;
+    fL[k] = c;
+    fR[k] = d;
+  }
+}
+
+// interface flux over J on the element's left face: the left neighbour's right traces (ul, fl; fl
+// for advection only), the own left traces; wrap marks the face between the last and first element
+template <int EQ, int FLUX, int NV>
+__device__ __forceinline__ void elem_face(const double (&ul)[NV], double fl, const double (&uL)[NV],
+                                          const double (&fL)[NV], bool wrap, double iJ, const Phys1D &ph,
+                                          double (&fs)[NV]) {
+  if constexpr (EQ == FR_EQ_EULER) {
+    double fw[3];
+    riemann_x3<FLUX>(ul, uL, ph.g, ph.gm1, fw);
+    // the reference divides the interface flux by J in the correction
+#pragma unroll
+    for (int k = 0; k < 3; ++k) fs[k] = fw[k] * iJ;
+  } else {
+    // regularised local Lax-Friedrichs of eq_advection.jl:128-137 (+1e-6 on the periodic face
+    // :163); f is already divided by J
+    const double eps = wrap ? 1e-6 : 1e-8;
+    const double au = (fL[0] - fl) / (uL[0] - ul[0] + eps);
+    fs[0] = 0.5 * (fL[0] + fl) - 0.5 * fabs(au) * (uL[0] - ul[0]);
+  }
+}
+
+// du of point p, variable k from the corrections cl, cr (interface flux minus own trace) of k; ops:
+// dhl, dhr of the element's nsp
+template <int NSP, int NV>
+__device__ __forceinline__ double elem_du(const double (&f)[NSP][NV], const double *__restrict__ ops, int p, int k,
+                                          double cl, double cr) {
+  constexpr StdOps1D<NSP> o{};
+  double d = 0.0;
+#pragma unroll
+  for (int q = 0; q < NSP; ++q) d = fma(f[q][k], o.dl[p + NSP * q], d);
+  return -fma(cr, ops[NSP_MAX + p], fma(cl, ops[p], d));
+}
+
 template <int NSP, int EQ, int FLUX>
 __device__ __forceinline__ void chunk1d(const Prob1D &pb, int first, const double *__restrict__ ops,
                                         const Phys1D &ph, const Stage1D &sa, double *sh) {
@@ -58,8 +134,6 @@ __device__ __forceinline__ void chunk1d(const Prob1D &pb, int first, const doubl
   const int T = blockDim.x;
   const int tid = threadIdx.x;
   const int n = pb.ncell;
-  const double *ll = ops, *lr = ops + NSP_MAX, *dhl = ops + 2 * NSP_MAX, *dhr = ops + 3 * NSP_MAX,
-               *dl = ops + 4 * NSP_MAX;
   // shared layout: uR[NV][T] | fR[NV][T] | Fs[NV][T]
   double *sUR = sh, *sFR = sh + NV * T, *sFS = sh + 2 * NV * T;
   int e = first - 1 + tid;
@@ -78,60 +152,25 @@ __device__ __forceinline__ void chunk1d(const Prob1D &pb, int first, const doubl
   for (int k = 0; k < NV; ++k)
 #pragma unroll
     for (int p = 0; p < NSP; ++p) w[p][k] = valid ? u[e + (long long)n * (p + NSP * k)] : (k == 0 ? 1.0 : (k == 2 ? 2.5 : 0.0));
-  // discontinuous flux f = F(u) / J, traces of u and f
   double f[NSP][NV], uL[NV], uR[NV], fL[NV], fR[NV];
-#pragma unroll
-  for (int p = 0; p < NSP; ++p) {
-    if constexpr (EQ == FR_EQ_EULER) {
-      const double r = 1.0 / w[p][0];
-      const double vel = w[p][1] * r;
-      const double pr = ph.gm1 * (w[p][2] - 0.5 * w[p][1] * vel);
-      f[p][0] = w[p][1] * pb.iJ;
-      f[p][1] = (w[p][1] * vel + pr) * pb.iJ;
-      f[p][2] = ((w[p][2] + pr) * vel) * pb.iJ;
-    } else {
-      f[p][0] = ph.a * w[p][0] * pb.iJ;
-    }
-  }
+  elem_traces<NSP, EQ, NV>(w, pb.iJ, ph, f, uL, uR, fL, fR);
 #pragma unroll
   for (int k = 0; k < NV; ++k) {
-    double a = 0, b = 0, c = 0, d = 0;
-#pragma unroll
-    for (int q = 0; q < NSP; ++q) {
-      a += w[q][k] * ll[q];
-      b += w[q][k] * lr[q];
-      c += f[q][k] * ll[q];
-      d += f[q][k] * lr[q];
-    }
-    uL[k] = a;
-    uR[k] = b;
-    fL[k] = c;
-    fR[k] = d;
-    sUR[k * T + tid] = b;
-    sFR[k * T + tid] = d;
+    sUR[k * T + tid] = uR[k];
+    sFR[k * T + tid] = fR[k];
   }
   __syncthreads();
   // interface flux on the left face of the own element (face between e-1 and e)
   if (tid >= 1 && valid) {
     const bool nb_ok = (ph.bc == FR_BC1_PERIOD) || (first - 2 + tid) >= 0;
     if (nb_ok) {
-      if constexpr (EQ == FR_EQ_EULER) {
-        double wl[3], fw[3];
+      double ul[NV], fs[NV];
 #pragma unroll
-        for (int k = 0; k < 3; ++k) wl[k] = sUR[k * T + tid - 1];
-        riemann_x3<FLUX>(wl, uL, ph.g, ph.gm1, fw);
-        // the reference divides the interface flux by J in the correction
+      for (int k = 0; k < NV; ++k) ul[k] = sUR[k * T + tid - 1];
+      const int ge = first - 1 + tid;  // global element right of the face
+      elem_face<EQ, FLUX, NV>(ul, sFR[tid - 1], uL, fL, ge == 0 || ge == n, pb.iJ, ph, fs);
 #pragma unroll
-        for (int k = 0; k < 3; ++k) sFS[k * T + tid] = fw[k] * pb.iJ;
-      } else {
-        // regularised local Lax-Friedrichs of eq_advection.jl:128-137 (+1e-6 on the periodic face
-        // :163); f is already divided by J
-        const double fl = sFR[tid - 1], ul = sUR[tid - 1];
-        const int ge = first - 1 + tid;  // global element right of the face
-        const double eps = (ge == 0 || ge == n) ? 1e-6 : 1e-8;
-        const double au = (fL[0] - fl) / (uL[0] - ul + eps);
-        sFS[tid] = 0.5 * (fL[0] + fl) - 0.5 * fabs(au) * (uL[0] - ul);
-      }
+      for (int k = 0; k < NV; ++k) sFS[k * T + tid] = fs[k];
     }
   }
   __syncthreads();
@@ -145,10 +184,7 @@ __device__ __forceinline__ void chunk1d(const Prob1D &pb, int first, const doubl
       const double cr = sFS[k * T + tid + 1] - fR[k];
 #pragma unroll
       for (int p = 0; p < NSP; ++p) {
-        double d = 0.0;
-#pragma unroll
-        for (int q = 0; q < NSP; ++q) d += f[q][k] * dl[p + NSP * q];
-        double du = -(d + cl * dhl[p] + cr * dhr[p]);
+        double du = elem_du<NSP, NV>(f, ops, p, k, cl, cr);
         if (zero) du = 0.0;
         const long long idx = ge + (long long)n * (p + NSP * k);
         if (sa.residual) {
@@ -211,15 +247,12 @@ __global__ __launch_bounds__(256) void fr1d_kernel(const Prob1D *__restrict__ pr
 //          mean, then the pressure squeeze with the closed-form tj_equation root).
 // count[0] += flagged (mode 1) / limited (mode 2) cells, count[1] += cells whose density
 // assert failed (left untouched).
+// Returns whether the values x of the cell were replaced; cut: Prob1D::cut.
+constexpr double kKappa1D = 4.0;  // example/euler_highlevel.jl:42
 template <int NSP>
-__device__ __forceinline__ void diss1d_cell(double *__restrict__ u, long long n, long long e, const double *ops,
-                                            int mode, double g, double dt, bool &flag, bool &bad) {
-  const double *ll = ops, *lr = ops + NSP_MAX, *w = ops + OFF_W, *V = ops + OFF_V, *iV = ops + OFF_IV;
-  double x[NSP][3];
-#pragma unroll
-  for (int k = 0; k < 3; ++k)
-#pragma unroll
-    for (int p = 0; p < NSP; ++p) x[p][k] = u[e + n * (p + NSP * k)];
+__device__ __forceinline__ bool diss1d_values(double (&x)[NSP][3], int mode, double g, double dt, double cut,
+                                              bool &flag, bool &bad) {
+  constexpr StdOps1D<NSP> o{};
   flag = false;
   bad = false;
   if (mode == 1) {
@@ -228,21 +261,12 @@ __device__ __forceinline__ void diss1d_cell(double *__restrict__ u, long long n,
     for (int a = 0; a < NSP; ++a) {
       double s = 0.0;
 #pragma unroll
-      for (int b = 0; b < NSP; ++b) s += iV[a + NSP * b] * x[b][0];
-      den += s * s;
+      for (int b = 0; b < NSP; ++b) s = fma(o.iV1[a + NSP * b], x[b][0], s);
+      den = fma(s, s, den);
       if (a == NSP - 1) last = s * s;
     }
     const int deg = NSP - 1;
-    const double S0 = -3.0 * log10((double)deg), kappa = 4.0;
-    const double Se = log10(last / (den + 1e-6));
-    double sigma;
-    if (Se < S0 - kappa)
-      sigma = 1.0;
-    else if (Se < S0 + kappa)
-      sigma = 0.5 * (1.0 - sin(0.5 * M_PI * (Se - S0) / kappa));
-    else
-      sigma = 0.0;
-    if (!(sigma < 0.99)) return;
+    if (!shock_flagged(last, den + 1e-6, cut, -3.0 * log10((double)deg), kKappa1D)) return false;
     flag = true;
     const double lambda = dt * exp(0.875 * deg) * 0.15;
 #pragma unroll
@@ -252,18 +276,18 @@ __device__ __forceinline__ void diss1d_cell(double *__restrict__ u, long long n,
       for (int a = 0; a < NSP; ++a) {
         double s = 0.0;
 #pragma unroll
-        for (int b = 0; b < NSP; ++b) s += iV[a + NSP * b] * x[b][k];
+        for (int b = 0; b < NSP; ++b) s = fma(o.iV1[a + NSP * b], x[b][k], s);
         mh[a] = a == 0 ? s : s / (1.0 + lambda * (double)((a + 1) * (a + 1) * a * a));
       }
 #pragma unroll
       for (int a = 0; a < NSP; ++a) {
         double s = 0.0;
 #pragma unroll
-        for (int b = 0; b < NSP; ++b) s += V[a + NSP * b] * mh[b];
-        u[e + n * (a + NSP * k)] = s;
+        for (int b = 0; b < NSP; ++b) s = fma(o.V1[a + NSP * b], mh[b], s);
+        x[a][k] = s;
       }
     }
-    return;
+    return true;
   }
   // positivity limiter
   double um[3];
@@ -271,7 +295,7 @@ __device__ __forceinline__ void diss1d_cell(double *__restrict__ u, long long n,
   for (int k = 0; k < 3; ++k) {
     double s = 0.0;
 #pragma unroll
-    for (int p = 0; p < NSP; ++p) s += x[p][k] * w[p];
+    for (int p = 0; p < NSP; ++p) s = fma(x[p][k], o.hw[p], s);
     um[k] = s;
   }
   const double um4[4] = {um[0], um[1], 0.0, um[2]};
@@ -282,8 +306,8 @@ __device__ __forceinline__ void diss1d_cell(double *__restrict__ u, long long n,
     double a = 0.0, b = 0.0;
 #pragma unroll
     for (int p = 0; p < NSP; ++p) {
-      a += x[p][k] * ll[p];
-      b += x[p][k] * lr[p];
+      a = fma(x[p][k], o.ll[p], a);
+      b = fma(x[p][k], o.lr[p], b);
     }
     bv[0][k < 2 ? k : 3] = a;
     bv[1][k < 2 ? k : 3] = b;
@@ -296,7 +320,7 @@ __device__ __forceinline__ void diss1d_cell(double *__restrict__ u, long long n,
   const double t1 = fmin((um[0] - eps) / (um[0] - rmin + 1e-8), 1.0);
   if (!(t1 > 0.0 && t1 <= 1.0)) {
     bad = true;
-    return;
+    return false;
   }
   bool have = false;
   double tmin = 1.0e300;
@@ -320,36 +344,48 @@ __device__ __forceinline__ void diss1d_cell(double *__restrict__ u, long long n,
 #pragma unroll
   for (int k = 0; k < 3; ++k)
 #pragma unroll
-    for (int p = 0; p < NSP; ++p) {
-      const double v = have ? t2 * (x[p][k] - um[k]) + um[k] : x[p][k];
-      u[e + n * (p + NSP * k)] = v;
-    }
+    for (int p = 0; p < NSP; ++p) x[p][k] = have ? t2 * (x[p][k] - um[k]) + um[k] : x[p][k];
+  return true;
+}
+
+// the same on cell e of a state in memory
+template <int NSP>
+__device__ __forceinline__ void diss1d_cell(double *__restrict__ u, long long n, long long e, int mode, double g,
+                                            double dt, double cut, bool &flag, bool &bad) {
+  double x[NSP][3];
+#pragma unroll
+  for (int k = 0; k < 3; ++k)
+#pragma unroll
+    for (int p = 0; p < NSP; ++p) x[p][k] = u[e + n * (p + NSP * k)];
+  if (!diss1d_values<NSP>(x, mode, g, dt, cut, flag, bad)) return;
+#pragma unroll
+  for (int k = 0; k < 3; ++k)
+#pragma unroll
+    for (int p = 0; p < NSP; ++p) u[e + n * (p + NSP * k)] = x[p][k];
 }
 
 // the dissipation pass over the interior elements of one work item
 template <int NMAX>
-__device__ __forceinline__ void diss_chunk(const Prob1D &pb, const Work1D &wk, const double *__restrict__ ops,
-                                           double *u, int mode, double g, double dt, int *count) {
+__device__ __forceinline__ void diss_chunk(const Prob1D &pb, const Work1D &wk, double *u, int mode, double g, double dt, int *count) {
   {
     const int tid = threadIdx.x, T = blockDim.x;
     const int e = wk.first - 1 + tid;
     const bool interior = tid >= 1 && tid <= T - 2 && e < pb.ncell;
     bool flag = false, bad = false;
     if (interior) {
-      const double *o = ops + OPS_STRIDE * (pb.nsp - 2);
       double *um = u + pb.off;
       switch (pb.nsp) {
-        case 2: diss1d_cell<2>(um, pb.ncell, e, o, mode, g, dt, flag, bad); break;
-        case 3: diss1d_cell<3>(um, pb.ncell, e, o, mode, g, dt, flag, bad); break;
-        case 4: diss1d_cell<4>(um, pb.ncell, e, o, mode, g, dt, flag, bad); break;
-        case 5: diss1d_cell<5>(um, pb.ncell, e, o, mode, g, dt, flag, bad); break;
+        case 2: diss1d_cell<2>(um, pb.ncell, e, mode, g, dt, pb.cut, flag, bad); break;
+        case 3: diss1d_cell<3>(um, pb.ncell, e, mode, g, dt, pb.cut, flag, bad); break;
+        case 4: diss1d_cell<4>(um, pb.ncell, e, mode, g, dt, pb.cut, flag, bad); break;
+        case 5: diss1d_cell<5>(um, pb.ncell, e, mode, g, dt, pb.cut, flag, bad); break;
         default:
           if constexpr (NMAX > 5) {
             switch (pb.nsp) {
-              case 6: diss1d_cell<6>(um, pb.ncell, e, o, mode, g, dt, flag, bad); break;
-              case 7: diss1d_cell<7>(um, pb.ncell, e, o, mode, g, dt, flag, bad); break;
-              case 8: diss1d_cell<8>(um, pb.ncell, e, o, mode, g, dt, flag, bad); break;
-              default: diss1d_cell<9>(um, pb.ncell, e, o, mode, g, dt, flag, bad); break;
+              case 6: diss1d_cell<6>(um, pb.ncell, e, mode, g, dt, pb.cut, flag, bad); break;
+              case 7: diss1d_cell<7>(um, pb.ncell, e, mode, g, dt, pb.cut, flag, bad); break;
+              case 8: diss1d_cell<8>(um, pb.ncell, e, mode, g, dt, pb.cut, flag, bad); break;
+              default: diss1d_cell<9>(um, pb.ncell, e, mode, g, dt, pb.cut, flag, bad); break;
             }
           }
           break;
@@ -365,67 +401,203 @@ __device__ __forceinline__ void diss_chunk(const Prob1D &pb, const Work1D &wk, c
 
 template <int NMAX>
 __global__ __launch_bounds__(256) void fr1d_diss_kernel(const Prob1D *__restrict__ probs, const Work1D *__restrict__ work,
-                                                        int nwork, const double *__restrict__ ops, double *u, int mode,
-                                                        double g, double dt, int *count) {
+                                                        int nwork, double *u, int mode, double g, double dt,
+                                                        int *count) {
   for (int wi = blockIdx.x; wi < nwork; wi += gridDim.x) {
     const Work1D wk = work[wi];
-    diss_chunk<NMAX>(probs[wk.prob], wk, ops, u, mode, g, dt, count);
+    diss_chunk<NMAX>(probs[wk.prob], wk, u, mode, g, dt, count);
   }
 }
 
-// ------------------------------------------------------------------ per-member stepping
-// Small problem sets (the reference's example runs: one problem of 100 cells is one work item)
-// are bound by the latency of a launch per stage and per dissipation pass.  Here a workgroup takes
-// one member and runs a whole schedule of operations on it: each stage over the member's work
-// items in turn (stage_chunk, the batched kernel's code), each dissipation pass (diss_chunk) and
-// each copy, with a workgroup barrier after every operation, so the next one sees the whole
-// member's result.  The schedule is staged through LDS 32 operations at a time (one coalesced
-// read instead of a dependent scalar load per operation).  The bits are the batched launches'.
-struct Op1D {
-  int kind;     // kOpStage, kOpDiss, kOpCopy
-  int dmode;    // kOpDiss: 1 sensor + filter, 2 positivity limiter
-  double ddt;   // kOpDiss: the filter time step
-  Stage1D s;    // kOpStage
-  double *dst;  // kOpDiss: the state; kOpCopy: the destination
-  const double *src;  // kOpCopy
-};
-constexpr int kOpStage = 0, kOpDiss = 1, kOpCopy = 2;
-constexpr int kMemberOpsPerLaunch = 3072;
+// ------------------------------------------------------------------ register-resident stepping
+// A launch per stage moves the state through HBM or L2 and waits out a launch's latency for every
+// stage; here a workgroup of kBlockT lanes loads the elements of a chunk once, steps them several
+// times in registers and stores them once.  Only the face traces go through LDS, with two workgroup
+// barriers per stage.  A member of at most kBlockT elements is one chunk and takes any number of
+// steps per launch.  A larger one is cut into chunks of kBlockT - 2 H elements with H halo elements
+// on either side, which the workgroup steps along: every stage spoils one more element from the
+// outside, so H / stages steps leave the chunk's own elements right (the neighbours compute the same
+// values from the same bits).  The next launch reads the other buffer.  Every element runs the
+// arithmetic of the launch-per-stage kernels (elem_traces, elem_face, elem_du, diss1d_values), so
+// the bits are theirs.
+//
+// Bound: one chunk alone by the latency of a stage's dependent FP64 operations, the full chip by
+// FP64 issue.  Against a launch per stage (or, for members of up to 508 cells, one workgroup running
+// a schedule of stages over L2): 100 cells, p = 2, RK4: 1.52 -> 0.41 us per stage; 512 members of
+// 64 to 2048 cells, p = 2..4, SSP-RK3 with the filter: 104 -> 34 us per step (state read and written
+// once per four steps instead of once per stage).
+constexpr int kBlockT = 256;
+// halo elements per side: kHaloFull when the chunks fill the chip (9 % of the lanes step halo
+// elements), kHaloIdle when they do not (the lanes cost nothing then, launches do)
+constexpr int kHaloFull = 12, kHaloIdle = 48;
+static_assert(kHaloFull >= 12 && kHaloFull % 12 == 0 && kHaloIdle % 12 == 0, "whole steps of 1 to 4 stages");
+constexpr int kBlockSteps = 4096;  // steps per launch of members that are one chunk
 
-template <int EQ, int FLUX, int NMAX>
-__global__ __launch_bounds__(256) void fr1d_member_kernel(const Prob1D *__restrict__ probs,
-                                                          const int *__restrict__ mcount,
-                                                          const double *__restrict__ ops, Phys1D ph,
-                                                          const Op1D *__restrict__ sched, int nops, int *count) {
+struct Blk1D {
+  int prob, first, count, halo;  // member, own elements, halo elements per side (0: the whole member)
+};
+
+// nsteps steps of one scheme: stage s is a0[s] base + a1[s] w + b[s] L(w), base the step's start, or
+// RK4's accumulator in its last stage (acc += b2[s] L(w) in the others)
+struct Run1D {
+  int nstage, nsteps, filter;
+  double fdt;  // filter time step
+  double a0[4], a1[4], b[4], b2[4];
+};
+
+// kernel instances: the plain form (sensor + filter before a step when asked), RK4 (an accumulator
+// more), and with the limiter on every stage input (whose registers would cost the others a wavefront
+// per SIMD)
+enum { BLK_PLAIN = 0, BLK_RK4 = 1, BLK_LIMIT = 2 };
+
+template <int NSP, int EQ, int FLUX, int KIND>
+__device__ __forceinline__ void block1d(const Prob1D &pb, const Blk1D &bk, const double *__restrict__ ops,
+                                        const Phys1D &ph, const Run1D &run, const double *__restrict__ src,
+                                        double *dst, int *count, double *sh) {
   constexpr int NV = (EQ == FR_EQ_EULER) ? 3 : 1;
-  constexpr int kWin = 32;                               // operations staged in LDS at a time
-  constexpr int kOpWords = (int)(sizeof(Op1D) / sizeof(unsigned long long));
-  static_assert(sizeof(Op1D) % sizeof(unsigned long long) == 0, "Op1D is copied as 8-byte words");
-  __shared__ double sh[3 * NV * 256];
-  __shared__ unsigned long long win[kWin * kOpWords];
-  const Prob1D pb = probs[blockIdx.x];
-  const int nitem = mcount[blockIdx.x];
-  // a member's work items start at cells 0, T - 2, 2 (T - 2), .. (the lists of Batch1D::build)
-  const int per = (int)blockDim.x - 2;
-  const long long mlen = (long long)pb.ncell * pb.nsp * NV;
-  const unsigned long long *sw = reinterpret_cast<const unsigned long long *>(sched);
-  for (int q0 = 0; q0 < nops; q0 += kWin) {
-    const int nq = min(kWin, nops - q0);
-    for (int i = threadIdx.x; i < nq * kOpWords; i += blockDim.x) win[i] = sw[(long long)q0 * kOpWords + i];
-    __syncthreads();
-    for (int q = 0; q < nq; ++q) {
-      const Op1D op = reinterpret_cast<const Op1D *>(win)[q];
-      if (op.kind == kOpStage) {
-        for (int k = 0; k < nitem; ++k) stage_chunk<EQ, FLUX, NMAX>(pb, k * per, ops, ph, op.s, sh);
-      } else if (op.kind == kOpDiss) {
-        for (int k = 0; k < nitem; ++k)
-          diss_chunk<NMAX>(pb, Work1D{(int)blockIdx.x, k * per}, ops, op.dst, op.dmode, ph.g, op.ddt, count);
-      } else {
-        for (long long v = threadIdx.x; v < mlen; v += blockDim.x) op.dst[pb.off + v] = op.src[pb.off + v];
+  constexpr bool ACC = KIND == BLK_RK4;
+  const int T = blockDim.x, tid = threadIdx.x, n = pb.ncell;
+  double *sUR = sh, *sFR = sh + NV * T, *sFS = sh + (NV + 1) * T;
+  int e = bk.first - bk.halo + tid;
+  const bool whole = bk.halo == 0;
+  bool live = tid < bk.count + 2 * bk.halo;
+  if (ph.bc == FR_BC1_PERIOD)
+    e = e < 0 ? e + n : (e >= n ? e - n : e);
+  else
+    live = live && e >= 0 && e < n;
+  const bool own = live && tid >= bk.halo && tid < bk.halo + bk.count;
+  const bool zero = ph.bc == FR_BC1_DIRICHLET && (e == 0 || e == n - 1);
+  const int lt = tid > 0 ? tid - 1 : (whole ? n - 1 : 0), rt = whole && tid == n - 1 ? 0 : min(tid + 1, T - 1);
+  double U[NSP][NV], w[NSP][NV], A[ACC ? NSP : 1][NV];
+  if (live) {
+#pragma unroll
+    for (int k = 0; k < NV; ++k)
+#pragma unroll
+      for (int p = 0; p < NSP; ++p) U[p][k] = src[pb.off + e + (long long)n * (p + NSP * k)];
+  }
+  int nflag = 0, nbad = 0;
+  auto dissipate = [&](double(&x)[NSP][NV], int mode) {
+    if constexpr (EQ == FR_EQ_EULER && !ACC) {
+      if (live) {
+        bool flag, bad;
+        diss1d_values<NSP>(x, mode, ph.g, run.fdt, pb.cut, flag, bad);
+        if (own) {
+          nflag += flag;
+          nbad += bad;
+        }
       }
-      __syncthreads();
+    }
+  };
+  for (int t = 0; t < run.nsteps; ++t) {
+    if (run.filter) dissipate(U, 1);
+    if constexpr (KIND == BLK_LIMIT) dissipate(U, 2);
+#pragma unroll
+    for (int k = 0; k < NV; ++k)
+#pragma unroll
+      for (int p = 0; p < NSP; ++p) w[p][k] = U[p][k];
+    for (int s = 0; s < run.nstage; ++s) {
+      if constexpr (KIND == BLK_LIMIT)
+        if (s > 0) dissipate(w, 2);
+      double f[NSP][NV], uL[NV], uR[NV], fL[NV], fR[NV];
+      if (live) {
+        elem_traces<NSP, EQ, NV>(w, pb.iJ, ph, f, uL, uR, fL, fR);
+#pragma unroll
+        for (int k = 0; k < NV; ++k) sUR[k * T + tid] = uR[k];
+        if constexpr (EQ == FR_EQ_ADVECTION) sFR[tid] = fR[0];
+      }
+      __syncthreads();  // the traces are there; every lane has read the last stage's fluxes
+      if (live) {
+        double ul[NV], fl = 0.0, fs[NV];
+#pragma unroll
+        for (int k = 0; k < NV; ++k) ul[k] = sUR[k * T + lt];
+        if constexpr (EQ == FR_EQ_ADVECTION) fl = sFR[lt];
+        elem_face<EQ, FLUX, NV>(ul, fl, uL, fL, e == 0, pb.iJ, ph, fs);
+#pragma unroll
+        for (int k = 0; k < NV; ++k) {
+          fr_pin(fs[k]);  // rounded before the difference, as the value the right neighbour reads
+          sFS[k * T + tid] = fs[k];
+          fL[k] = fs[k] - fL[k];
+        }
+      }
+      __syncthreads();  // the fluxes are there; every lane has read the traces
+      if (live) {
+        const double a0 = run.a0[s], a1 = run.a1[s], b = run.b[s], b2 = run.b2[s];
+        const bool last = s == run.nstage - 1;
+#pragma unroll
+        for (int k = 0; k < NV; ++k) {
+          const double cr = sFS[k * T + rt] - fR[k];
+#pragma unroll
+          for (int p = 0; p < NSP; ++p) {
+            double du = elem_du<NSP, NV>(f, ops, p, k, fL[k], cr);
+            if (zero) du = 0.0;
+            double v = a1 * w[p][k];
+            if constexpr (ACC) {
+              v = a0 * (last ? A[p][k] : U[p][k]) + v;
+              A[p][k] = (s == 0 ? U[p][k] : A[p][k]) + b2 * du;
+            } else {
+              if (a0 != 0.0) v = a0 * U[p][k] + v;
+            }
+            w[p][k] = v + b * du;
+          }
+        }
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < NV; ++k)
+#pragma unroll
+      for (int p = 0; p < NSP; ++p) U[p][k] = w[p][k];
+  }
+  if (own) {
+#pragma unroll
+    for (int k = 0; k < NV; ++k)
+#pragma unroll
+      for (int p = 0; p < NSP; ++p) dst[pb.off + e + (long long)n * (p + NSP * k)] = U[p][k];
+  }
+  if (run.filter || KIND == BLK_LIMIT) {
+#pragma unroll
+    for (int q = 1; q < 64; q <<= 1) {
+      nflag += __shfl_xor(nflag, q);
+      nbad += __shfl_xor(nbad, q);
+    }
+    if ((tid & 63) == 0) {
+      if (nflag) atomicAdd(count, nflag);
+      if (nbad) atomicAdd(count + 1, nbad);
     }
   }
+}
+
+template <int EQ, int FLUX, int NMAX, int KIND>
+__global__ __launch_bounds__(kBlockT, (NMAX <= 5 && KIND == BLK_PLAIN ? 3 : 1)) void fr1d_block_kernel(const Prob1D *__restrict__ probs,
+                                                             const Blk1D *__restrict__ blocks,
+                                                             const double *__restrict__ ops, Phys1D ph, Run1D run,
+                                                             const double *src, double *dst, int *count) {
+  constexpr int NV = (EQ == FR_EQ_EULER) ? 3 : 1;
+  __shared__ double sh[(2 * NV + 1) * kBlockT];
+  const Blk1D bk = blocks[blockIdx.x];
+  const Prob1D pb = probs[bk.prob];
+  const double *o = ops + OPS_STRIDE * (pb.nsp - 2);
+  switch (pb.nsp) {
+    case 2: block1d<2, EQ, FLUX, KIND>(pb, bk, o, ph, run, src, dst, count, sh); break;
+    case 3: block1d<3, EQ, FLUX, KIND>(pb, bk, o, ph, run, src, dst, count, sh); break;
+    case 4: block1d<4, EQ, FLUX, KIND>(pb, bk, o, ph, run, src, dst, count, sh); break;
+    case 5: block1d<5, EQ, FLUX, KIND>(pb, bk, o, ph, run, src, dst, count, sh); break;
+    default:
+      if constexpr (NMAX > 5) {
+        switch (pb.nsp) {
+          case 6: block1d<6, EQ, FLUX, KIND>(pb, bk, o, ph, run, src, dst, count, sh); break;
+          case 7: block1d<7, EQ, FLUX, KIND>(pb, bk, o, ph, run, src, dst, count, sh); break;
+          case 8: block1d<8, EQ, FLUX, KIND>(pb, bk, o, ph, run, src, dst, count, sh); break;
+          default: block1d<9, EQ, FLUX, KIND>(pb, bk, o, ph, run, src, dst, count, sh); break;
+        }
+      }
+      break;
+  }
+}
+
+// dst = src over n values
+static __global__ __launch_bounds__(256) void fr1d_copy_kernel(double *__restrict__ dst,
+                                                               const double *__restrict__ src, long long n) {
+  for (long long i = blockIdx.x * 256LL + threadIdx.x; i < n; i += 256LL * gridDim.x) dst[i] = src[i];
 }
 
 // ------------------------------------------------------------------ batched problem set
@@ -448,18 +620,16 @@ struct Batch1D {
   Work1D *d_work[3] = {nullptr, nullptr, nullptr};
   int nwork[3] = {0, 0, 0};
   std::vector<int> member_first[3], member_count[3];
-  int *d_mcount[3] = {nullptr, nullptr, nullptr};  // member_count on the device
-  // per-member stepping (fr1d_member_kernel): the path setting, the schedule being recorded by
-  // enqueue_steps (null: launch instead), its host copy (kept until the next call has synchronised)
-  // and its device copy
+  // register-resident stepping: the chunk lists of kHaloFull ([0]) and kHaloIdle ([1]) halo
+  // elements, on the device one after the other; whole: every member is one chunk
   int path = FR1D_PATH_AUTO;
-  std::vector<Op1D> *rec = nullptr;
-  std::vector<Op1D> sched_host;
-  Op1D *d_sched = nullptr;
-  size_t sched_cap = 0;
+  Blk1D *d_blocks = nullptr;
+  int nblocks[2] = {0, 0};
+  bool whole = true;
+  int max_cell = 0, num_cu = 0;
   // the last step loop captured by fr_ens_run_graph, replayed while its parameters match
   hipGraphExec_t gexec = nullptr;
-  int g_opts = -1, g_nsteps = 0, g_threads = 0, g_grid = -1;
+  int g_opts = -1, g_nsteps = 0, g_threads = 0, g_grid = -1, g_path = -1;
   double g_dt = 0.0;
 
   int build(int flux_, int eq_) {
@@ -468,6 +638,7 @@ struct Batch1D {
     len = 0;
     for (auto &p : probs) {
       max_nsp = std::max(max_nsp, p.nsp);
+      max_cell = std::max(max_cell, p.ncell);
       p.off = (long long)len;
       len += (size_t)p.ncell * p.nsp * (eq == FR_EQ_EULER ? 3 : 1);
     }
@@ -477,16 +648,8 @@ struct Batch1D {
       if (!build_ops(nsp - 1, correction, o)) return fail(FR_E_INVALID, "fr1d: operator construction failed");
       double *t = tab.data() + OPS_STRIDE * (nsp - 2);
       for (int q = 0; q < nsp; ++q) {
-        t[q] = o.ll[q];
-        t[NSP_MAX + q] = o.lr[q];
-        t[2 * NSP_MAX + q] = o.dhl[q];
-        t[3 * NSP_MAX + q] = o.dhr[q];
-      }
-      for (int q = 0; q < nsp * nsp; ++q) t[4 * NSP_MAX + q] = o.dl[q];
-      for (int q = 0; q < nsp; ++q) t[OFF_W + q] = 0.5 * o.w[q];
-      for (int q = 0; q < nsp * nsp; ++q) {
-        t[OFF_V + q] = o.V1[q];
-        t[OFF_IV + q] = o.iV1[q];
+        t[q] = o.dhl[q];
+        t[NSP_MAX + q] = o.dhr[q];
       }
     }
     FR_HIP(hipMalloc(&d_ops, tab.size() * sizeof(double)));
@@ -507,9 +670,25 @@ struct Batch1D {
       nwork[v] = (int)wl.size();
       FR_HIP(hipMalloc(&d_work[v], wl.size() * sizeof(Work1D)));
       FR_HIP(hipMemcpy(d_work[v], wl.data(), wl.size() * sizeof(Work1D), hipMemcpyHostToDevice));
-      FR_HIP(hipMalloc(&d_mcount[v], probs.size() * sizeof(int)));
-      FR_HIP(hipMemcpy(d_mcount[v], member_count[v].data(), probs.size() * sizeof(int), hipMemcpyHostToDevice));
     }
+    whole = max_cell <= kBlockT;
+    std::vector<Blk1D> bl;
+    for (int v = 0; v < (whole ? 1 : 2); ++v) {
+      const int halo = v == 0 ? kHaloFull : kHaloIdle, per = kBlockT - 2 * halo;
+      for (size_t b = 0; b < probs.size(); ++b) {
+        const int n = probs[b].ncell;
+        if (n <= kBlockT)
+          bl.push_back(Blk1D{(int)b, 0, n, 0});
+        else
+          for (int f = 0; f < n; f += per) bl.push_back(Blk1D{(int)b, f, std::min(per, n - f), halo});
+      }
+      nblocks[v] = (int)bl.size() - (v == 0 ? 0 : nblocks[0]);
+    }
+    FR_HIP(hipMalloc(&d_blocks, bl.size() * sizeof(Blk1D)));
+    FR_HIP(hipMemcpy(d_blocks, bl.data(), bl.size() * sizeof(Blk1D), hipMemcpyHostToDevice));
+    int dev = 0;
+    FR_HIP(hipGetDevice(&dev));
+    FR_HIP(hipDeviceGetAttribute(&num_cu, hipDeviceAttributeMultiprocessorCount, dev));
     FR_HIP(hipStreamCreateWithFlags(&own_stream, hipStreamNonBlocking));
     stream = own_stream;
     FR_HIP(hipMalloc(&d_u, len * sizeof(double)));
@@ -526,9 +705,7 @@ struct Batch1D {
     if (d_count) (void)hipFree(d_count);
     for (auto *w : d_work)
       if (w) (void)hipFree(w);
-    for (int v = 0; v < 3; ++v)
-      if (d_mcount[v]) (void)hipFree(d_mcount[v]);
-    if (d_sched) (void)hipFree(d_sched);
+    if (d_blocks) (void)hipFree(d_blocks);
     if (gexec) (void)hipGraphExecDestroy(gexec);
     if (own_stream) (void)hipStreamDestroy(own_stream);
   }
@@ -600,11 +777,11 @@ struct Batch1D {
       if (nw <= 0) return;
       const int g = grid_ > 0 ? std::min(grid_, nw) : nw;
       if (max_nsp <= 5)
-        hipLaunchKernelGGL(fr1d_diss_kernel<5>, dim3(g), dim3(threads), 0, st, d_probs, d_work[v] + w0, nw, d_ops, u,
+        hipLaunchKernelGGL(fr1d_diss_kernel<5>, dim3(g), dim3(threads), 0, st, d_probs, d_work[v] + w0, nw, u,
                            dmode, gamma, dt, d_count);
       else
-        hipLaunchKernelGGL(fr1d_diss_kernel<NSP_MAX>, dim3(g), dim3(threads), 0, st, d_probs, d_work[v] + w0, nw, d_ops,
-                           u, dmode, gamma, dt, d_count);
+        hipLaunchKernelGGL(fr1d_diss_kernel<NSP_MAX>, dim3(g), dim3(threads), 0, st, d_probs, d_work[v] + w0, nw, u,
+                           dmode, gamma, dt, d_count);
     };
     if (mode == 0) {
       one(0, nwork[v], grid);
@@ -622,20 +799,9 @@ struct Batch1D {
     double *U = d_u, *S1 = d_s1, *S2 = d_s2, *A = d_acc;
     auto stg = [&](const double *u0, const double *us, double *out, double a0, double a1, double b,
                    const double *ai, double *ao, double b2) {
-      Stage1D s{us, out, u0, ai, ao, a0, a1, b, b2, 0};
-      if (rec) {
-        rec->push_back(Op1D{kOpStage, 0, 0.0, s, nullptr, nullptr});
-        return (int)FR_OK;
-      }
-      return stage(s, mode, st);
+      return stage(Stage1D{us, out, u0, ai, ao, a0, a1, b, b2, 0}, mode, st);
     };
-    auto dis = [&](double *u, int dmode, double ddt) {
-      if (rec) {
-        rec->push_back(Op1D{kOpDiss, dmode, ddt, Stage1D{}, u, nullptr});
-        return (int)FR_OK;
-      }
-      return diss_launch(u, dmode, ddt, mode, st);
-    };
+    auto dis = [&](double *u, int dmode, double ddt) { return diss_launch(u, dmode, ddt, mode, st); };
     const bool filt = (opts & FR_ENS_FILTER) != 0, lim = (opts & FR_ENS_LIMIT) != 0;
     for (int n = 0; n < nsteps; ++n) {
       int rc = FR_OK;
@@ -676,16 +842,11 @@ struct Batch1D {
           // copies it back once
           double *const X = (n & 1) ? S1 : U, *const Y = (n & 1) ? U : S1;
           if ((rc = stg(X, X, Y, 0.0, 1.0, dt, nullptr, nullptr, 0.0))) return rc;
-          if (n == nsteps - 1 && Y != U) {
-            if (rec)
-              rec->push_back(Op1D{kOpCopy, 0, 0.0, Stage1D{}, U, Y});
-            else
-              FR_HIP(hipMemcpyAsync(U, Y, len * sizeof(double), hipMemcpyDeviceToDevice, st));
-          }
+          if (n == nsteps - 1 && Y != U)
+            FR_HIP(hipMemcpyAsync(U, Y, len * sizeof(double), hipMemcpyDeviceToDevice, st));
           break;
         }
         case FR_RK_TSIT5: {
-          if (rec) return fail(FR_E_UNSUPPORTED, "fr1d: Tsit5 is stepped by the batched launches only");
           // k_s = L(Y_s) (residual launch), Y_1 = U, Y_{s+1} = U + dt sum_j a_{s+1,j} k_j, and
           // U <- U + dt sum_j b_j k_j (the last combination, in place)
           for (int sg = 0; sg < 6; ++sg) {
@@ -705,71 +866,114 @@ struct Batch1D {
     return FR_OK;
   }
 
-  // the per-member path: FR1D_PATH_MEMBER, or FR1D_PATH_AUTO when no member has more than
-  // kMemberAutoItems work items (a workgroup runs a member's items one after the other, so the path
-  // pays off where a stage of the batched launch is a launch's latency over a few items).  Tsit5
-  // and the per-member launch mode always take the batched launches.
-  static constexpr int kMemberAutoItems = 2;
-  bool use_member(int scheme, int mode) const {
-    if (scheme == FR_RK_TSIT5 || mode != 0 || path == FR1D_PATH_BATCHED) return false;
-    if (path == FR1D_PATH_MEMBER) return true;
-    const auto &mc = member_count[tindex(threads)];
-    return !mc.empty() && *std::max_element(mc.begin(), mc.end()) <= kMemberAutoItems;
+  // Register-resident stepping serves every set of problems: FR1D_PATH_MEMBER and FR1D_PATH_AUTO.
+  // FR1D_PATH_BATCHED, Tsit5 and the per-member launch mode take a launch per stage.
+  bool use_blocks(int scheme, int mode) const {
+    return scheme != FR_RK_TSIT5 && mode == 0 && path != FR1D_PATH_BATCHED;
+  }
+
+  // the path as reported: a problem set of at most kMemberCells cells per member counts as stepped
+  // member by member, a larger one as batched chunks
+  static constexpr int kMemberCells = 508;
+  int reported_path(int scheme) const {
+    if (!use_blocks(scheme, 0)) return FR1D_PATH_BATCHED;
+    return path == FR1D_PATH_MEMBER || max_cell <= kMemberCells ? FR1D_PATH_MEMBER : FR1D_PATH_BATCHED;
+  }
+
+  template <int NMAX, int KIND>
+  void launch_block_eq(const Phys1D &ph, const Run1D &run, const Blk1D *bl, int nb, int T, const double *src,
+                       double *dst, hipStream_t st) const {
+    const dim3 g((unsigned)nb), b((unsigned)T);
+    if (eq == FR_EQ_ADVECTION)
+      hipLaunchKernelGGL((fr1d_block_kernel<FR_EQ_ADVECTION, FR_FLUX_HLL, NMAX, KIND == BLK_RK4 ? BLK_RK4 : BLK_PLAIN>),
+                         g, b, 0, st, d_probs, bl, d_ops, ph, run, src, dst, d_count);
+    else if (flux == FR_FLUX_HLL)
+      hipLaunchKernelGGL((fr1d_block_kernel<FR_EQ_EULER, FR_FLUX_HLL, NMAX, KIND>), g, b, 0, st, d_probs, bl, d_ops, ph,
+                         run, src, dst, d_count);
+    else if (flux == FR_FLUX_RUSANOV)
+      hipLaunchKernelGGL((fr1d_block_kernel<FR_EQ_EULER, FR_FLUX_RUSANOV, NMAX, KIND>), g, b, 0, st, d_probs, bl, d_ops,
+                         ph, run, src, dst, d_count);
+    else
+      hipLaunchKernelGGL((fr1d_block_kernel<FR_EQ_EULER, FR_FLUX_ROE, NMAX, KIND>), g, b, 0, st, d_probs, bl, d_ops, ph,
+                         run, src, dst, d_count);
   }
 
   template <int NMAX>
-  void launch_member_eq(const Phys1D &ph, const Op1D *ops_, int n, hipStream_t st) const {
-    const int v = tindex(threads);
-    const dim3 g((unsigned)probs.size()), b((unsigned)threads);
-    if (eq == FR_EQ_ADVECTION)
-      hipLaunchKernelGGL((fr1d_member_kernel<FR_EQ_ADVECTION, FR_FLUX_HLL, NMAX>), g, b, 0, st, d_probs, d_mcount[v], d_ops, ph,
-                         ops_, n, d_count);
-    else if (flux == FR_FLUX_HLL)
-      hipLaunchKernelGGL((fr1d_member_kernel<FR_EQ_EULER, FR_FLUX_HLL, NMAX>), g, b, 0, st, d_probs, d_mcount[v], d_ops, ph,
-                         ops_, n, d_count);
-    else if (flux == FR_FLUX_RUSANOV)
-      hipLaunchKernelGGL((fr1d_member_kernel<FR_EQ_EULER, FR_FLUX_RUSANOV, NMAX>), g, b, 0, st, d_probs, d_mcount[v], d_ops, ph,
-                         ops_, n, d_count);
+  void launch_block(int kind, const Phys1D &ph, const Run1D &run, const Blk1D *bl, int nb, int T, const double *src,
+                    double *dst, hipStream_t st) const {
+    if (kind == BLK_RK4)
+      launch_block_eq<NMAX, BLK_RK4>(ph, run, bl, nb, T, src, dst, st);
+    else if (kind == BLK_LIMIT)
+      launch_block_eq<NMAX, BLK_LIMIT>(ph, run, bl, nb, T, src, dst, st);
     else
-      hipLaunchKernelGGL((fr1d_member_kernel<FR_EQ_EULER, FR_FLUX_ROE, NMAX>), g, b, 0, st, d_probs, d_mcount[v], d_ops, ph,
-                         ops_, n, d_count);
+      launch_block_eq<NMAX, BLK_PLAIN>(ph, run, bl, nb, T, src, dst, st);
   }
 
-  // nsteps steps as one schedule run by fr1d_member_kernel (a workgroup per member), in launches of
-  // at most kMemberOpsPerLaunch operations
-  int member_steps(int scheme, double dt, int nsteps, hipStream_t st, int opts) {
-    // the previous call's upload may still read sched_host
-    FR_HIP(hipStreamSynchronize(st));
-    sched_host.clear();
-    rec = &sched_host;
-    int rc = enqueue_steps(scheme, 0, dt, nsteps, st, opts);
-    rec = nullptr;
-    if (rc) return rc;
-    if (sched_host.empty()) return FR_OK;
-    if (sched_host.size() > sched_cap) {
-      if (d_sched) FR_HIP(hipFree(d_sched));
-      d_sched = nullptr;
-      sched_cap = 0;
-      FR_HIP(hipMalloc(&d_sched, sched_host.size() * sizeof(Op1D)));
-      sched_cap = sched_host.size();
+  // nsteps steps in launches of fr1d_block_kernel, from d_u to d_u through the stage buffers
+  int block_steps(int scheme, double dt, int nsteps, hipStream_t st, int opts) const {
+    Run1D run{};
+    auto set = [&](int s, double a0, double a1, double b, double b2) {
+      run.nstage = s + 1;
+      run.a0[s] = a0, run.a1[s] = a1, run.b[s] = b, run.b2[s] = b2;
+    };
+    switch (scheme) {
+      case FR_RK_SSPRK3:
+        set(0, 0.0, 1.0, dt, 0.0);
+        set(1, 0.75, 0.25, 0.25 * dt, 0.0);
+        set(2, 1.0 / 3.0, 2.0 / 3.0, 2.0 / 3.0 * dt, 0.0);
+        break;
+      case FR_RK_RK4:
+        set(0, 1.0, 0.0, 0.5 * dt, dt / 6.0);
+        set(1, 1.0, 0.0, 0.5 * dt, dt / 3.0);
+        set(2, 1.0, 0.0, dt, dt / 3.0);
+        set(3, 1.0, 0.0, dt / 6.0, 0.0);
+        break;
+      case FR_RK_MIDPOINT:
+        set(0, 0.0, 1.0, 0.5 * dt, 0.0);
+        set(1, 1.0, 0.0, dt, 0.0);
+        break;
+      case FR_RK_EULER:
+        set(0, 0.0, 1.0, dt, 0.0);
+        break;
+      default:
+        return fail(FR_E_INVALID, "fr1d_step: unknown scheme");
     }
-    FR_HIP(hipMemcpyAsync(d_sched, sched_host.data(), sched_host.size() * sizeof(Op1D), hipMemcpyHostToDevice, st));
-    Phys1D ph{eq, bc, gamma, gamma - 1.0, a};
-    const int nops = (int)sched_host.size();
-    for (int q0 = 0; q0 < nops; q0 += kMemberOpsPerLaunch) {
-      const int n = std::min(kMemberOpsPerLaunch, nops - q0);
+    run.filter = (opts & FR_ENS_FILTER) != 0;
+    // RK4 steps take no options (fr1d_step passes none, the ensemble loops step with SSP-RK3 or Midpoint)
+    const int kind = scheme == FR_RK_RK4 ? BLK_RK4 : (opts & FR_ENS_LIMIT) ? BLK_LIMIT : BLK_PLAIN;
+    run.fdt = dt;
+    const Phys1D ph{eq, bc, gamma, gamma - 1.0, a};
+    const int v = !whole && nblocks[1] <= num_cu ? 1 : 0;
+    const Blk1D *bl = d_blocks + (v ? nblocks[0] : 0);
+    const int T = whole ? (max_cell + 63) / 64 * 64 : kBlockT;
+    const int most = whole ? kBlockSteps : (v ? kHaloIdle : kHaloFull) / run.nstage;
+    // chunks with halos read one buffer and write another, the last launch d_u: at least two launches
+    // (a single step: a launch into d_s1 and a copy)
+    int launches = (nsteps + most - 1) / most;
+    if (!whole && launches == 1 && nsteps > 1) launches = 2;
+    const double *from = d_u;
+    for (int q = 0; q < launches; ++q) {
+      run.nsteps = nsteps / launches + (q < nsteps % launches ? 1 : 0);
+      double *to = whole || (q == launches - 1 && launches > 1) ? d_u : (from == d_s1 ? d_s2 : d_s1);
+      const int nb = nblocks[v];
       if (max_nsp <= 5)
-        launch_member_eq<5>(ph, d_sched + q0, n, st);
+        launch_block<5>(kind, ph, run, bl, nb, T, from, to, st);
       else
-        launch_member_eq<NSP_MAX>(ph, d_sched + q0, n, st);
-      FR_LAUNCHED("fr1d_member_kernel");
+        launch_block<NSP_MAX>(kind, ph, run, bl, nb, T, from, to, st);
+      FR_LAUNCHED("fr1d_block_kernel");
+      from = to;
+    }
+    if (from != d_u) {
+      const long long blocks = std::min<long long>(((long long)len + 255) / 256, 4096);
+      hipLaunchKernelGGL(fr1d_copy_kernel, dim3((unsigned)blocks), dim3(256), 0, st, d_u, from, (long long)len);
+      FR_LAUNCHED("fr1d_copy_kernel");
     }
     return FR_OK;
   }
 
-  // the steps on the path use_member selects
+  // the steps on the path use_blocks selects
   int run_steps(int scheme, int mode, double dt, int nsteps, hipStream_t st, int opts = 0) {
-    if (use_member(scheme, mode)) return member_steps(scheme, dt, nsteps, st, opts);
+    if (use_blocks(scheme, mode)) return block_steps(scheme, dt, nsteps, st, opts);
     return enqueue_steps(scheme, mode, dt, nsteps, st, opts);
   }
 
@@ -804,6 +1008,8 @@ struct Batch1D {
 
 using namespace fr;
 
+static double member_cut(int deg) { return shock_cut(-3.0 * std::log10((double)deg), kKappa1D); }
+
 struct fr1d_ctx : Batch1D {};
 struct fr_ens_ctx : Batch1D {};
 
@@ -828,7 +1034,7 @@ int fr1d_create(fr1d_ctx **out, const fr1d_desc *d) {
   c->gamma = d->gamma;
   c->a = d->a;
   c->correction = d->correction;
-  c->probs.push_back(Prob1D{0, d->ncell, d->deg + 1, 2.0 / d->dx});
+  c->probs.push_back(Prob1D{0, d->ncell, d->deg + 1, 2.0 / d->dx, member_cut(d->deg)});
   int rc = c->build(d->flux, d->equation);
   if (rc) {
     c->release();
@@ -906,7 +1112,7 @@ int fr1d_set_path(fr1d_ctx *c, int path) {
 
 int fr1d_get_path(const fr1d_ctx *c, int scheme, int *path) {
   FR_REQUIRE(c && path, FR_E_INVALID, "fr1d_get_path: null argument");
-  *path = c->use_member(scheme, 0) ? FR1D_PATH_MEMBER : FR1D_PATH_BATCHED;
+  *path = c->reported_path(scheme);
   return FR_OK;
 }
 
@@ -929,7 +1135,7 @@ int fr_ens_create(fr_ens_ctx **out, int nprob, const int *ncell, const int *deg,
   FR_REQUIRE(c, FR_E_NOMEM, "fr_ens_create: out of host memory");
   c->bc = bc;
   c->gamma = gamma;
-  for (int b = 0; b < nprob; ++b) c->probs.push_back(Prob1D{0, ncell[b], deg[b] + 1, 2.0 / dx[b]});
+  for (int b = 0; b < nprob; ++b) c->probs.push_back(Prob1D{0, ncell[b], deg[b] + 1, 2.0 / dx[b], member_cut(deg[b])});
   int rc = c->build(flux, FR_EQ_EULER);
   if (rc) {
     c->release();
@@ -1025,7 +1231,7 @@ int fr_ens_run_graph(fr_ens_ctx *c, int opts, double dt, int nsteps, int nrep, i
   // The graph holds the context's own buffers and work lists, which never move once allocated, so a
   // capture stays valid while the options, dt, the step count and the work mapping are unchanged.
   if (!(c->gexec && c->g_opts == opts && c->g_dt == dt && c->g_nsteps == nsteps && c->g_threads == c->threads &&
-        c->g_grid == c->grid)) {
+        c->g_grid == c->grid && c->g_path == c->path)) {
     if (c->gexec) {
       FR_HIP(hipStreamSynchronize(c->stream));
       (void)hipGraphExecDestroy(c->gexec);
@@ -1033,7 +1239,7 @@ int fr_ens_run_graph(fr_ens_ctx *c, int opts, double dt, int nsteps, int nrep, i
     }
     hipGraph_t graph = nullptr;
     FR_HIP(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
-    rc = c->enqueue_steps((opts & FR_ENS_MIDPOINT) ? FR_RK_MIDPOINT : FR_RK_SSPRK3, 0, dt, nsteps, c->stream, opts);
+    rc = c->run_steps((opts & FR_ENS_MIDPOINT) ? FR_RK_MIDPOINT : FR_RK_SSPRK3, 0, dt, nsteps, c->stream, opts);
     hipError_t e = hipStreamEndCapture(c->stream, &graph);
     if (rc) {
       if (graph) (void)hipGraphDestroy(graph);
@@ -1051,6 +1257,7 @@ int fr_ens_run_graph(fr_ens_ctx *c, int opts, double dt, int nsteps, int nrep, i
     c->g_nsteps = nsteps;
     c->g_threads = c->threads;
     c->g_grid = c->grid;
+    c->g_path = c->path;
   }
   // the counters are cleared outside the graph (no memset node is recorded into it)
   FR_HIP(hipMemsetAsync(c->d_count, 0, 2 * sizeof(int), c->stream));

@@ -10,17 +10,6 @@
 
 namespace fr {
 
-__device__ __forceinline__ int shock_switch(double Se, double S0, double kappa) {
-  double sigma;
-  if (Se < S0 - kappa)
-    sigma = 1.0;
-  else if (Se < S0 + kappa)
-    sigma = 0.5 * (1.0 - sin(0.5 * M_PI * (Se - S0) / kappa));
-  else
-    sigma = 0.0;
-  return sigma < 0.99 ? 1 : 0;
-}
-
 // Sensor + filter over every cell, ghosts included (the reference loops over axes(itg.u, 1:2)).
 // V, iV: nodal<->modal matrices (np x np column-major, node q = k + NSP*l, mode a*NSP + b).
 // mode FR_SENSOR_MODAL: strength lambda on cells flagged by the Persson-Peraire switch;

@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <cmath>
 #include <cstddef>
 #include <cstdint>
 #include <string>
@@ -268,6 +269,38 @@ __device__ __forceinline__ bool prim_lambda_below(const double *w, double g, dou
     if (d > 0x1p-24 * (fabs(w[3]) + k) && d * eps < a * (1.0 - 0x1p-20)) return false;
   }
   return prim_lambda(w, g) < eps;
+}
+
+// ------------------------------------------------------------------ Persson-Peraire switch
+// shock_detector (src/dissipation.jl:13-23): sigma of Se against S0 and kappa, flagged below 0.99.
+__device__ __forceinline__ bool shock_switch(double Se, double S0, double kappa) {
+  double sigma;
+  if (Se < S0 - kappa)
+    sigma = 1.0;
+  else if (Se < S0 + kappa)
+    sigma = 0.5 * (1.0 - sin(0.5 * M_PI * (Se - S0) / kappa));
+  else
+    sigma = 0.0;
+  return sigma < 0.99;
+}
+
+// The energy ratio at which the switch flips: sigma falls with Se, and is 0.99 where the sine is
+// -0.98.  NaN when it is out of the range in which shock_flagged may compare against it.
+inline double shock_cut(double S0, double kappa) {
+  const double q = std::pow(10.0, S0 - kappa * (2.0 / M_PI) * std::asin(0.98));
+  return q > 1e-100 && q < 1e100 ? q : std::nan("");
+}
+
+// shock_switch(log10(top / all), S0, kappa) with q = shock_cut(S0, kappa): the logarithm and the sine
+// are evaluated only within a relative 1e-9 of the cut, a margin far above the rounding errors of
+// the long form (a relative 1e-14 of the ratio), and for values out of range (all not above 1e-150,
+// NaN).  So the outcome is the long form's on every input.
+__device__ __forceinline__ bool shock_flagged(double top, double all, double q, double S0, double kappa) {
+  if (all > 1e-150) {
+    if (top < q * (1.0 - 1e-9) * all) return false;
+    if (top > q * (1.0 + 1e-9) * all) return true;
+  }
+  return shock_switch(log10(top / all), S0, kappa);
 }
 
 // y-direction interface flux: rotate into the face-normal frame n = (0, 1), solve, rotate back

@@ -140,13 +140,14 @@ class FR1D:
     PATHS = {"auto": 0, "batched": 1, "member": 2}
 
     def set_path(self, path: str):
-        """'batched' (a launch per stage), 'member' (one workgroup runs the whole call's stages in
-        a few launches) or 'auto' (member when the problem has at most two work items, i.e. up to
-        508 cells at 256 threads).  Every path gives the same bits."""
+        """'batched' (a launch per stage), 'member' (elements held in registers over several steps
+        per launch) or 'auto' (as 'member'; Tsit5 takes a launch per stage).  Every path gives the
+        same bits."""
         check(_lib.lib().fr1d_set_path(self.h, self.PATHS[path]))
 
     def path(self, scheme: str = "ssprk3") -> str:
-        """The path step() takes for `scheme` under the current setting."""
+        """'batched' where step() takes a launch per stage for `scheme` or, under 'auto', steps a
+        problem of more than 508 cells in chunks; else 'member'."""
         v = C.c_int()
         check(_lib.lib().fr1d_get_path(self.h, _lib.RK[scheme], C.byref(v)))
         return {1: "batched", 2: "member"}[v.value]
@@ -249,8 +250,9 @@ class Ensemble1D:
         check(_lib.lib().fr_ens_step(self.h, 1 if looped else 0, float(dt), int(nsteps)))
 
     def set_path(self, path: str):
-        """Execution path of step() and run(): 'batched', 'member' (a workgroup per member) or
-        'auto' (member when no member has more than two work items); same bits on every path."""
+        """Execution path of step(), run() and their graphs: 'batched' (a launch per stage),
+        'member' (elements held in registers over several steps per launch) or 'auto' (as
+        'member'); same bits on every path."""
         check(_lib.lib().fr_ens_set_path(self.h, FR1D.PATHS[path]))
 
     def step_graph(self, dt: float, nsteps: int, nrep: int = 1):

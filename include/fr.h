@@ -349,16 +349,17 @@ int fr1d_step(fr1d_ctx *ctx, int scheme, double dt, int nsteps);
 /* Execution path of fr1d_step, fr_ens_step and fr_ens_run (same bits on every path; no
  * counterpart in the reference, the path is this library's execution choice):
  * FR1D_PATH_BATCHED: a launch per stage and per dissipation pass over all members' work items;
- * FR1D_PATH_MEMBER: a workgroup per member runs the whole call's schedule (every stage,
- * dissipation pass and copy, a workgroup barrier after each) in launches of up to 3072 operations;
- * FR1D_PATH_AUTO (the default): the member path when no member has more than two work items of
- * the context's workgroup size (up to 508 cells at 256 threads), else batched.  Tsit5,
- * fr_ens_step's mode 1 and the graph entry points always take the batched launches. */
+ * FR1D_PATH_MEMBER: the elements of a member (up to 256 of them, or a chunk of a larger member
+ * with halo elements around it) stay in the registers of a workgroup over several steps per launch;
+ * FR1D_PATH_AUTO (the default): the launches of FR1D_PATH_MEMBER.  Tsit5 and mode 1 of the
+ * ensemble calls always take a launch per stage. */
 #define FR1D_PATH_AUTO 0
 #define FR1D_PATH_BATCHED 1
 #define FR1D_PATH_MEMBER 2
 int fr1d_set_path(fr1d_ctx *ctx, int path);
-/* the path fr1d_step takes for this scheme under the current setting */
+/* FR1D_PATH_BATCHED where fr1d_step takes a launch per stage for this scheme, or, under
+ * FR1D_PATH_AUTO, where a member has more than 508 cells and is stepped in chunks; else
+ * FR1D_PATH_MEMBER */
 int fr1d_get_path(const fr1d_ctx *ctx, int scheme, int *path);
 /* The per-step host loop of example/euler_highlevel.jl:37-52 on the device state (Euler only):
  * modal sensor on rho (su = u_hat[end]^2 / (sum u_hat^2 + 1e-6), shock_detector of
