@@ -7,15 +7,19 @@
 // relaxes to the Maxwellian, du = -(div f + corrections) + (M - f) / tau.
 //
 // State f(i, j, k, l, a, b, member), column-major: the cell index is fastest, so a wavefront of
-// consecutive cells reads contiguous memory for a fixed (point, velocity).  Two kernels per stage:
-// moments (one thread per solution point, loop over the velocities, FP64 sums; it also writes the
-// separable Maxwellian factors of the point) and transport + relaxation + RK stage (one workgroup
-// per (member, velocity, 16 x 16 cell tile), one thread per cell; the upwind traces of the
-// neighbours come from LDS or from the halo threads).
+// consecutive cells reads contiguous memory for a fixed (point, velocity).  Two paths:
+// - states that the caches serve (kBgkStream): moments (one thread per solution point, loop over the velocities, FP64
+//   sums; it also writes the separable Maxwellian factors of the point), then transport + relaxation +
+//   RK stage (one workgroup per (member, velocity, 16 x 16 cell tile), one thread per cell; the upwind
+//   traces of the neighbours come from LDS or from the halo threads);
+// - larger states: a stage kernel that walks a tile through a range of velocities and leaves partial
+//   velocity sums of its result, and a closure that adds them per point and writes the factors, so no
+//   stage reads the state a second time for its moments.
 #include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <new>
+#include <type_traits>
 #include <vector>
 
 #include "fr_common.h"
@@ -25,13 +29,16 @@ namespace fr {
 constexpr int BT = 16;  // tile edge in cells (BT x BT threads)
 
 template <int NSP>
-struct BgkOps {
+struct BgkTileOps {
   double ll[NSP], lr[NSP], dl[NSP * NSP], dhl[NSP], dhr[NSP];
 };
 
 struct BgkGeo {
   int nx, ny, nu, nv, nmem;
-  long long npts;   // nx * ny * nsp^2 (one velocity plane)
+  int per, ngrp;      // velocities per group, groups
+  int tsh;            // log2 of the tile's width
+  long long cells;    // nx * ny
+  long long npts;     // nx * ny * nsp^2 (one velocity plane)
   long long mstride;  // doubles per member
   double iJx, iJy, gamma;
 };
@@ -43,7 +50,7 @@ struct BgkStage {
   int residual;
 };
 
-// moments -> prim (rho, U, V, lambda) per solution point, prim[member][c][pt], and the separable
+// moments cons[member][c][pt] (rho, rho U, rho V, E) of every solution point, and the separable
 // Maxwellian M(a, b) = Ea[a] * Eb[b] of every point: Ea[member][a][pt] = exp(-lambda (u_a - U)^2),
 // Eb[member][b][pt] = rho lambda / pi exp(-lambda (v_b - V)^2), so that the transport kernel spends
 // one multiplication per value on it.  A wavefront takes 64 consecutive points (the lanes); nq
@@ -55,7 +62,7 @@ __global__ __launch_bounds__(64 * MQ) void bgk_moments_kernel(BgkGeo g, const do
                                                               const double *__restrict__ uv,
                                                               const double *__restrict__ vv,
                                                               const double *__restrict__ wu,
-                                                              const double *__restrict__ wv, double *prim,
+                                                              const double *__restrict__ wv, double *cons,
                                                               double *__restrict__ tab, int nq) {
   __shared__ double sm[MQ][4][64];
   __shared__ double sp[MQ][4][64];
@@ -113,11 +120,11 @@ __global__ __launch_bounds__(64 * MQ) void bgk_moments_kernel(BgkGeo g, const do
     sp[grp][2][lane] = V;
     sp[grp][3][lane] = lam;
     if (act) {
-      double *pr = prim + mem * 4 * g.npts + p;
-      pr[0] = rho;
-      pr[g.npts] = U;
-      pr[2 * g.npts] = V;
-      pr[3 * g.npts] = lam;
+      double *o = cons + mem * 4 * g.npts + p;
+      o[0] = mm[0];
+      o[g.npts] = mm[1];
+      o[2 * g.npts] = mm[2];
+      o[3 * g.npts] = mm[3];
     }
   }
   __syncthreads();
@@ -136,7 +143,7 @@ __global__ __launch_bounds__(64 * MQ) void bgk_moments_kernel(BgkGeo g, const do
 }
 
 template <int NSP>
-__global__ __launch_bounds__(BT *BT) void bgk_rhs_kernel(BgkGeo g, BgkOps<NSP> ops, const double *__restrict__ uv,
+__global__ __launch_bounds__(BT *BT) void bgk_rhs_kernel(BgkGeo g, BgkTileOps<NSP> ops, const double *__restrict__ uv,
                                                          const double *__restrict__ vv,
                                                          const double *__restrict__ tau,
                                                          const double *__restrict__ tab, BgkStage sa) {
@@ -273,37 +280,409 @@ __global__ __launch_bounds__(BT *BT) void bgk_rhs_kernel(BgkGeo g, BgkOps<NSP> o
     }
 }
 
+// ------------------------------------------------------------------ states above kBgkStream
+// Cells of a workgroup's tile, 64 x BC/64, 32 x BC/32 or 16 x BC/16 (bgk_tile): 256 where nsp wavefronts
+// per 64 cells leave the registers that a line needs, fewer above.
+template <int NSP>
+constexpr int kBgkCells = NSP <= 3 ? 256 : NSP == 4 ? 128 : 64;
+// whether the stage kernel also sums its result (at nsp = 5 the sums' registers would be spilled)
+template <int NSP>
+constexpr bool kBgkSums = NSP < 5;
+// Bytes of a state up to which the cached path is the faster one.  Three steps, cached path / this one:
+// 8 MB (20 x 33, p = 2, 16 x 11 velocities) 225 / 271 us, 32 MB 328 / 342, 68 MB 620 / 517, 97 MB
+// (57 x 43, p = 2, 24 x 24) 1207 / 727.
+constexpr size_t kBgkStream = 64u << 20;
+
+// Operators by the sign of the velocity component (0: positive, 1: otherwise).  Upwind, only the face
+// towards the neighbour has a correction: D carries its own-trace part, D = dl - dhl ll' (positive) or
+// dl - dhr lr' (D[k][q], rounded once from long double), nb forms the neighbour's trace there, dh
+// weighs it.
+template <int NSP>
+struct BgkOps {
+  double D[2][NSP * NSP], nb[2][NSP], dh[2][NSP];
+};
+
+// per velocity: u iJx, v iJy, the weights w, w u, w v, w (u^2 + v^2) / 2 of the moments, the signs
+// (BgkOps) and the velocity indices
+struct BgkVel {
+  double cx, cy, w[4];
+  int sx, sy, a, b;
+};
+
+// Velocity sums.  The velocities (a fastest) are cut into ngrp groups of `per`; the sums of a group
+// run in velocity order and are kept as part[member][group][moment][point], so the stage kernel
+// (which sums its results as it forms them) and bgk_partial_kernel (which reads a state) give the
+// same bits.
+__device__ __forceinline__ void bgk_add(double *m, const BgkVel &e, double f) {
+#pragma unroll
+  for (int c = 0; c < 4; ++c) m[c] += e.w[c] * f;
+}
+
+__global__ __launch_bounds__(256) void bgk_partial_kernel(BgkGeo g, const double *__restrict__ f,
+                                                          const BgkVel *__restrict__ vt, double *__restrict__ part) {
+  const unsigned nb = (unsigned)((g.npts + 255) / 256);
+  const long long p = (blockIdx.x % nb) * 256LL + threadIdx.x;
+  if (p >= g.npts) return;
+  const int grp = blockIdx.x / nb % g.ngrp, mem = blockIdx.x / nb / g.ngrp;
+  const int v0 = grp * g.per, v1 = min(v0 + g.per, g.nu * g.nv);
+  const double *fb = f + mem * g.mstride + p;
+  double m[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll 8
+  for (int v = v0; v < v1; ++v) bgk_add(m, vt[v], fb[g.npts * v]);
+  double *o = part + ((long long)mem * g.ngrp + grp) * 4 * g.npts + p;
+#pragma unroll
+  for (int c = 0; c < 4; ++c) o[g.npts * c] = m[c];
+}
+
+// Closure: the sums of all groups, the primitive variables (KitBase conserve_prim at gamma) and the
+// separable Maxwellian M(a, b) = Ea[a] * Eb[b] of every point: Ea[member][a][pt] =
+// exp(-lambda (u_a - U)^2), Eb[member][b][pt] = rho lambda / pi exp(-lambda (v_b - V)^2), so that the
+// stage kernel spends one multiplication per value on it.  A wavefront takes 64 consecutive points;
+// the four wavefronts of a workgroup share them and split the groups (group = wavefront mod 4, added
+// in wavefront order) and then the factors.
+__global__ __launch_bounds__(64 * MQ) void bgk_close_kernel(BgkGeo g, const double *__restrict__ part,
+                                                            const double *__restrict__ uv,
+                                                            const double *__restrict__ vv, double *__restrict__ tab) {
+  __shared__ double sm[MQ][4][64];
+  const int lane = threadIdx.x & 63, q = threadIdx.x >> 6;
+  const long long t = blockIdx.x * 64LL + lane;
+  const bool act = t < g.npts * g.nmem;
+  const long long mem = act ? t / g.npts : 0, p = act ? t % g.npts : 0;
+  double m[4] = {0.0, 0.0, 0.0, 0.0};
+  if (act) {
+    const double *pb = part + mem * g.ngrp * 4 * g.npts + p;
+#pragma unroll 4
+    for (int r = q; r < g.ngrp; r += MQ)
+#pragma unroll
+      for (int c = 0; c < 4; ++c) m[c] += pb[g.npts * (4LL * r + c)];
+  }
+#pragma unroll
+  for (int c = 0; c < 4; ++c) sm[q][c][lane] = m[c];
+  __syncthreads();
+  if (!act) return;
+#pragma unroll
+  for (int c = 0; c < 4; ++c) m[c] = (sm[0][c][lane] + sm[1][c][lane]) + (sm[2][c][lane] + sm[3][c][lane]);
+  const double rho = m[0], U = m[1] / m[0], V = m[2] / m[0];
+  const double lam = 0.5 * m[0] / (g.gamma - 1.0) / (m[3] - 0.5 * (m[1] * m[1] + m[2] * m[2]) / m[0]);
+  double *ta = tab + mem * (long long)(g.nu + g.nv) * g.npts + p;
+  for (int a = q; a < g.nu; a += MQ) {
+    const double du = uv[a] - U;
+    ta[g.npts * (long long)a] = exp(-lam * (du * du));
+  }
+  const double c0 = rho * (lam / M_PI);
+  for (int b = q; b < g.nv; b += MQ) {
+    const double dv = vv[b] - V;
+    ta[g.npts * (long long)(g.nu + b)] = c0 * exp(-lam * (dv * dv));
+  }
+}
+
+// Transport + relaxation + RK stage of a tile over one group of velocities.  A thread
+// holds the points (k, line) of one cell, so the line is uniform over a wavefront and the moments of
+// the result stay in 4 nsp registers over the whole group.  Per velocity: the tile and the one upwind
+// column and row go to LDS (two buffers in turn: one barrier), the loads of the next velocity are put
+// in flight, and each thread forms its x sums from its registers and its y sums from LDS.
+// No branch lies around a load or a store, so the waits count them exactly and a wavefront never
+// waits for its own stores: places outside the grid repeat the last cell of their row and column
+// (and store its values again).  COMBINE: with the a0 u0 term.  BUF: buffer access with 32-bit offsets
+// inside one velocity's plane of points (below 4 GiB), which spends no vector instruction on
+// addresses; flat addresses above.
+// 128 x 128, p = 2, 24 x 24 velocities (679 MB a state): 317 us for the first stage, 423 us with u0 (4.6
+// and 5.0 TB/s; a plain copy of 1 GB reaches 5.0), against 135 us of moments and 360 / 578 us of the
+// cached path's transport.  64-cell tiles 357 / 491 us; waits for every load and store 570 us; stores
+// without the streaming hint 4-5 % slower; 128 registers (34 spilled) 1085 us.
+template <int NSP, bool COMBINE, bool BUF>
+__global__ __launch_bounds__(kBgkCells<NSP> *NSP) void bgk_stage_kernel(BgkGeo g, BgkOps<NSP> ops,
+                                                            const BgkVel *__restrict__ vt,
+                                                            const double *__restrict__ tau,
+                                                            const double *__restrict__ tab, BgkStage sa,
+                                                            double *__restrict__ part) {
+  constexpr int NP = NSP * NSP, BC = kBgkCells<NSP>;
+  constexpr int PL = BC + BC / 16 + 17 > BC + BC / 64 + 65 ? BC + BC / 16 + 17 : BC + BC / 64 + 65;  // widest and tallest
+  constexpr int NT = ((BC / 64 + 64) * NP + BC * NSP - 1) / (BC * NSP);  // halo values per thread
+  static_assert(BC % 64 == 0, "the line is uniform over a wavefront");
+  __shared__ double lds[2][NP * PL];
+  const int BTX = 1 << g.tsh, BTY = BC >> g.tsh, RX = BTX + 1, NH = BTX + BTY;
+  const int tiles_x = (g.nx + BTX - 1) / BTX, tiles = tiles_x * ((g.ny + BTY - 1) / BTY);
+  // groups of a tile side by side on one XCD: they read the same factors Ea
+  const int bid = xcd_tile(blockIdx.x, gridDim.x);
+  const int grp = bid % g.ngrp, tile = bid / g.ngrp % tiles, mem = bid / g.ngrp / tiles;
+  const int tid = threadIdx.x, line = __builtin_amdgcn_readfirstlane(tid / BC), c = tid % BC;
+  const int i0 = (tile % tiles_x) * BTX, j0 = (tile / tiles_x) * BTY;
+  const int ncx = min(BTX, g.nx - i0), ncy = min(BTY, g.ny - j0);
+  const int tx = min(c & (BTX - 1), ncx - 1), ty = min(c >> g.tsh, ncy - 1);
+  using OFF = std::conditional_t<BUF, unsigned, unsigned long long>;  // bytes
+  auto at_cell = [&](int i, int j) { return (OFF)8 * ((OFF)i + (OFF)g.nx * (OFF)j); };
+  const OFF kb = (OFF)(8 * g.cells);  // from one point's cells to the next one's
+  // value at byte offset o of point k (uniform) of the plane at base
+  auto get = [&](const double *base, OFF o, int k) {
+    if constexpr (BUF)
+      return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(plane_rsrc(base, 0xFFFFFFFFu), o,
+                                                                             (int)(kb * (OFF)k), 0));
+    else
+      return *reinterpret_cast<const double *>(reinterpret_cast<const char *>(base) + kb * (OFF)k + o);
+  };
+  constexpr int kAuxNt = 2;
+  auto put = [&](double *base, OFF o, int k, double v, auto nt) {
+    if constexpr (BUF)
+      __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(fr_u2, v), plane_rsrc(base, 0xFFFFFFFFu), o,
+                                            (int)(kb * (OFF)k), decltype(nt)::value ? kAuxNt : 0);
+    else
+      *reinterpret_cast<double *>(reinterpret_cast<char *>(base) + kb * (OFF)k + o) = v;
+  };
+  const OFF own = at_cell(i0 + tx, j0 + ty);
+
+  // halo values of this thread: point hp of the upwind row's cell i0 + h (h < BTX) or of the upwind
+  // column's cell j0 + h - BTX, for a positive and another component (periodic wrap), and their
+  // place in LDS but for the sign of the other direction
+  OFF hat[NT][2];
+  int hslot[NT][2], hstep[NT];
+  bool hx[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+    const int n = min(tid + t * BC * NSP, NH * NP - 1), h0 = n % NH, hp = n / NH;
+    hx[t] = h0 >= BTX;
+    const int h = hx[t] ? min(h0 - BTX, ncy - 1) : min(h0, ncx - 1);
+    hstep[t] = hx[t] ? RX : 1;
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      const int hi = hx[t] ? (s == 0 ? (i0 > 0 ? i0 - 1 : g.nx - 1) : (i0 + ncx < g.nx ? i0 + ncx : 0)) : i0 + h;
+      const int hj = hx[t] ? j0 + h : (s == 0 ? (j0 > 0 ? j0 - 1 : g.ny - 1) : (j0 + ncy < g.ny ? j0 + ncy : 0));
+      hat[t][s] = at_cell(hi, hj) + kb * (OFF)hp;
+      hslot[t][s] = hp * PL + (hx[t] ? h * RX + (s == 0 ? 0 : ncx) : (s == 0 ? 0 : ncy) * RX + h);
+    }
+  }
+
+  const long long mb = mem * g.mstride, lb = g.cells * (NSP * line);
+  const double *const Ea = tab + (long long)mem * (g.nu + g.nv) * g.npts + lb;
+  const double *const Eb = Ea + (long long)g.nu * g.npts;
+  struct Vals {
+    double w[NSP], u0[NSP], ea[NSP], h[NT];
+    BgkVel e;
+  } A, B;
+  double eb[NSP];
+  auto load = [&](int v, Vals &r) {
+    r.e = vt[v];
+    const double *const f = sa.u + mb + g.npts * v;
+#pragma unroll
+    for (int k = 0; k < NSP; ++k) r.w[k] = get(f + lb, own, k);
+#pragma unroll
+    for (int t = 0; t < NT; ++t) r.h[t] = get(f, (hx[t] ? r.e.sx : r.e.sy) == 0 ? hat[t][0] : hat[t][1], 0);
+    const double *const ea = Ea + g.npts * r.e.a;
+#pragma unroll
+    for (int k = 0; k < NSP; ++k) r.ea[k] = get(ea, own, k);
+    if constexpr (COMBINE) {
+      const double *const f0 = sa.u0 + mb + g.npts * v + lb;
+#pragma unroll
+      for (int k = 0; k < NSP; ++k) r.u0[k] = get(f0, own, k);
+    }
+  };
+  const int v0 = grp * g.per, v1 = min(v0 + g.per, g.nu * g.nv);
+  const double itau = 1.0 / tau[mem];
+  double m[NSP][4] = {};
+  // operators of the current signs: they change a few times over a group
+  double D[NP], nbx[NSP], dhx[NSP], Dy[NSP], nby[NSP], dhy = 0.0;
+  int px = -1, py = -1, pb = -1;
+
+  auto body = [&](int v, double *buf, const Vals &cur, Vals &nxt) {
+    const int sx = cur.e.sx, sy = cur.e.sy;
+    // own cells one place in from the halo column and row where those lie left and below
+    const int at = (ty + 1 - sy) * RX + tx + 1 - sx;
+#pragma unroll
+    for (int k = 0; k < NSP; ++k) buf[(k + NSP * line) * PL + at] = cur.w[k];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      const int sn = hx[t] ? sx : sy, so = hx[t] ? sy : sx;
+      buf[(sn == 0 ? hslot[t][0] : hslot[t][1]) + (so == 0 ? hstep[t] : 0)] = cur.h[t];
+    }
+    // before the next velocity's loads: the waits for these (now and then) then leave those alone
+    if (cur.e.b != pb) {
+      pb = cur.e.b;
+#pragma unroll
+      for (int k = 0; k < NSP; ++k) eb[k] = get(Eb + g.npts * pb, own, k);
+    }
+    load(min(v + 1, v1 - 1), nxt);
+    if (sx != px) {
+      px = sx;
+#pragma unroll
+      for (int q = 0; q < NP; ++q) D[q] = ops.D[sx][q];
+#pragma unroll
+      for (int q = 0; q < NSP; ++q) {
+        nbx[q] = ops.nb[sx][q];
+        dhx[q] = ops.dh[sx][q];
+      }
+    }
+    if (sy != py) {
+      py = sy;
+#pragma unroll
+      for (int q = 0; q < NSP; ++q) {
+        Dy[q] = ops.D[sy][line * NSP + q];
+        nby[q] = ops.nb[sy][q];
+      }
+      dhy = ops.dh[sy][line];
+    }
+    // barrier over LDS alone: the loads above stay in flight
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    const int dx = sx == 0 ? -1 : 1, dy = sy == 0 ? -RX : RX;
+    double nx = 0.0;
+#pragma unroll
+    for (int q = 0; q < NSP; ++q) nx += nbx[q] * buf[(q + NSP * line) * PL + at + dx];
+    double *const o = sa.out + mb + g.npts * v + lb;
+#pragma unroll
+    for (int k = 0; k < NSP; ++k) {
+      double X = dhx[k] * nx, ny = 0.0, Y = 0.0;
+#pragma unroll
+      for (int q = 0; q < NSP; ++q) {
+        X += D[k * NSP + q] * cur.w[q];
+        Y += Dy[q] * buf[(k + NSP * q) * PL + at];
+        ny += nby[q] * buf[(k + NSP * q) * PL + at + dy];
+      }
+      Y += dhy * ny;
+      double s = (eb[k] * cur.ea[k] - cur.w[k]) * itau - (cur.e.cx * X + cur.e.cy * Y);
+      double t = sa.a1 * cur.w[k];
+      if constexpr (COMBINE) t = sa.a0 * cur.u0[k] + t;
+      s = t + sa.b * s;
+      if constexpr (kBgkSums<NSP>) bgk_add(m[k], cur.e, s);
+      put(o, own, k, s, std::true_type{});
+    }
+  };
+  load(v0, A);
+  for (int v = v0;;) {
+    body(v, lds[0], A, B);
+    if (++v == v1) break;
+    body(v, lds[1], B, A);
+    if (++v == v1) break;
+  }
+  if constexpr (kBgkSums<NSP>) {
+    double *const o = part + ((long long)mem * g.ngrp + grp) * 4 * g.npts + lb;
+#pragma unroll
+    for (int n = 0; n < 4; ++n)
+#pragma unroll
+      for (int k = 0; k < NSP; ++k) put(o + g.npts * n, own, k, m[k][n], std::false_type{});
+  }
+}
+
 // ------------------------------------------------------------------ context
 struct BgkCtx {
   int nx = 0, ny = 0, nsp = 0, nu = 0, nv = 0, nmem = 1;
   double dx = 1, dy = 1, gamma = 2.0;
+  int num_cu = 256;
   HostOps ops;
   size_t len = 0;
   hipStream_t stream = nullptr;
   double *d_vel = nullptr;  // uv | vv | wu | wv
+  BgkVel *d_vt = nullptr;
   double *d_tau = nullptr;
-  double *d_prim = nullptr;
+  double *d_cons = nullptr;  // moments of the last moments launch
+  double *d_part = nullptr;  // sums of the velocity groups (large states)
   double *d_tab = nullptr;  // Maxwellian factors Ea | Eb per member
   double *d_u = nullptr, *d_s1 = nullptr, *d_s2 = nullptr, *d_in = nullptr, *d_out = nullptr;
 
-  BgkGeo geo() const {
+  long long bgk_tiles(int cells, int sh) const {
+    const int tx = 1 << sh, ty = cells >> sh;
+    return (long long)((nx + tx - 1) / tx) * ((ny + ty - 1) / ty);
+  }
+
+  BgkGeo geom;
+  const BgkGeo &geo() const { return geom; }
+
+  BgkGeo plan() const {
     BgkGeo g;
     g.nx = nx;
     g.ny = ny;
     g.nu = nu;
     g.nv = nv;
     g.nmem = nmem;
-    g.npts = (long long)nx * ny * nsp * nsp;
-    g.mstride = g.npts * nu * nv;
     g.iJx = 2.0 / dx;
     g.iJy = 2.0 / dy;
+    g.cells = (long long)nx * ny;
+    g.npts = g.cells * nsp * nsp;
+    g.mstride = g.npts * nu * nv;
     g.gamma = gamma;
+    // the tile that covers the grid with the fewest cells, the widest of equals
+    const int bc = nsp <= 3 ? kBgkCells<3> : nsp == 4 ? kBgkCells<4> : kBgkCells<5>;
+    long long best = 0;
+    for (int sh = 6; sh >= 4; --sh) {
+      const long long n = bgk_tiles(bc, sh);
+      if (!best || n < best) best = n, g.tsh = sh;
+    }
+    // Groups: workgroups of one size in rounds of one per CU, so the time goes as rounds x
+    // velocities per group; the fewer rounds the better beside that (128 x 128,
+    // p = 2, three steps: 1 round 3.45 ms, 2 rounds 3.82, 3 rounds 3.96)
+    const long long nvel = (long long)nu * nv;
+    double cost = 0.0;
+    for (long long n = 1; n <= std::max(1LL, nvel / 4); ++n) {
+      const long long per = (nvel + n - 1) / n, rounds = (best * nmem * n + num_cu - 1) / num_cu;
+      const double t = (double)(rounds * per) * (1.0 + 0.15 * (double)(rounds - 1));
+      if (n == 1 || t < cost) cost = t, g.per = (int)per;
+    }
+    g.ngrp = (int)((nvel + g.per - 1) / g.per);
     return g;
   }
 
   template <int NSP>
-  int launch_rhs(const BgkStage &sa, hipStream_t st) const {
+  int launch_stage(const BgkStage &sa, hipStream_t st) const {
     BgkOps<NSP> o;
+    for (int s = 0; s < 2; ++s) {
+      const double *t = s ? ops.lr : ops.ll, *dh = s ? ops.dhr : ops.dhl;
+      for (int k = 0; k < NSP; ++k) {
+        o.nb[s][k] = s ? ops.ll[k] : ops.lr[k];
+        o.dh[s][k] = dh[k];
+        for (int q = 0; q < NSP; ++q)
+          o.D[s][k * NSP + q] = (double)((long double)ops.dl[k + NSP * q] - (long double)t[q] * (long double)dh[k]);
+      }
+    }
+    const BgkGeo &g = geo();
+    const long long tiles = bgk_tiles(kBgkCells<NSP>, g.tsh);
+    const bool buf = g.npts < (1LL << 29);
+    auto go = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, dim3((unsigned)(tiles * g.ngrp * nmem)), dim3(kBgkCells<NSP> * NSP), 0, st, g, o, d_vt, d_tau,
+                         d_tab, sa, d_part);
+    };
+    if (sa.a0 == 0.0)
+      buf ? go(bgk_stage_kernel<NSP, false, true>) : go(bgk_stage_kernel<NSP, false, false>);
+    else
+      buf ? go(bgk_stage_kernel<NSP, true, true>) : go(bgk_stage_kernel<NSP, true, false>);
+    FR_LAUNCHED("bgk_stage_kernel");
+    return FR_OK;
+  }
+
+  // velocity sums of a state
+  int launch_partial(const double *d_f, hipStream_t st) const {
+    const BgkGeo &g = geo();
+    hipLaunchKernelGGL(bgk_partial_kernel, dim3((unsigned)((g.npts + 255) / 256 * g.ngrp * nmem)), dim3(256), 0, st, g, d_f, d_vt, d_part);
+    FR_LAUNCHED("bgk_partial_kernel");
+    return FR_OK;
+  }
+
+  int launch_close(hipStream_t st) const {
+    const BgkGeo &g = geo();
+    hipLaunchKernelGGL(bgk_close_kernel, dim3((unsigned)((g.npts * nmem + 63) / 64)), dim3(64 * MQ), 0, st, g, d_part,
+                       d_vel, d_vel + nu, d_tab);
+    FR_LAUNCHED("bgk_close_kernel");
+    return FR_OK;
+  }
+
+  // one stage of sa.u, whose velocity sums are in d_part; leaves those of the result there
+  int stage_large(const BgkStage &sa, hipStream_t st) const {
+    int rc = launch_close(st);
+    if (rc) return rc;
+    switch (nsp) {
+      case 2: return launch_stage<2>(sa, st);
+      case 3: return launch_stage<3>(sa, st);
+      case 4: return launch_stage<4>(sa, st);
+      default: rc = launch_stage<5>(sa, st);
+    }
+    return rc ? rc : launch_partial(sa.out, st);  // kBgkSums<5>
+  }
+
+  int stage(const BgkStage &sa, hipStream_t st) const { return large() ? stage_large(sa, st) : stage_cached(sa, st); }
+
+  template <int NSP>
+  int launch_rhs(const BgkStage &sa, hipStream_t st) const {
+    BgkTileOps<NSP> o;
     for (int q = 0; q < NSP; ++q) {
       o.ll[q] = ops.ll[q];
       o.lr[q] = ops.lr[q];
@@ -311,7 +690,7 @@ struct BgkCtx {
       o.dhr[q] = ops.dhr[q];
     }
     for (int q = 0; q < NSP * NSP; ++q) o.dl[q] = ops.dl[q];
-    const BgkGeo g = geo();
+    const BgkGeo &g = geo();
     const long long tiles = (long long)((nx + BT - 1) / BT) * ((ny + BT - 1) / BT);
     const long long nb = tiles * nu * nv * nmem;
     hipLaunchKernelGGL(bgk_rhs_kernel<NSP>, dim3((unsigned)nb), dim3(BT * BT), 0, st, g, o, d_vel, d_vel + nu,
@@ -323,20 +702,22 @@ struct BgkCtx {
   // moments kernel launch: nq wavefronts per group of 64 points, enough for about eight
   // wavefronts per SIMD; MQ / nq point groups per workgroup
   int launch_moments(const double *d_f, hipStream_t st) const {
-    const BgkGeo g = geo();
+    const BgkGeo &g = geo();
     const long long n = g.npts * nmem, groups = (n + 63) / 64;
     int nq = 1;
     while (nq < MQ && groups * nq < 8LL * 1024) nq *= 2;
     const long long nb = (groups + (MQ / nq) - 1) / (MQ / nq);
     hipLaunchKernelGGL(bgk_moments_kernel, dim3((unsigned)nb), dim3(64 * MQ), 0, st, g, d_f, d_vel, d_vel + nu,
-                       d_vel + nu + nv, d_vel + 2 * nu + nv, d_prim, d_tab, nq);
+                       d_vel + nu + nv, d_vel + 2 * nu + nv, d_cons, d_tab, nq);
     FR_LAUNCHED("bgk_moments_kernel");
     return FR_OK;
   }
 
-  int stage(const BgkStage &sa, hipStream_t st) const {
-    int rc0 = launch_moments(sa.u, st);
-    if (rc0) return rc0;
+  bool large() const { return len * sizeof(double) > kBgkStream; }
+
+  int stage_cached(const BgkStage &sa, hipStream_t st) const {
+    const int rc = launch_moments(sa.u, st);
+    if (rc) return rc;
     switch (nsp) {
       case 2: return launch_rhs<2>(sa, st);
       case 3: return launch_rhs<3>(sa, st);
@@ -347,9 +728,10 @@ struct BgkCtx {
 
   void release() {
     if (stream) (void)hipStreamSynchronize(stream);
-    double *bufs[] = {d_vel, d_tau, d_prim, d_tab, d_u, d_s1, d_s2, d_in, d_out};
+    double *bufs[] = {d_vel, d_tau, d_cons, d_part, d_tab, d_u, d_s1, d_s2, d_in, d_out};
     for (double *b : bufs)
       if (b) (void)hipFree(b);
+    if (d_vt) (void)hipFree(d_vt);
     if (stream) (void)hipStreamDestroy(stream);
   }
 };
@@ -388,19 +770,35 @@ int fr_bgk_create(fr_bgk_ctx **out, const fr_bgk_desc *d) {
     delete c;
     return fail(FR_E_INVALID, "fr_bgk_create: operator construction failed");
   }
-  const BgkGeo g = c->geo();
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&c->num_cu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || c->num_cu < 1)
+    c->num_cu = 256;
+  c->geom = c->plan();
+  const BgkGeo &g = c->geom;
   c->len = (size_t)g.mstride * d->nmem;
   std::vector<double> vel;
   vel.insert(vel.end(), d->u, d->u + d->nu);
   vel.insert(vel.end(), d->v, d->v + d->nv);
   vel.insert(vel.end(), d->wu, d->wu + d->nu);
   vel.insert(vel.end(), d->wv, d->wv + d->nv);
+  std::vector<BgkVel> vt;
+  for (int b = 0; b < d->nv; ++b)
+    for (int a = 0; a < d->nu; ++a) {
+      const double u = d->u[a], v = d->v[b], w = d->wu[a] * d->wv[b];
+      vt.push_back({u * (2.0 / d->dx), v * (2.0 / d->dy), {w, w * u, w * v, w * 0.5 * (u * u + v * v)},
+                    u > 0.0 ? 0 : 1, v > 0.0 ? 0 : 1, a, b});
+    }
   hipError_t e = hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking);
   if (e == hipSuccess) e = hipMalloc(&c->d_vel, vel.size() * sizeof(double));
   if (e == hipSuccess) e = hipMemcpy(c->d_vel, vel.data(), vel.size() * sizeof(double), hipMemcpyHostToDevice);
+  if (e == hipSuccess) e = hipMalloc(&c->d_vt, vt.size() * sizeof(BgkVel));
+  if (e == hipSuccess) e = hipMemcpy(c->d_vt, vt.data(), vt.size() * sizeof(BgkVel), hipMemcpyHostToDevice);
   if (e == hipSuccess) e = hipMalloc(&c->d_tau, d->nmem * sizeof(double));
   if (e == hipSuccess) e = hipMemcpy(c->d_tau, d->tau, d->nmem * sizeof(double), hipMemcpyHostToDevice);
-  if (e == hipSuccess) e = hipMalloc(&c->d_prim, (size_t)g.npts * 4 * d->nmem * sizeof(double));
+  if (e == hipSuccess) e = hipMalloc(&c->d_cons, (size_t)g.npts * 4 * d->nmem * sizeof(double));
+  if (e == hipSuccess && c->large())
+    e = hipMalloc(&c->d_part, (size_t)g.npts * 4 * g.ngrp * d->nmem * sizeof(double));
   if (e == hipSuccess) e = hipMalloc(&c->d_tab, (size_t)g.npts * (d->nu + d->nv) * d->nmem * sizeof(double));
   if (e == hipSuccess) e = hipMalloc(&c->d_u, c->len * sizeof(double));
   if (e != hipSuccess) {
@@ -429,7 +827,7 @@ int fr_bgk_rhs(fr_bgk_ctx *c, const double *f, double *df) {
   if (!c->d_out) FR_HIP(hipMalloc(&c->d_out, bytes));
   FR_HIP(hipMemcpyAsync(c->d_in, f, bytes, hipMemcpyHostToDevice, c->stream));
   BgkStage sa{c->d_in, nullptr, c->d_out, 0.0, 0.0, 0.0, 1};
-  int rc = c->stage(sa, c->stream);
+  int rc = c->stage_cached(sa, c->stream);
   if (rc) return rc;
   FR_HIP(hipMemcpyAsync(df, c->d_out, bytes, hipMemcpyDeviceToHost, c->stream));
   FR_HIP(hipStreamSynchronize(c->stream));
@@ -457,15 +855,16 @@ int fr_bgk_get_state(fr_bgk_ctx *c, double *f) {
   return FR_OK;
 }
 
-// nsteps Shu-Osher SSP-RK3 steps of all members; each stage = moments + transport/relaxation
+// nsteps Shu-Osher SSP-RK3 steps of all members; each stage = closure + transport/relaxation
 int fr_bgk_step(fr_bgk_ctx *c, double dt, int nsteps) {
   FR_REQUIRE(c && nsteps >= 0 && std::isfinite(dt), FR_E_INVALID, "fr_bgk_step: bad arguments");
   if (!c->d_s1) FR_HIP(hipMalloc(&c->d_s1, c->len * sizeof(double)));
   if (!c->d_s2) FR_HIP(hipMalloc(&c->d_s2, c->len * sizeof(double)));
   // Consecutive steps alternate the state between d_u and d_s1 (every stage writes every value),
   // so the last stage never writes the u^n it reads; the call's last step writes d_u.
+  int rc = nsteps > 0 && c->large() ? c->launch_partial(c->d_u, c->stream) : FR_OK;
+  if (rc) return rc;
   for (int n = 0; n < nsteps; ++n) {
-    int rc;
     double *const X = (n & 1) ? c->d_s1 : c->d_u, *const Y = (n & 1) ? c->d_u : c->d_s1;
     double *const out = n == nsteps - 1 ? c->d_u : Y;
     if ((rc = c->stage(BgkStage{X, X, Y, 0.0, 1.0, dt, 0}, c->stream))) return rc;
@@ -481,24 +880,11 @@ int fr_bgk_step(fr_bgk_ctx *c, double dt, int nsteps) {
 // output w[member][c][pt]
 int fr_bgk_moments(fr_bgk_ctx *c, double *w) {
   FR_REQUIRE(c && w, FR_E_INVALID, "fr_bgk_moments: null argument");
-  const BgkGeo g = c->geo();
-  const long long n = g.npts * c->nmem;
   int rc = c->launch_moments(c->d_u, c->stream);
   if (rc) return rc;
-  std::vector<double> prim((size_t)n * 4);
-  FR_HIP(hipMemcpyAsync(prim.data(), c->d_prim, prim.size() * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+  const size_t bytes = (size_t)c->geo().npts * 4 * c->nmem * sizeof(double);
+  FR_HIP(hipMemcpyAsync(w, c->d_cons, bytes, hipMemcpyDeviceToHost, c->stream));
   FR_HIP(hipStreamSynchronize(c->stream));
-  // prim -> conserved (KitBase prim_conserve)
-  for (long long mem = 0; mem < c->nmem; ++mem)
-    for (long long p = 0; p < g.npts; ++p) {
-      const double *pr = prim.data() + mem * 4 * g.npts + p;
-      const double rho = pr[0], U = pr[g.npts], V = pr[2 * g.npts], lam = pr[3 * g.npts];
-      double *o = w + mem * 4 * g.npts + p;
-      o[0] = rho;
-      o[g.npts] = rho * U;
-      o[2 * g.npts] = rho * V;
-      o[3 * g.npts] = 0.5 * rho / lam / (c->gamma - 1.0) + 0.5 * rho * (U * U + V * V);
-    }
   return FR_OK;
 }
 

@@ -1,0 +1,39 @@
+"""The 2D BGK stage kernel of states above 64 MiB (a tile walked through a group of velocities, the
+moments summed on the way) against the CPU oracle, on grids with partial tiles of every width."""
+import numpy as np
+import pytest
+
+from frhip import bgk
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("nx,ny,deg,nu,nv,nmem", [(67, 61, 1, 23, 24, 1), (37, 29, 2, 21, 22, 2),
+                                                  (130, 5, 3, 31, 29, 1), (21, 23, 4, 26, 27, 1),
+                                                  (8, 9, 2, 124, 123, 1)])
+def test_large_state_step_parity(nx, ny, deg, nu, nv, nmem):
+    u, wu = bgk.velocity_grid(nu)
+    v, wv = bgk.velocity_grid(nv)
+    taus = np.array([1e-2, 1e-1])[:nmem]
+    f0 = bgk.maxwellian_state(nx, ny, deg, u, v, amp=0.1, nmem=nmem)
+    f0 = f0 * (1.0 + 0.02 * np.random.default_rng(nx).uniform(-1, 1, size=f0.size))
+    assert f0.nbytes > 64 << 20
+    dt = 0.1 / (deg + 1) / max(nx, ny) / np.abs(u).max()
+    g = bgk.BGK2D(nx, ny, deg, u, wu, v, wv, taus)
+    g.set_state(f0)
+    g.step(dt, 1)
+    out = g.get_state().reshape(nmem, -1)
+    # one step: dt L is below f, and L agrees to 1e-12 of its largest value
+    for f, got, tau in zip(f0.reshape(nmem, -1), out, taus):
+        L = lambda x: O.bgk2d_rhs(x, nx, ny, deg, u, wu, v, wv, tau).ravel()  # noqa: E731
+        a = f + dt * L(f)
+        b = 0.75 * f + 0.25 * a + 0.25 * dt * L(a)
+        ref = f / 3 + 2 / 3 * b + 2 / 3 * dt * L(b)
+        assert np.linalg.norm(got - ref) <= 1e-12 * np.linalg.norm(ref)
+    # the sums of a state and those of the stage that made it agree: a split call gives the same bits
+    g.step(dt, 1)
+    two = g.get_state()
+    g.set_state(f0)
+    g.step(dt, 2)
+    assert np.array_equal(g.get_state(), two)
