@@ -168,7 +168,7 @@ def main():
     ap.add_argument("--no-cpu", action="store_true", help="skip the CPU baseline leg")
     ap.add_argument("--stagger", type=int, default=None,
                     help="fix the stage launches' staggered-start delay (units of 512 clocks) instead of the "
-                         "library's device timing, e.g. under a profiler, whose dispatch handling skews that timing")
+                         "library's")
     ap.add_argument("--no-extras", action="store_true", help="only the headline 2D Euler measurement")
     ap.add_argument("--copy-calibration", action="store_true",
                     help="also run 10 plain device copies of 64 MiB (reference kernel for HBM counters)")
@@ -199,8 +199,7 @@ def main():
     solver.set_state(u0)
     # The timed steps replay a hipGraph of CHUNK SSP-RK3 steps that the context captured and
     # replayed once during the warm-up, so that no first-replay cost falls in the timed region
-    # (the remainder runs as eager launches).  Warm-up: the capture and one replay (the context's
-    # first stepping call also tunes its staggered start), the W eager steps, then eager steps up
+    # (the remainder runs as eager launches).  Warm-up: the capture and one replay, the W eager steps, then eager steps up
     # to SETTLE_STEPS in all, about 30 ms of sustained launches, so that the clocks have settled
     # as they have in any longer run.  The state is reset on the device before timing.
     chunk = max(1, min(GRAPH_CHUNK, args.steps))

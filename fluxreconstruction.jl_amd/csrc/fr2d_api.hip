@@ -209,13 +209,7 @@ static int prepare_step(Fr2dCtx &c, int scheme, hipStream_t st) {
   // the stage buffers take the state's ghost layer inside the first stage of every step
   (void)st;
   int rc = ensure_stage_buffers(c, scheme == FR_RK_RK4, scheme == FR_RK_TSIT5);
-  // the first stepping call of a context picks the staggered-start delay on the device, on the
-  // context's own stream (so a caller stream under capture records nothing of it); it reads the
-  // state and writes only the first stage buffer, which the steps overwrite
-  if (!rc && c.stagger < 0) {
-    if ((rc = fr2d_tune_stagger(c, c.own_stream))) return rc;
-    FR_HIP(hipStreamSynchronize(c.own_stream));
-  }
+  if (!rc && c.stagger < 0) c.stagger = fr2d_default_stagger(c);
   return rc;
 }
 

@@ -768,59 +768,14 @@ bool fr2d_single_round(const Fr2dCtx &c) {
          nb <= 4LL * c.num_cu;
 }
 
-// Times the stage launches of SSP-RK3 steps (state and second stage buffer -> first stage buffer,
-// both buffers scratch here) for each stagger candidate, interleaved over four passes after a
-// warm-up, and keeps the fastest.  The state is only read; st must not be capturing (the timing
-// synchronises on an event).
-int fr2d_tune_stagger(Fr2dCtx &c, hipStream_t st) {
-  if (!fr2d_single_round(c)) {
-    c.stagger = 0;
-    return FR_OK;
-  }
-  static const int cand[] = {0, 3, 4, 5, 6, 7};  // units of s_sleep(8): 0 to 3584 clocks per slot
-  constexpr int NC = sizeof(cand) / sizeof(cand[0]), LAUNCH = 18, PASSES = 4;
-  float best[NC];
-  for (int k = 0; k < NC; ++k) best[k] = 1e30f;
-  hipEvent_t e0, e1;
-  FR_HIP(hipEventCreate(&e0));
-  FR_HIP(hipEventCreate(&e1));
-  const int keep = c.stagger;
-  int rc = FR_OK;
-  // the launch mix of an SSP-RK3 step: one stage reading the state (16 B/DOF), two reading the
-  // state and a second array (24 B/DOF); results go to the first stage buffer
-  auto run = [&](int n) {
-    for (int q = 0; q < n && rc == FR_OK; ++q)
-      rc = (q % 3 == 0) ? fr2d_launch_stage(c, c.d_u, c.d_u, c.d_s1, 0.0, 1.0, 1e-9, nullptr, nullptr, 0.0, st)
-                        : fr2d_launch_stage(c, c.d_s2, c.d_u, c.d_s1, 0.75, 0.25, 1e-9, nullptr, nullptr, 0.0, st);
-  };
-  c.stagger = 0;
-  run(1500);  // the clocks settle under sustained load (about 27 ms at 256^2)
-  for (int pass = 0; pass < PASSES && rc == FR_OK; ++pass)
-    for (int k = 0; k < NC && rc == FR_OK; ++k) {
-      c.stagger = cand[k];
-      hipError_t e = hipEventRecord(e0, st);
-      run(LAUNCH);
-      if (e == hipSuccess) e = hipEventRecord(e1, st);
-      if (e == hipSuccess) e = hipEventSynchronize(e1);
-      float ms = 0.f;
-      if (e == hipSuccess) e = hipEventElapsedTime(&ms, e0, e1);
-      if (e != hipSuccess) {
-        rc = hip_fail(e, "fr2d_tune_stagger", __FILE__, __LINE__);
-        break;
-      }
-      best[k] = std::min(best[k], ms);
-    }
-  (void)hipEventDestroy(e0);
-  (void)hipEventDestroy(e1);
-  if (rc) {
-    c.stagger = keep;
-    return rc;
-  }
-  int bi = 0;
-  for (int k = 1; k < NC; ++k)
-    if (best[k] < best[bi]) bi = k;
-  c.stagger = cand[bi];
-  return FR_OK;
+// Delay of the staggered start for a context that has none set.  20 SSP-RK3 steps in us with 0 / 3 / 5 / 7
+// units: Rusanov 256 x 256 periodic 1103 / 1052 / 1056 / 1188, with ghosts 1228 / 1167 / 1178 / 1314,
+// 256 x 240 1173 / 1138 / 1154 / 1262, parallelograms 300 x 200 1114 / 1106 / 1115 / 1243, 250 x 199
+// 1117 / 1104 / 1112 / 1139, 200 x 150 (two workgroups per CU) 679 / 676 / 676 / 676; HLL 256 x 256
+// 1296 / 1297 / 1294 / 1293 and 180 x 180 968 / 973 / 972 / 974.  Timing the candidates on the device
+// in a context's first call chose no better and cost that call 34 ms.
+int fr2d_default_stagger(const Fr2dCtx &c) {
+  return fr2d_single_round(c) && c.flux == FR_FLUX_RUSANOV ? 3 : 0;
 }
 
 int fr2d_launch_fill_ghost(const Fr2dCtx &c, double *d_u, int rule, hipStream_t st) {

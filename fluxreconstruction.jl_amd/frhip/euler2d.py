@@ -193,15 +193,14 @@ class FREuler2D:
         return p.value, q.value
 
     def stagger(self) -> int:
-        """Staggered-start delay of the RK stage launches picked on the device by the context's
-        first stepping call (units of 512 clocks per workgroup slot; 0 off, -1 not tuned yet)."""
+        """Staggered-start delay of the RK stage launches (units of 512 clocks per workgroup slot; 0
+        off, -1 not set yet: the first stepping call takes the library's)."""
         v = C.c_int(0)
         check(_lib.lib().fr2d_get_stagger(self.h, C.byref(v)))
         return v.value
 
     def set_stagger(self, stagger: int) -> None:
-        """Fix the staggered-start delay (0..16; 0 off) instead of the first stepping call's device
-        timing, or (-1) have the next stepping call time the candidates again."""
+        """Fix the staggered-start delay (0..16; 0 off), or (-1) go back to the library's."""
         check(_lib.lib().fr2d_set_stagger(self.h, int(stagger)))
 
     def step(self, dt: float, nsteps: int = 1, scheme: str = "ssprk3"):

@@ -244,7 +244,7 @@ def parallelogram_stage(n=256, steps=20, shear=0.4, stagger=None):
     b = (shear dx, dy), x faces in the frame of grad r, y faces in that of grad s), Rusanov,
     periodic, the isentropic vortex; 20 graph-replayed steps after 300 eager ones, HIP events on the
     launch stream.  Algorithmic bytes: 21.33 per DOF and stage (the metric is two scalars).
-    stagger: a fixed staggered-start delay instead of the device timing (fr2d_set_stagger)."""
+    stagger: a fixed staggered-start delay instead of the library's (fr2d_set_stagger)."""
     import torch
 
     ps = FRPSpace2D(0.0, 10.0, n, 0.0, 10.0, n, 3, 1, 1)
@@ -378,7 +378,7 @@ def main():
     ap.add_argument("--steps", type=int, default=None)
     ap.add_argument("--mode", default="modal", choices=["modal", "learned", "off"])
     ap.add_argument("--stagger", type=int, default=None,
-                    help="parallelogram: fixed staggered-start delay (e.g. under a profiler)")
+                    help="parallelogram: fixed staggered-start delay")
     a = ap.parse_args()
     if a.workload == "ensemble":
         r = riemann_ensemble(a.steps or 10)

@@ -195,16 +195,14 @@ int fr2d_step(fr2d_ctx *ctx, int scheme, double dt, int nsteps);
  * stream (asynchronous, like fr2d_step); the context keeps the instantiated graph and reuses it
  * while scheme, dt and nsteps are unchanged.  No reference counterpart (a replay of fr2d_step). */
 int fr2d_step_graph(fr2d_ctx *ctx, int scheme, double dt, int nsteps, int nrep);
-/* No reference counterpart (launch tuning of this library): the staggered-start delay the
- * context's first stepping call picked on the device for its RK stage launches, in units of 512
- * clocks per workgroup slot of a CU (0: off, -1: not tuned yet).  Grids whose tiles are all
+/* No reference counterpart (launch tuning of this library): the staggered-start delay of
+ * the context's RK stage launches, in units of 512 clocks per workgroup slot of a CU (0: off, -1: not
+ * set yet, the first stepping call takes the library's).  Grids whose tiles are all
  * resident at once start the workgroups sharing a CU one after another, so that their load phases
  * do not coincide; the delay changes the timing only, never the results. */
 int fr2d_get_stagger(const fr2d_ctx *ctx, int *stagger);
 /* No reference counterpart (launch tuning of this library): fixes the staggered-start delay (0..16
- * units; 0 off) instead of the device timing of the first stepping call, or (-1) asks the next
- * stepping call to time the candidates again.  For runs whose timing of the candidates is not
- * representative, such as runs under a profiler; only the timing changes, never the results. */
+ * units; 0 off), or (-1) goes back to the library's.  Only the timing changes, never the results. */
 int fr2d_set_stagger(fr2d_ctx *ctx, int stagger);
 /* No counterpart in the reference: fr2d_step for callers that cannot allocate device memory (code
  * under HIP graph capture, tight serving loops, harnesses that forbid hipMalloc).  nsteps steps
