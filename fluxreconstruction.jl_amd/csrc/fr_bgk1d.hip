@@ -9,7 +9,7 @@
 //   w f, w u f and w u^2 f / 2 (KitBase moments_conserve), then the primitive variables at gamma (conserve_prim:
 //   rho, U, lambda) of the point and the Maxwellian's prefactor rho sqrt(lambda / pi), so that the
 //   transport kernel spends one exp per value on M;
-// - transport + relaxation + RK stage: one thread per (member, cell, 8 velocities).  f = u_j u / J, the
+// - transport + relaxation + RK stage: one thread per (member, cell, up to 8 velocities).  f = u_j u / J, the
 //   traces f . ll and f . lr, the upwind interface value (the Heaviside blend of the script picks
 //   the left cell's right trace for u_j > 0, the right cell's left trace otherwise; the other term
 //   of the blend is the other trace times zero), the derivative, the Radau corrections and
@@ -56,7 +56,7 @@ struct Bgk1dStage {
 // - S = 1 (P = 64): each thread sums all slices of its point itself; for large states, where one
 //   thread per point already fills the chip.
 constexpr int kMomSlices = 8;
-constexpr int kMomSplitPts = 32;
+constexpr int kMomSplitPts = 64;
 constexpr long long kMomSplitBelow = 262144;  // points: below, S = kMomSlices
 
 // U, lambda and rho sqrt(lambda / pi) of a point from its moments (rho, rho U, 2E) (conserve_prim
@@ -76,7 +76,8 @@ __global__ __launch_bounds__(S * P) void bgk1d_moments_kernel(Bgk1dGeo g, const 
                                                               const double *__restrict__ wv, double *prim) {
   static_assert(S == 1 || S == kMomSlices, "one thread per point or one per slice");
   __shared__ double part[S > 1 ? S - 1 : 1][3][P];
-  const int lane = threadIdx.x % P, s = threadIdx.x / P;
+  static_assert(P == 64, "the slice is uniform over a wavefront: its velocities and weights are scalar loads");
+  const int lane = threadIdx.x % P, s = __builtin_amdgcn_readfirstlane(threadIdx.x / P);
   const long long t = blockIdx.x * (long long)P + lane;
   const bool act = t < g.npts * g.nmem;
   const long long mem = act ? t / g.npts : 0, p = act ? t % g.npts : 0;
@@ -142,23 +143,32 @@ __global__ __launch_bounds__(S * P) void bgk1d_moments_kernel(Bgk1dGeo g, const 
   bgk1d_close(m0, m1, m2, g.gamma, pr[g.npts], pr[2 * g.npts], pr[3 * g.npts]);
 }
 
+// x / d with r = 1 / d at hand (d = 0 for an infinite divisor): the quotient by the reciprocal and one
+// correction by its exact remainder, the division's result but for the rarest of last bits (three
+// operations, not ten)
+__device__ __forceinline__ double div_by(double x, double d, double r) {
+  const double q = x * r;
+  return fma(fma(-q, d, x), r, q);
+}
+
+// Relaxation time of a member as div_by takes it.
+struct Bgk1dTau {
+  double d, r;
+  __device__ __forceinline__ explicit Bgk1dTau(double tau) : d(isinf(tau) ? 0.0 : tau), r(1.0 / tau) {}
+};
+
 // res[k] of the transport/relaxation operator (bgk_wave.jl:84-128) at one cell and velocity vel,
 // every point k: f = vel u / J, the upwind interface value (the neighbour's trace: the left cell's
 // right trace for vel > 0, the right cell's left trace otherwise), derivative and Radau
-// corrections, plus (M - u) / tau with M = c0 exp(-lambda (vel - U)^2).  u holds the state values
-// at base + kst k (the cell) and nbase + kst k (the upwind neighbour); w receives the cell's own.
-// Shared by the streaming and the LDS-resident kernels, so both give the same bits.
+// corrections, plus (M - u) / tau with M = c0 exp(-lambda (vel - U)^2).  w: the cell's values, un: the
+// upwind neighbour's.  Shared by the streaming and the LDS-resident kernels, so both give the same bits.
 template <int NSP>
-__device__ __forceinline__ void bgk1d_cell_velocity(const Bgk1dOps &ops, double iJ, const double *__restrict__ u,
-                                                    long long base, long long nbase, long long kst, double vel,
-                                                    bool pos, const double *U, const double *lam, const double *c0,
-                                                    double tv, double *w, double *res) {
+__device__ __forceinline__ void bgk1d_cell_velocity(const Bgk1dOps &ops, double iJ, const double *w, const double *un,
+                                                    double vel, bool pos, const double *U, const double *lam,
+                                                    const double *c0, const Bgk1dTau &tau, double *res) {
   double f[NSP];
 #pragma unroll
-  for (int k = 0; k < NSP; ++k) {
-    w[k] = u[base + kst * k];
-    f[k] = vel * w[k] * iJ;
-  }
+  for (int k = 0; k < NSP; ++k) f[k] = vel * w[k] * iJ;
   double tl = 0.0, tr = 0.0;
 #pragma unroll
   for (int k = 0; k < NSP; ++k) {
@@ -167,7 +177,7 @@ __device__ __forceinline__ void bgk1d_cell_velocity(const Bgk1dOps &ops, double 
   }
   double nb = 0.0;
 #pragma unroll
-  for (int k = 0; k < NSP; ++k) nb += vel * u[nbase + kst * k] * iJ * (pos ? ops.lr[k] : ops.ll[k]);
+  for (int k = 0; k < NSP; ++k) nb += vel * un[k] * iJ * (pos ? ops.lr[k] : ops.ll[k]);
   const double iL = pos ? nb : tl, iR = pos ? tr : nb;
 #pragma unroll
   for (int k = 0; k < NSP; ++k) {
@@ -176,35 +186,42 @@ __device__ __forceinline__ void bgk1d_cell_velocity(const Bgk1dOps &ops, double 
     for (int q = 0; q < NSP; ++q) r1 += f[q] * ops.dl[k + NSP * q];
     const double c = vel - U[k];
     const double M = c0[k] * exp(-lam[k] * (c * c));
-    res[k] = -(r1 + (iL - tl) * ops.dhl[k] + (iR - tr) * ops.dhr[k]) + (M - w[k]) / tv;
+    res[k] = -(r1 + (iL - tl) * ops.dhl[k] + (iR - tr) * ops.dhr[k]) + div_by(M - w[k], tau.d, tau.r);
   }
 }
 
-// a0 u0 + a1 u + b res, the stage combination (u0 read only when a0 != 0)
-__device__ __forceinline__ double bgk1d_combine(double a0, double a1, double b, double w, const double *u0,
-                                                long long o, double res) {
+// a0 u0 + a1 u + b res, the stage combination (u0 left out when a0 = 0); the roundings are spelled out,
+// so that an instance that knows a0 gives the same bits as one that does not
+__device__ __forceinline__ double bgk1d_combine(double a0, double a1, double b, double w, double u0, double res) {
   double v = a1 * w;
-  if (a0 != 0.0) v = a0 * u0[o] + v;
-  return v + b * res;
+  if (a0 != 0.0) v = fma(a0, u0, v);
+  return fma(b, res, v);
 }
 
-// A thread takes one cell and kVelPerThread consecutive velocities: the point data of the cell
-// (U, lambda, rho sqrt(lambda / pi)) is loaded once for all of them.
-constexpr int kVelPerThread = 8;
+// A thread takes one cell and vpt consecutive velocities: the point data of the cell (U, lambda, rho
+// sqrt(lambda / pi)) is loaded once for all of them.  The next velocity's values (and the velocity
+// after it, whose sign places the neighbour) are loaded before the current one is worked on.  Bound by
+// HBM and by FP64 issue (129 FP64 instructions per cell and velocity at p = 2).  8192 x 256, p = 2: 23.5
+// -> 21.2 us a call (4.7 TB/s); 16384 x 256, p = 4: 139 -> 114 us with its moments.
+// vpt: as many as leave a wavefront per SIMD (65536 threads), 8 at most.  50 steps with 8 / 4 velocities:
+// 400 x 128, p = 4, 8 members (51200 threads at 8) 3113 / 2870 us; 100 x 100, p = 3, 8 members (10400)
+// 1648 / 1304; mol! at 3000 x 256, p = 1, 2 members (192000) 41 / 48 us.
+constexpr int kVelMax = 8;
+constexpr long long kVelThreads = 65536;
 
-template <int NSP>
+template <int NSP, bool WITH_U0>
 __global__ __launch_bounds__(256) void bgk1d_rhs_kernel(Bgk1dGeo g, Bgk1dOps ops, const double *__restrict__ uv,
                                                         const double *__restrict__ tau,
-                                                        const double *__restrict__ prim, Bgk1dStage sa) {
+                                                        const double *__restrict__ prim, Bgk1dStage sa,
+                                                        int vpt) {
   const long long t = blockIdx.x * (long long)blockDim.x + threadIdx.x;
-  const int nvg = (g.nu + kVelPerThread - 1) / kVelPerThread;  // velocity groups
+  const int nvg = (g.nu + vpt - 1) / vpt;  // velocity groups
   const long long per = (long long)g.nx * nvg;
   if (t >= per * g.nmem) return;
   const long long mem = t / per, r = t % per;
-  const int i = (int)(r % g.nx), j0 = (int)(r / g.nx) * kVelPerThread;
+  const int i = (int)(r % g.nx), j0 = (int)(r / g.nx) * vpt;
   const long long kst = (long long)g.nx * g.nu;  // stride of the point index
-  const double *__restrict__ u = sa.u;
-  const double tv = tau[mem];
+  const Bgk1dTau tv(tau[mem]);
   const double *pr = prim + mem * 4 * g.npts + i;
   double U[NSP], lam[NSP], c0[NSP];
 #pragma unroll
@@ -213,20 +230,45 @@ __global__ __launch_bounds__(256) void bgk1d_rhs_kernel(Bgk1dGeo g, Bgk1dOps ops
     lam[k] = pr[2 * g.npts + (long long)g.nx * k];
     c0[k] = pr[3 * g.npts + (long long)g.nx * k];
   }
-  const int jend = min(g.nu, j0 + kVelPerThread);
-  for (int j = j0; j < jend; ++j) {
-    const double vel = uv[j];
-    const bool pos = vel > 0.0;  // heaviside(u_j)
-    const long long base = mem * g.mstride + (long long)i + (long long)g.nx * j;
-    // the upwind neighbour: the left cell (u_j > 0) or the right cell, periodic
-    const int in = pos ? (i == 0 ? g.nx - 1 : i - 1) : (i == g.nx - 1 ? 0 : i + 1);
-    double w[NSP], res[NSP];
-    bgk1d_cell_velocity<NSP>(ops, g.iJ, u, base, base + (long long)(in - i), kst, vel, pos, U, lam, c0, tv, w, res);
+  const int jlast = min(g.nu, j0 + vpt) - 1;
+  // the upwind neighbour: the left cell (u_j > 0) or the right cell, periodic
+  const int left = i == 0 ? g.nx - 1 : i - 1, right = i == g.nx - 1 ? 0 : i + 1;
+  struct Vals {
+    double w[NSP], un[NSP], u0[WITH_U0 ? NSP : 1];
+  } A, B;
+  auto load = [&](int j, double vel, Vals &v) {
+    const long long row = mem * g.mstride + (long long)g.nx * j;
+    const double *const f = sa.u + row, *const n = f + (vel > 0.0 ? left : right);
 #pragma unroll
     for (int k = 0; k < NSP; ++k) {
-      const long long o = base + kst * k;
-      sa.out[o] = sa.residual ? res[k] : bgk1d_combine(sa.a0, sa.a1, sa.b, w[k], sa.u0, o, res[k]);
+      v.w[k] = f[i + kst * k];
+      v.un[k] = n[kst * k];
+      if constexpr (WITH_U0) v.u0[k] = sa.u0[row + i + kst * k];
     }
+  };
+  auto work = [&](int j, double vel, const Vals &v) {
+    double res[NSP];
+    bgk1d_cell_velocity<NSP>(ops, g.iJ, v.w, v.un, vel, vel > 0.0, U, lam, c0, tv, res);
+    double *const o = sa.out + mem * g.mstride + (long long)g.nx * j + i;
+#pragma unroll
+    for (int k = 0; k < NSP; ++k) {
+      const double c = bgk1d_combine(WITH_U0 ? sa.a0 : 0.0, sa.a1, sa.b, v.w[k], WITH_U0 ? v.u0[k] : 0.0, res[k]);
+      o[kst * k] = sa.residual ? res[k] : c;
+    }
+  };
+  double va = uv[j0], vb = uv[min(j0 + 1, jlast)];
+  load(j0, va, A);
+  for (int j = j0;;) {
+    load(min(j + 1, jlast), vb, B);
+    const double vc = uv[min(j + 2, jlast)];
+    work(j, va, A);
+    if (++j > jlast) break;
+    load(min(j + 1, jlast), vc, A);
+    va = vc;
+    const double vd = uv[min(j + 2, jlast)];
+    work(j, vb, B);
+    if (++j > jlast) break;
+    vb = vd;
   }
 }
 
@@ -248,6 +290,14 @@ struct Bgk1dSteps {
 
 __host__ __device__ inline int resident_arrays(int scheme) { return scheme == FR_RK_SSPRK3 ? 3 : 2; }
 
+// Threads of the workgroup: one for every (cell, velocity) and every slice sum of a point as far as
+// 1024 go, so that small members meet at barriers of few wavefronts.  8 cells x 16
+// velocities, p = 1, 50 Euler steps with 128 threads: 94.6 us, with 1024: 97.4.
+inline int resident_threads(const Bgk1dGeo &g) {
+  const long long n = std::max((long long)g.nx * g.nu, (long long)kMomSlices * g.npts);
+  return (int)std::min<long long>(kResidentThreads, (n + 63) / 64 * 64);
+}
+
 // LDS of one member: the state and stage arrays, 3 kMomSlices slice sums and U, lambda, c0 per
 // point, the velocities and weights
 inline size_t resident_lds_bytes(const Bgk1dGeo &g, int scheme) {
@@ -256,23 +306,32 @@ inline size_t resident_lds_bytes(const Bgk1dGeo &g, int scheme) {
          sizeof(double);
 }
 
+// x / n for x, n below 2^16 (everything indexed inside one workgroup's LDS): floor(x m / 2^32) with
+// m = floor(2^32 / n) + 1 overshoots x / n by less than x / 2^32, below 1 / n
+struct Div16 {
+  unsigned n, m;
+  __device__ __forceinline__ explicit Div16(unsigned d) : n(d), m(0xFFFFFFFFu / d + 1u) {}
+  __device__ __forceinline__ int operator()(unsigned x) const { return (int)(n == 1 ? x : __umulhi(x, m)); }
+};
+
 // One stage C = a0 B + a1 A + b L(A) of the member held in LDS; every thread of the workgroup
 // calls it (it ends with a barrier).  C may be B (written at the value each thread read), never A.
 template <int NSP>
-__device__ __forceinline__ void resident_stage(const Bgk1dGeo &g, const Bgk1dOps &ops, const double *uv,
-                                               const double *wv, double tv, const double *A,
+__device__ __forceinline__ void resident_stage(const Bgk1dGeo &g, const Bgk1dOps &ops, const Div16 &by_pts,
+                                               const Div16 &by_nx, const double *uv,
+                                               const double *wv, const Bgk1dTau &tv, const double *A,
                                                const double *B, double *C, double a0, double a1, double b,
                                                double *part, double *pt) {
   const int tid = threadIdx.x;
   const int npts = (int)g.npts;
-  const long long kst = (long long)g.nx * g.nu;
-  for (int idx = tid; idx < kMomSlices * npts; idx += kResidentThreads) {
-    const int sl = idx / npts, p = idx - sl * npts;
-    const double *fb = A + (p % g.nx) + kst * (p / g.nx);
+  const int kst = g.nx * g.nu;
+  for (int idx = tid; idx < kMomSlices * npts; idx += (int)blockDim.x) {
+    const int sl = by_pts(idx), p = idx - sl * npts, k = by_nx(p);
+    const double *fb = A + p + (kst - g.nx) * k;
     double m0 = 0.0, m1 = 0.0, m2 = 0.0;
 #pragma unroll 4
     for (int j = sl; j < g.nu; j += kMomSlices) {
-      const double fv = fb[(long long)g.nx * j];
+      const double fv = fb[g.nx * j];
       const double wj = wv[j], uj = uv[j];
       m0 += wj * fv;
       m1 += wj * uj * fv;
@@ -283,7 +342,7 @@ __device__ __forceinline__ void resident_stage(const Bgk1dGeo &g, const Bgk1dOps
     part[(3 * sl + 2) * npts + p] = m2;
   }
   __syncthreads();
-  for (int p = tid; p < npts; p += kResidentThreads) {
+  for (int p = tid; p < npts; p += (int)blockDim.x) {
     double m0 = part[p], m1 = part[npts + p], m2 = part[2 * npts + p];
 #pragma unroll
     for (int q = 1; q < kMomSlices; ++q) {
@@ -294,8 +353,8 @@ __device__ __forceinline__ void resident_stage(const Bgk1dGeo &g, const Bgk1dOps
     bgk1d_close(m0, m1, m2, g.gamma, pt[p], pt[npts + p], pt[2 * npts + p]);
   }
   __syncthreads();
-  for (int r = tid; r < g.nx * g.nu; r += kResidentThreads) {
-    const int i = r % g.nx, j = r / g.nx;
+  for (int r = tid; r < g.nx * g.nu; r += (int)blockDim.x) {
+    const int j = by_nx(r), i = r - g.nx * j;
     const double vel = uv[j];
     const bool pos = vel > 0.0;
     double U[NSP], lam[NSP], c0[NSP];
@@ -305,15 +364,17 @@ __device__ __forceinline__ void resident_stage(const Bgk1dGeo &g, const Bgk1dOps
       lam[k] = pt[npts + i + g.nx * k];
       c0[k] = pt[2 * npts + i + g.nx * k];
     }
-    const long long base = (long long)i + (long long)g.nx * j;
-    const int in = pos ? (i == 0 ? g.nx - 1 : i - 1) : (i == g.nx - 1 ? 0 : i + 1);
-    double w[NSP], res[NSP];
-    bgk1d_cell_velocity<NSP>(ops, g.iJ, A, base, base + (long long)(in - i), kst, vel, pos, U, lam, c0, tv, w, res);
+    const int in = r + (pos ? (i == 0 ? g.nx - 1 : -1) : (i == g.nx - 1 ? 1 - g.nx : 1));
+    double w[NSP], un[NSP], u0[NSP], res[NSP];
 #pragma unroll
     for (int k = 0; k < NSP; ++k) {
-      const long long o = base + kst * k;
-      C[o] = bgk1d_combine(a0, a1, b, w[k], B, o, res[k]);
+      w[k] = A[r + kst * k];
+      un[k] = A[in + kst * k];
+      u0[k] = a0 != 0.0 ? B[r + kst * k] : 0.0;
     }
+    bgk1d_cell_velocity<NSP>(ops, g.iJ, w, un, vel, pos, U, lam, c0, tv, res);
+#pragma unroll
+    for (int k = 0; k < NSP; ++k) C[r + kst * k] = bgk1d_combine(a0, a1, b, w[k], u0[k], res[k]);
   }
   __syncthreads();
 }
@@ -332,29 +393,30 @@ __global__ __launch_bounds__(kResidentThreads) void bgk1d_resident_kernel(Bgk1dG
   double *pt = part + (long long)3 * kMomSlices * g.npts;
   double *uv = pt + 3 * g.npts, *wv = uv + g.nu;
   double *gs = state + (long long)blockIdx.x * ms;
-  const double tv = tau[blockIdx.x];
-  for (long long v = threadIdx.x; v < ms; v += kResidentThreads) X[v] = gs[v];
-  for (int j = threadIdx.x; j < g.nu; j += kResidentThreads) {
+  const Bgk1dTau tv(tau[blockIdx.x]);
+  const Div16 by_pts((unsigned)g.npts), by_nx((unsigned)g.nx);
+  for (long long v = threadIdx.x; v < ms; v += (int)blockDim.x) X[v] = gs[v];
+  for (int j = threadIdx.x; j < g.nu; j += (int)blockDim.x) {
     uv[j] = uvg[j];
     wv[j] = wvg[j];
   }
   __syncthreads();
   for (int n = 0; n < nsteps; ++n) {
     if (sc.scheme == FR_RK_SSPRK3) {
-      resident_stage<NSP>(g, ops, uv, wv, tv, X, X, Y, sc.a0[0], sc.a1[0], sc.b[0], part, pt);
-      resident_stage<NSP>(g, ops, uv, wv, tv, Y, X, Z, sc.a0[1], sc.a1[1], sc.b[1], part, pt);
-      resident_stage<NSP>(g, ops, uv, wv, tv, Z, X, X, sc.a0[2], sc.a1[2], sc.b[2], part, pt);
+      resident_stage<NSP>(g, ops, by_pts, by_nx, uv, wv, tv, X, X, Y, sc.a0[0], sc.a1[0], sc.b[0], part, pt);
+      resident_stage<NSP>(g, ops, by_pts, by_nx, uv, wv, tv, Y, X, Z, sc.a0[1], sc.a1[1], sc.b[1], part, pt);
+      resident_stage<NSP>(g, ops, by_pts, by_nx, uv, wv, tv, Z, X, X, sc.a0[2], sc.a1[2], sc.b[2], part, pt);
     } else if (sc.scheme == FR_RK_MIDPOINT) {
-      resident_stage<NSP>(g, ops, uv, wv, tv, X, X, Y, sc.a0[0], sc.a1[0], sc.b[0], part, pt);
-      resident_stage<NSP>(g, ops, uv, wv, tv, Y, X, X, sc.a0[1], sc.a1[1], sc.b[1], part, pt);
+      resident_stage<NSP>(g, ops, by_pts, by_nx, uv, wv, tv, X, X, Y, sc.a0[0], sc.a1[0], sc.b[0], part, pt);
+      resident_stage<NSP>(g, ops, by_pts, by_nx, uv, wv, tv, Y, X, X, sc.a0[1], sc.a1[1], sc.b[1], part, pt);
     } else {
-      resident_stage<NSP>(g, ops, uv, wv, tv, X, X, Y, sc.a0[0], sc.a1[0], sc.b[0], part, pt);
+      resident_stage<NSP>(g, ops, by_pts, by_nx, uv, wv, tv, X, X, Y, sc.a0[0], sc.a1[0], sc.b[0], part, pt);
       double *t = X;
       X = Y;
       Y = t;
     }
   }
-  for (long long v = threadIdx.x; v < ms; v += kResidentThreads) gs[v] = X[v];
+  for (long long v = threadIdx.x; v < ms; v += (int)blockDim.x) gs[v] = X[v];
 }
 
 // dst = src over n values (the Euler step's final copy; a kernel, so a captured graph holds no
@@ -415,7 +477,7 @@ struct Bgk1dCtx {
   template <int NSP>
   int launch_resident_n(const Bgk1dSteps &sc, int n, hipStream_t st) const {
     const Bgk1dGeo g = geo();
-    hipLaunchKernelGGL(bgk1d_resident_kernel<NSP>, dim3((unsigned)nmem), dim3(kResidentThreads),
+    hipLaunchKernelGGL(bgk1d_resident_kernel<NSP>, dim3((unsigned)nmem), dim3((unsigned)resident_threads(g)),
                        (unsigned)resident_lds_bytes(g, sc.scheme), st, g, dev_ops(), d_vel, d_vel + nu, d_tau, d_u,
                        sc, n);
     FR_LAUNCHED("bgk1d_resident_kernel");
@@ -466,9 +528,13 @@ struct Bgk1dCtx {
   int launch_rhs(const Bgk1dStage &sa, hipStream_t st) const {
     const Bgk1dOps o = dev_ops();
     const Bgk1dGeo g = geo();
-    const long long n = (long long)nx * ((nu + kVelPerThread - 1) / kVelPerThread) * nmem;
-    hipLaunchKernelGGL(bgk1d_rhs_kernel<NSP>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, g, o, d_vel,
-                       d_tau, d_prim, sa);
+    int vpt = kVelMax;
+    auto threads = [&] { return (long long)nx * ((nu + vpt - 1) / vpt) * nmem; };
+    while (vpt > 1 && threads() < kVelThreads) vpt /= 2;
+    const long long n = threads();
+    const bool u0 = !sa.residual && sa.a0 != 0.0;
+    hipLaunchKernelGGL((u0 ? bgk1d_rhs_kernel<NSP, true> : bgk1d_rhs_kernel<NSP, false>),
+                       dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, g, o, d_vel, d_tau, d_prim, sa, vpt);
     FR_LAUNCHED("bgk1d_rhs_kernel");
     return FR_OK;
   }
