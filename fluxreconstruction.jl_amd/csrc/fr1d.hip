@@ -608,6 +608,7 @@ struct Batch1D {
   int max_nsp = 2;  // largest nsp of the problem set (selects the kernel instance)
   size_t len = 0;
   hipStream_t stream = nullptr;      // the stream every call runs on
+  HostStaging staging;
   hipStream_t own_stream = nullptr;  // the context's own non-blocking stream
   Prob1D *d_probs = nullptr;
   double *d_ops = nullptr;
@@ -698,6 +699,7 @@ struct Batch1D {
 
   void release() {
     if (stream) (void)hipStreamSynchronize(stream);
+    staging.release();
     double *bufs[] = {d_ops, d_u, d_s1, d_s2, d_acc, d_k, d_in, d_out};
     for (double *b : bufs)
       if (b) (void)hipFree(b);
@@ -1082,16 +1084,12 @@ int fr1d_rhs(fr1d_ctx *c, const double *u, double *du, double t) {
 
 int fr1d_set_state(fr1d_ctx *c, const double *u) {
   FR_REQUIRE(c && u, FR_E_INVALID, "fr1d_set_state: null argument");
-  FR_HIP(hipMemcpyAsync(c->d_u, u, c->len * sizeof(double), hipMemcpyHostToDevice, c->stream));
-  FR_HIP(hipStreamSynchronize(c->stream));
-  return FR_OK;
+  return copy_to_device(c->staging, c->d_u, u, c->len, c->stream);
 }
 
 int fr1d_get_state(fr1d_ctx *c, double *u) {
   FR_REQUIRE(c && u, FR_E_INVALID, "fr1d_get_state: null argument");
-  FR_HIP(hipMemcpyAsync(u, c->d_u, c->len * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-  FR_HIP(hipStreamSynchronize(c->stream));
-  return FR_OK;
+  return copy_to_host(c->staging, u, c->d_u, c->len, c->stream);
 }
 
 int fr1d_step(fr1d_ctx *c, int scheme, double dt, int nsteps) {
@@ -1162,16 +1160,12 @@ size_t fr_ens_offset(const fr_ens_ctx *c, int member) {
 
 int fr_ens_set_state(fr_ens_ctx *c, const double *u) {
   FR_REQUIRE(c && u, FR_E_INVALID, "fr_ens_set_state: null argument");
-  FR_HIP(hipMemcpyAsync(c->d_u, u, c->len * sizeof(double), hipMemcpyHostToDevice, c->stream));
-  FR_HIP(hipStreamSynchronize(c->stream));
-  return FR_OK;
+  return copy_to_device(c->staging, c->d_u, u, c->len, c->stream);
 }
 
 int fr_ens_get_state(fr_ens_ctx *c, double *u) {
   FR_REQUIRE(c && u, FR_E_INVALID, "fr_ens_get_state: null argument");
-  FR_HIP(hipMemcpyAsync(u, c->d_u, c->len * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-  FR_HIP(hipStreamSynchronize(c->stream));
-  return FR_OK;
+  return copy_to_host(c->staging, u, c->d_u, c->len, c->stream);
 }
 
 int fr_ens_step(fr_ens_ctx *c, int mode, double dt, int nsteps) {

@@ -572,6 +572,7 @@ struct BgkCtx {
   HostOps ops;
   size_t len = 0;
   hipStream_t stream = nullptr;
+  HostStaging staging;
   double *d_vel = nullptr;  // uv | vv | wu | wv
   BgkVel *d_vt = nullptr;
   double *d_tau = nullptr;
@@ -728,6 +729,7 @@ struct BgkCtx {
 
   void release() {
     if (stream) (void)hipStreamSynchronize(stream);
+    staging.release();
     double *bufs[] = {d_vel, d_tau, d_cons, d_part, d_tab, d_u, d_s1, d_s2, d_in, d_out};
     for (double *b : bufs)
       if (b) (void)hipFree(b);
@@ -836,9 +838,7 @@ int fr_bgk_rhs(fr_bgk_ctx *c, const double *f, double *df) {
 
 int fr_bgk_set_state(fr_bgk_ctx *c, const double *f) {
   FR_REQUIRE(c && f, FR_E_INVALID, "fr_bgk_set_state: null argument");
-  FR_HIP(hipMemcpyAsync(c->d_u, f, c->len * sizeof(double), hipMemcpyHostToDevice, c->stream));
-  FR_HIP(hipStreamSynchronize(c->stream));
-  return FR_OK;
+  return copy_to_device(c->staging, c->d_u, f, c->len, c->stream);
 }
 
 int fr_bgk_set_state_dev(fr_bgk_ctx *c, const double *d_f) {
@@ -850,9 +850,7 @@ int fr_bgk_set_state_dev(fr_bgk_ctx *c, const double *d_f) {
 
 int fr_bgk_get_state(fr_bgk_ctx *c, double *f) {
   FR_REQUIRE(c && f, FR_E_INVALID, "fr_bgk_get_state: null argument");
-  FR_HIP(hipMemcpyAsync(f, c->d_u, c->len * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-  FR_HIP(hipStreamSynchronize(c->stream));
-  return FR_OK;
+  return copy_to_host(c->staging, f, c->d_u, c->len, c->stream);
 }
 
 // nsteps Shu-Osher SSP-RK3 steps of all members; each stage = closure + transport/relaxation

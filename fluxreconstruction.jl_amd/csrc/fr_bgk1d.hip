@@ -433,6 +433,7 @@ struct Bgk1dCtx {
   HostOps ops;
   size_t len = 0;
   hipStream_t stream = nullptr;
+  HostStaging staging;
   hipEvent_t ev = nullptr;  // orders work on a caller stream against the context's stream
   double *d_vel = nullptr;  // u | w
   double *d_tau = nullptr, *d_prim = nullptr;
@@ -630,6 +631,7 @@ struct Bgk1dCtx {
 
   void release() {
     if (stream) (void)hipStreamSynchronize(stream);
+    staging.release();
     if (gexec) (void)hipGraphExecDestroy(gexec);
     double *bufs[] = {d_vel, d_tau, d_prim, d_u, d_s1, d_s2, d_in, d_out};
     for (double *b : bufs)
@@ -733,16 +735,12 @@ int fr_bgk1d_rhs_dev(fr_bgk1d_ctx *c, const double *d_f, double *d_df, void *str
 
 int fr_bgk1d_set_state(fr_bgk1d_ctx *c, const double *f) {
   FR_REQUIRE(c && f, FR_E_INVALID, "fr_bgk1d_set_state: null argument");
-  FR_HIP(hipMemcpyAsync(c->d_u, f, c->len * sizeof(double), hipMemcpyHostToDevice, c->stream));
-  FR_HIP(hipStreamSynchronize(c->stream));
-  return FR_OK;
+  return copy_to_device(c->staging, c->d_u, f, c->len, c->stream);
 }
 
 int fr_bgk1d_get_state(fr_bgk1d_ctx *c, double *f) {
   FR_REQUIRE(c && f, FR_E_INVALID, "fr_bgk1d_get_state: null argument");
-  FR_HIP(hipMemcpyAsync(f, c->d_u, c->len * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-  FR_HIP(hipStreamSynchronize(c->stream));
-  return FR_OK;
+  return copy_to_host(c->staging, f, c->d_u, c->len, c->stream);
 }
 
 int fr_bgk1d_set_path(fr_bgk1d_ctx *c, int path) {

@@ -31,6 +31,23 @@ int hip_fail(hipError_t e, const char *what, const char *file, int line);
 // A kernel launch is checked with hipGetLastError right after it.
 #define FR_LAUNCHED(name) FR_HIP(hipGetLastError())
 
+// ------------------------------------------------------------------ host arrays
+// Pinned chunks that a context's large copies to and from pageable host arrays go through
+// (fr_host_copy.cpp): allocated by the first such copy, released with the context.
+struct HostStaging {
+  static constexpr int kWorkers = 4;
+  static constexpr size_t kChunk = 2u << 20;
+  static constexpr size_t kFrom = 24u << 20;  // bytes of a copy from which on it pays, its first one too
+  char *buf = nullptr;
+  hipEvent_t ev[2 * kWorkers] = {};
+  int device = 0;
+  int ensure(hipStream_t st);
+  void release();
+};
+// n doubles; both are done when they return
+int copy_to_device(HostStaging &s, double *dev, const double *host, size_t n, hipStream_t st);
+int copy_to_host(HostStaging &s, double *host, const double *dev, size_t n, hipStream_t st);
+
 // ------------------------------------------------------------------ host operator builders
 // (fr_host_ops.cpp; the same routines back the fr_* operator entry points of fr.h)
 void gauss_legendre(int n, double *x, double *w);

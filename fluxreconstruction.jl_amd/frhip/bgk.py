@@ -132,7 +132,7 @@ class BGK2D:
         check(_lib.lib().fr_bgk_set_state(self.h, dptr(flat)))
 
     def get_state(self):
-        f = np.zeros(self.len)
+        f = np.empty(self.len)
         check(_lib.lib().fr_bgk_get_state(self.h, dptr(f)))
         return f
 
@@ -262,7 +262,7 @@ class BGK1D:
         check(_lib.lib().fr_bgk1d_set_state(self.h, dptr(self._flat(f))))
 
     def get_state(self):
-        f = np.zeros(self.len)
+        f = np.empty(self.len)
         check(_lib.lib().fr_bgk1d_get_state(self.h, dptr(f)))
         return f.reshape(self.shape + ((self.nmem,) if self.nmem > 1 else ()), order="F")
 

@@ -242,7 +242,7 @@ class Ensemble1D:
         check(_lib.lib().fr_ens_set_state(self.h, dptr(np.ascontiguousarray(flat, dtype=np.float64))))
 
     def get_state(self):
-        out = np.zeros(self.len)
+        out = np.empty(self.len)
         check(_lib.lib().fr_ens_get_state(self.h, dptr(out)))
         return out
 
