@@ -37,3 +37,21 @@ def test_large_state_step_parity(nx, ny, deg, nu, nv, nmem):
     g.set_state(f0)
     g.step(dt, 2)
     assert np.array_equal(g.get_state(), two)
+
+
+@pytest.mark.parametrize("nx,ny,deg,nv", [(67, 61, 1, 23), (37, 29, 2, 31), (20, 33, 2, 16)])
+def test_steps_of_one_call_and_of_several(nx, ny, deg, nv):
+    # odd and even step counts end in different buffers; partial tiles read u^n for cells stored elsewhere
+    u, wu = bgk.velocity_grid(nv)
+    f0 = bgk.maxwellian_state(nx, ny, deg, u, u, amp=0.1)
+    dt = 0.1 / (deg + 1) / max(nx, ny) / np.abs(u).max()
+    g = bgk.BGK2D(nx, ny, deg, u, wu, u, wu, [1e-2])
+    g.set_state(f0)
+    outs = []
+    for _ in range(3):
+        g.step(dt, 1)
+        outs.append(g.get_state())
+    for n in (1, 2, 3):
+        g.set_state(f0)
+        g.step(dt, n)
+        assert np.array_equal(g.get_state(), outs[n - 1])
