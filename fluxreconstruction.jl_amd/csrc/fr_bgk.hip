@@ -18,6 +18,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <exception>
 #include <new>
 #include <type_traits>
 #include <utility>
@@ -785,8 +786,14 @@ int fr_bgk_create(fr_bgk_ctx **out, const fr_bgk_desc *d) {
   vel.insert(vel.end(), d->v, d->v + d->nv);
   vel.insert(vel.end(), d->wu, d->wu + d->nu);
   vel.insert(vel.end(), d->wv, d->wv + d->nv);
-  std::vector<BgkVel> vt;
-  for (int b = 0; b < d->nv; ++b)
+  std::vector<BgkVel> vt;  // of the stage kernel alone
+  try {
+    if (c->large()) vt.reserve((size_t)d->nu * d->nv);
+  } catch (const std::exception &) {
+    delete c;
+    return fail(FR_E_NOMEM, "fr_bgk_create: out of host memory");
+  }
+  for (int b = 0; c->large() && b < d->nv; ++b)
     for (int a = 0; a < d->nu; ++a) {
       const double u = d->u[a], v = d->v[b], w = d->wu[a] * d->wv[b];
       vt.push_back({u * (2.0 / d->dx), v * (2.0 / d->dy), {w, w * u, w * v, w * 0.5 * (u * u + v * v)},
@@ -795,8 +802,9 @@ int fr_bgk_create(fr_bgk_ctx **out, const fr_bgk_desc *d) {
   hipError_t e = hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking);
   if (e == hipSuccess) e = hipMalloc(&c->d_vel, vel.size() * sizeof(double));
   if (e == hipSuccess) e = hipMemcpy(c->d_vel, vel.data(), vel.size() * sizeof(double), hipMemcpyHostToDevice);
-  if (e == hipSuccess) e = hipMalloc(&c->d_vt, vt.size() * sizeof(BgkVel));
-  if (e == hipSuccess) e = hipMemcpy(c->d_vt, vt.data(), vt.size() * sizeof(BgkVel), hipMemcpyHostToDevice);
+  if (e == hipSuccess && c->large()) e = hipMalloc(&c->d_vt, vt.size() * sizeof(BgkVel));
+  if (e == hipSuccess && c->large())
+    e = hipMemcpy(c->d_vt, vt.data(), vt.size() * sizeof(BgkVel), hipMemcpyHostToDevice);
   if (e == hipSuccess) e = hipMalloc(&c->d_tau, d->nmem * sizeof(double));
   if (e == hipSuccess) e = hipMemcpy(c->d_tau, d->tau, d->nmem * sizeof(double), hipMemcpyHostToDevice);
   if (e == hipSuccess) e = hipMalloc(&c->d_cons, (size_t)g.npts * 4 * d->nmem * sizeof(double));

@@ -9,7 +9,7 @@
 // and 1.87 ms at 53 MB, of 4 MB 1.74 and 1.34.
 #include <algorithm>
 #include <cstring>
-#include <system_error>
+#include <exception>
 #include <thread>
 
 #include "fr_common.h"
@@ -81,7 +81,7 @@ static int staged(HostStaging &s, char *dev, char *host, size_t bytes, bool up, 
   for (int w = 1; w < HostStaging::kWorkers; ++w) {
     try {
       th[w] = std::thread([&, w] { err[w] = work(s, w, dev, host, bytes, up, st); });
-    } catch (const std::system_error &) {  // no thread to be had: this one does its part below
+    } catch (const std::exception &) {  // no thread to be had: this one does its part below
     }
   }
   err[0] = work(s, 0, dev, host, bytes, up, st);
