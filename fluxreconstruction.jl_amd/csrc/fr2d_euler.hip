@@ -13,9 +13,11 @@
 // same thread then holds column `line` for the y direction.  All face data of a line stays inside
 // its wavefront (the neighbours of an element are lanes -1/+1 along x and -TX/+TX along y; the
 // traces of the halo elements around the tile come from halo tasks on lanes of the same
-// wavefront), so faces need only wavefront-level LDS ordering: x faces in a per-line slice,
+// wavefront), so faces need no workgroup barrier: x faces go from lane to lane by DPP (through an
+// LDS slice per line they took 8 KB more at nsp = 4 and, per stage, 251 x 133 cells of p = 3, HLL 16.3
+// against 15.3 us, 502 x 133 of p = 1, Rusanov 9.1 against 8.7, 167 x 133 of p = 5 26.9 against 24.9),
 // y faces in the line's own column block of the transpose buffer once that column is read.
-// At nsp = 4 a workgroup takes 40 KB of LDS and 128 VGPRs (Rusanov), so four workgroups share
+// At nsp = 4 a workgroup takes 33 KB of LDS and 128 VGPRs, so four workgroups share
 // a CU and a 256 x 256 grid (1024 tiles) is resident at once.  Every element is read from HBM
 // once; halo re-reads hit L2 (tiles are ordered XCD-aware).
 #include <algorithm>
@@ -93,21 +95,34 @@ __device__ __forceinline__ void strip_tile(int t, int ntx, int nty, int sw, int 
 // The point-metric instances keep the default as well: their metric values stay live from the
 // x sweep to the corrections.
 template <int NSP, int FLUX, int EPI, int GEO>
-constexpr int fr2d_min_blocks() {
+constexpr int fr2d_min_waves() {
   return (NSP == 4 && FLUX != FR_FLUX_ROE && EPI != EPI_ACC && GEO != GEO_POINT) ? 4 : 1;
 }
 
+// x of the lane D places to the left (D = 1) or right (-1) in the row of 16 lanes; 0 where there is none.
+// All lanes of the wavefront must be active.
+template <int D>
+__device__ __forceinline__ double row_shift(double x) {
+  static_assert(D == 1 || D == -1, "one place");
+  constexpr int ctrl = D == 1 ? 0x111 : 0x101;  // row_shr:1, row_shl:1
+  const fr_u2 v = __builtin_bit_cast(fr_u2, x);
+  fr_u2 r;
+  r.x = (unsigned)__builtin_amdgcn_update_dpp(0, (int)v.x, ctrl, 0xf, 0xf, true);
+  r.y = (unsigned)__builtin_amdgcn_update_dpp(0, (int)v.y, ctrl, 0xf, 0xf, true);
+  return __builtin_bit_cast(double, r);
+}
+
 template <int NSP, int FLUX, int EPI, int ADDR, int GEO>
-__global__ __launch_bounds__(NSP * 64, (fr2d_min_blocks<NSP, FLUX, EPI, GEO>())) void fr2d_kernel(const Geo2D geo,
+__global__ __launch_bounds__(NSP * 64, (fr2d_min_waves<NSP, FLUX, EPI, GEO>())) void fr2d_kernel(const Geo2D geo,
                                                                                               const StageArgs sa) {
   // operators are compile-time constants (Gauss-Legendre points, Radau correction), so they
   // occupy no scalar registers for the length of the kernel
   constexpr StdOps2D<NSP> ops{};
   // LDS: the tile transpose sU (rows -> columns, then the y contributions columns -> rows) and
-  // the x faces of every line (sX).  The y faces of a line live in that line's own column block
+  // the tile's right x-faces (sX).  The y faces of a line live in that line's own column block
   // of sU between the column read and the write-back of the y contributions.
   __shared__ double sU[NSP * NSP * 4 * TE];
-  __shared__ double sX[4 * NSP * TY * TX];
+  __shared__ double sX[4 * NSP * TY];
 
   const int tid = threadIdx.x;
   // the line index is uniform over a wavefront, so every plane offset below is a scalar
@@ -130,9 +145,8 @@ __global__ __launch_bounds__(NSP * 64, (fr2d_min_blocks<NSP, FLUX, EPI, GEO>()))
   const double ua = EPI == EPI_STAGE ? sa.a1 / sxs : 0.0;
 
   auto SU = [&](int k, int l, int m) -> double & { return sU[((k * NSP + l) * 4 + m) * TE + lane]; };
-  // x-face slot s of row y holds face s + 1 (between elements s and s + 1 of the row): first the
-  // right trace of element s, then the face flux
-  auto SX = [&](int m, int y, int s) -> double & { return sX[((m * NSP + line) * TY + y) * TX + s]; };
+  // right x-face of the tile in row y: the last element's right trace, then the face flux
+  auto SX = [&](int m, int y) -> double & { return sX[(m * NSP + line) * TY + y]; };
   double *const sYl = sU + line * (NSP * 4 * TE);
   static_assert(4 * (TY + 1) * TX <= 4 * 2 * TE, "the y faces of a line fit in its column block");
   // y-face slot fy of column x: face between elements fy - 1 and fy of the column
@@ -307,20 +321,38 @@ __global__ __launch_bounds__(NSP * 64, (fr2d_min_blocks<NSP, FLUX, EPI, GEO>()))
     }
   }
 
-  // x sweep of the row: traces (right traces into the line's x-face slots), LDS transpose copy,
-  // x flux and its derivative with the flux-trace parts of the corrections folded in (dc); the
-  // stage seeds it with (a1 / sxs)*u, so that sxs times it carries a1*u and the row dies here
-  double uLx[4], dxr[NSP][4];
+  // x faces of the row: the left neighbour's right trace and the right neighbour's left-face flux
+  // come over DPP from the lanes beside (a row of the tile is a row of 16 lanes; every lane takes
+  // part); the row's first lane holds the left halo's trace
+  double cl[4], cr[4];
+  {
+    double wl[4], uLx[4];
 #pragma unroll
-  for (int m = 0; m < 4; ++m) {
-    double a = 0.0, b = 0.0;
+    for (int m = 0; m < 4; ++m) {
+      double a = 0.0, b = 0.0;
 #pragma unroll
-    for (int k = 0; k < NSP; ++k) {
-      a += ur[k][m] * ops.ll[k];
-      b += ur[k][m] * ops.lr[k];
+      for (int k = 0; k < NSP; ++k) {
+        a += ur[k][m] * ops.ll[k];
+        b += ur[k][m] * ops.lr[k];
+      }
+      uLx[m] = a;
+      if (ex == ncx - 1) SX(m, ey) = b;
+      const double l = row_shift<1>(b);
+      wl[m] = ex > 0 ? l : htr[m];
     }
-    uLx[m] = a;
-    if (act) SX(m, ey, ex) = b;
+    if constexpr (AFF) {
+      riemann_n4<FLUX>(wl, uLx, geo.n1c, geo.n1s, g, gm1, cl);
+#pragma unroll
+      for (int m = 0; m < 4; ++m) cl[m] *= geo.q1;
+    } else {
+      riemann_x4<FLUX>(wl, uLx, g, gm1, cl);
+    }
+    // the tile's last element of a row takes its right face after the halo pass
+#pragma unroll
+    for (int m = 0; m < 4; ++m) {
+      const double r = row_shift<-1>(cl[m]);
+      cr[m] = ex < ncx - 1 ? r : 0.0;
+    }
   }
   if (act) {
 #pragma unroll
@@ -328,8 +360,11 @@ __global__ __launch_bounds__(NSP * 64, (fr2d_min_blocks<NSP, FLUX, EPI, GEO>()))
 #pragma unroll
       for (int m = 0; m < 4; ++m) SU(k, line, m) = ur[k][m];
   }
-  // point metrics: r_x of the row's points, which also scales their x-face terms
-  double jx[NSP];
+  // x flux, its derivative with the flux-trace parts of the corrections folded in (dc) and the face
+  // corrections: the x part of the result, -iJ11*x (residual, RK4 form) or a1*u - b*iJ11*x (stage; the
+  // a1 part as (a1 / sxs)*u inside, so that the row dies here).  Point metrics: r_x of the row's
+  // points, which also scales their x-face terms
+  double jx[NSP], res[NSP][4];
   {
     double f1[NSP][4];
 #pragma unroll
@@ -359,7 +394,12 @@ __global__ __launch_bounds__(NSP * 64, (fr2d_min_blocks<NSP, FLUX, EPI, GEO>()))
         double d = 0.0;
 #pragma unroll
         for (int q = 0; q < NSP; ++q) d += f1[q][m] * ops.dc[k + NSP * q];
-        dxr[k][m] = EPI == EPI_STAGE ? ua * ur[k][m] + d : d;
+        if constexpr (EPI == EPI_STAGE) d = ua * ur[k][m] + d;
+        if constexpr (PT)
+          res[k][m] = sxs * (d + jx[k] * (cl[m] * ops.dhl[k] + cr[m] * ops.dhr[k]));
+        else
+          res[k][m] = sxs * (d + cl[m] * ops.dhl[k] + cr[m] * ops.dhr[k]);
+        fr_pin(res[k][m]);
       }
   }
   // RK4 form: stage operand a1*u of the own row
@@ -369,47 +409,6 @@ __global__ __launch_bounds__(NSP * 64, (fr2d_min_blocks<NSP, FLUX, EPI, GEO>()))
     for (int m = 0; m < 4; ++m)
 #pragma unroll
       for (int k = 0; k < NSP; ++k) pre[k][m] = sa.a1 * ur[k][m];
-  }
-  wave_lds_sync();  // the right traces of this line are visible to its lanes
-
-  // own left x-face: the left neighbour's right trace (the left halo on the row's first lane);
-  // the flux replaces the trace in its slot, where the left neighbour reads it
-  double cl[4] = {0.0, 0.0, 0.0, 0.0};
-  if (act) {
-    double wl[4];
-    const int s = ex > 0 ? ex - 1 : 0;
-#pragma unroll
-    for (int m = 0; m < 4; ++m) wl[m] = ex > 0 ? SX(m, ey, s) : htr[m];
-    if constexpr (AFF) {
-      riemann_n4<FLUX>(wl, uLx, geo.n1c, geo.n1s, g, gm1, cl);
-#pragma unroll
-      for (int m = 0; m < 4; ++m) cl[m] *= geo.q1;
-    } else {
-      riemann_x4<FLUX>(wl, uLx, g, gm1, cl);
-    }
-    if (ex > 0) {
-#pragma unroll
-      for (int m = 0; m < 4; ++m) SX(m, ey, s) = cl[m];
-    }
-  }
-  wave_lds_sync();
-  // x corrections (the tile's last element of a row takes its right face after the halo pass);
-  // the x part of the result: -iJ11*x (residual, RK4 form) or a1*u - b*iJ11*x (stage)
-  double res[NSP][4];
-  {
-    const bool has_r = ex < ncx - 1;
-#pragma unroll
-    for (int m = 0; m < 4; ++m) {
-      const double cr = has_r ? SX(m, ey, ex) : 0.0;
-#pragma unroll
-      for (int k = 0; k < NSP; ++k) {
-        if constexpr (PT)
-          res[k][m] = sxs * (dxr[k][m] + jx[k] * (cl[m] * ops.dhl[k] + cr * ops.dhr[k]));
-        else
-          res[k][m] = sxs * (dxr[k][m] + cl[m] * ops.dhl[k] + cr * ops.dhr[k]);
-        fr_pin(res[k][m]);
-      }
-    }
   }
   __syncthreads();  // B1: the rows of every line are in sU
 
@@ -506,7 +505,7 @@ __global__ __launch_bounds__(NSP * 64, (fr2d_min_blocks<NSP, FLUX, EPI, GEO>()))
     const bool xf = hkind == 3;
     double *slot[4];
 #pragma unroll
-    for (int m = 0; m < 4; ++m) slot[m] = xf ? &SX(m, hpos, ncx - 1) : &SY(m, ncy, hpos);
+    for (int m = 0; m < 4; ++m) slot[m] = xf ? &SX(m, hpos) : &SY(m, ncy, hpos);
     double w[4], fw[4];
 #pragma unroll
     for (int m = 0; m < 4; ++m) w[m] = *slot[m];
@@ -550,7 +549,7 @@ __global__ __launch_bounds__(NSP * 64, (fr2d_min_blocks<NSP, FLUX, EPI, GEO>()))
     if (ex == ncx - 1) {  // right face of the row's last element, solved by the right task
 #pragma unroll
       for (int m = 0; m < 4; ++m) {
-        const double cr = sxs * SX(m, ey, ex);
+        const double cr = sxs * SX(m, ey);
 #pragma unroll
         for (int k = 0; k < NSP; ++k) res[k][m] += (PT ? cr * jx[k] : cr) * ops.dhr[k];
       }
