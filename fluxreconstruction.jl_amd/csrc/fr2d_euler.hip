@@ -4,7 +4,8 @@
 // ll/lr interpolation to flux points, interface Riemann flux, dl derivative, dhl/dhr correction)
 // and, in stage mode, the explicit RK update out = a0*u0 + a1*u + b*L(u) in its epilogue.
 //
-// Mapping: a workgroup owns a tile of TX x TY = 16 x 4 elements and has NSP wavefronts.  Lane =
+// Mapping: a tile of TX x TY = 16 x 4 elements is worked on by NSP wavefronts, a workgroup owns one
+// tile (two at nsp = 5, kTilesPerWg).  Lane =
 // element of the tile (16 consecutive elements along x per row, so every global access of a
 // wavefront covers four 128-byte segments of the element-fastest SoA layout), wave index = one
 // line of solution points.  Each thread first holds row `line` of its element and finishes the
@@ -112,21 +113,33 @@ __device__ __forceinline__ double row_shift(double x) {
   return __builtin_bit_cast(double, r);
 }
 
+// Tiles of a workgroup.  The waves of a workgroup of five go 2, 1, 1, 1 to the SIMDs, which at the 145 to
+// 168 VGPRs of nsp = 5 hold three each, and one such workgroup was resident per CU (5.06 waves by the
+// counters) where LDS and registers allow two; with two tiles in a workgroup of ten (3, 3, 2, 2) ten are.
+// Per SSP-RK3 stage: 201 x 133, HLL 24.9 -> 19.1 us, 560 x 500, Rusanov 201 -> 176 us, Roe 223 -> 187, polar
+// cells 268 -> 231.  At nsp = 6 two tiles have to fit 168 VGPRs and spill: 466 x 500 239 -> 249 us, polar
+// cells 289 -> 387.
+template <int NSP>
+constexpr int kTilesPerWg = NSP == 5 ? 2 : 1;
+
 template <int NSP, int FLUX, int EPI, int ADDR, int GEO>
-__global__ __launch_bounds__(NSP * 64, (fr2d_min_waves<NSP, FLUX, EPI, GEO>())) void fr2d_kernel(const Geo2D geo,
-                                                                                              const StageArgs sa) {
+__global__ __launch_bounds__(kTilesPerWg<NSP> * NSP * 64, (fr2d_min_waves<NSP, FLUX, EPI, GEO>())) void fr2d_kernel(
+    const Geo2D geo, const StageArgs sa) {
   // operators are compile-time constants (Gauss-Legendre points, Radau correction), so they
   // occupy no scalar registers for the length of the kernel
   constexpr StdOps2D<NSP> ops{};
   // LDS: the tile transpose sU (rows -> columns, then the y contributions columns -> rows) and
   // the tile's right x-faces (sX).  The y faces of a line live in that line's own column block
   // of sU between the column read and the write-back of the y contributions.
-  __shared__ double sU[NSP * NSP * 4 * TE];
-  __shared__ double sX[4 * NSP * TY];
+  constexpr int NT = kTilesPerWg<NSP>, THREADS = NT * NSP * 64;
+  __shared__ double sUt[NT][NSP * NSP * 4 * TE];
+  __shared__ double sXt[NT][4 * NSP * TY];
 
   const int tid = threadIdx.x;
-  // the line index is uniform over a wavefront, so every plane offset below is a scalar
-  const int line = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // the tile and line indices are uniform over a wavefront, so every plane offset below is a scalar
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int half = NT > 1 ? wave / NSP : 0, line = wave - NSP * half;
+  double *const sU = sUt[half], *const sX = sXt[half];
   const int lane = tid & 63;
   const int ex = lane % TX, ey = lane / TX;
   const unsigned nxg = geo.pitch;
@@ -196,17 +209,19 @@ __global__ __launch_bounds__(NSP * 64, (fr2d_min_waves<NSP, FLUX, EPI, GEO>())) 
     for (int q = 0; q < n; ++q) __builtin_amdgcn_s_sleep(8);
   }
   int bx, by;
-  strip_tile(xcd_tile(blockIdx.x, gridDim.x), geo.ntx, geo.nty, geo.strip, bx, by);
+  const int t0 = NT * xcd_tile(blockIdx.x, gridDim.x) + half, tiles = geo.ntx * geo.nty;
+  const bool have = NT == 1 || t0 < tiles;  // the last workgroup may lack its second tile
+  strip_tile(have ? t0 : tiles - 1, geo.ntx, geo.nty, geo.strip, bx, by);
   const int i0 = 1 + bx * TX, j0 = 1 + by * TY;
   const int ncx = min(TX, geo.nx - i0 + 1), ncy = min(TY, geo.ny - j0 + 1);
-  const bool act = ex < ncx && ey < ncy;
+  const bool act = have && ex < ncx && ey < ncy;
   // byte offset of the own element inside a plane (pitch (ny+2) < 2^29 on the host)
   const unsigned ebo = 8u * ((unsigned)(i0 + ex) + nxg * (unsigned)(j0 + ey));
 
   if constexpr (EPI == EPI_RESIDUAL) {
     if (blockIdx.x == 0) {  // du vanishes on the four ghost corners (example/shock-vortex.jl:27)
       constexpr int per = NSP * NSP * 4;
-      for (int v = tid; v < 4 * per; v += NSP * 64) {
+      for (int v = tid; v < 4 * per; v += THREADS) {
         const int c = v / per, o = v % per;
         const long long ci = (c & 1) ? geo.nx + 1 : 0, cj = (c & 2) ? geo.ny + 1 : 0;
         sa.out[ci + (long long)nxg * cj + ldp * o] = 0.0;
@@ -215,7 +230,7 @@ __global__ __launch_bounds__(NSP * 64, (fr2d_min_waves<NSP, FLUX, EPI, GEO>())) 
   } else {
     if (blockIdx.x == 0 && sa.gc0) {  // the four ghost corners, which no halo task loads
       constexpr int per = NSP * NSP * 4;
-      for (int v = tid; v < 4 * per; v += NSP * 64) {
+      for (int v = tid; v < 4 * per; v += THREADS) {
         const int c = v / per, o = v % per;
         const long long ci = (c & 1) ? geo.nx + 1 : 0, cj = (c & 2) ? geo.ny + 1 : 0;
         const long long at = ci + (long long)nxg * cj + ldp * o;
@@ -261,7 +276,7 @@ __global__ __launch_bounds__(NSP * 64, (fr2d_min_waves<NSP, FLUX, EPI, GEO>())) 
       hpos = t - TX;
     }
   }
-  if (hkind >= 0 && hpos >= (hkind <= 1 ? ncx : ncy)) hkind = -1;
+  if (!have || hpos >= (hkind <= 1 ? ncx : ncy)) hkind = -1;
   double htr[4] = {0.0, 0.0, 0.0, 0.0};
   if (hkind >= 0) {
     int hi, hj;
@@ -682,23 +697,24 @@ static int launch_nsp(const Fr2dCtx &c, const StageArgs &sa, hipStream_t st) {
   // reference-layout one when the padded pitch is nx + 2)
   geo.mj = geo.pitch == c.nx + 2 ? c.d_mj_ref : c.d_mj_pad;
   if (c.geom == 2 && !geo.mj) return fail(FR_E_INVALID, "fr2d: point metrics missing on the device");
-  const unsigned nb = (unsigned)(geo.ntx * geo.nty);  // one tile per workgroup
+  constexpr int NT = kTilesPerWg<NSP>;
+  const unsigned nb = (unsigned)((geo.ntx * geo.nty + NT - 1) / NT);
   const bool stag = !caller && c.stagger > 0 && fr2d_single_round(c);
   geo.stag_cu = stag ? c.num_cu : 0;
   geo.stag = stag ? c.stagger : 0;
   const bool buf = (caller ? c.len : c.lenp) * sizeof(double) < (size_t)0xFFFFFFFFu;
   if (c.geom == 0 && buf)
-    hipLaunchKernelGGL((fr2d_kernel<NSP, FLUX, EPI, ADDR_BUFFER, GEO_RECT>), dim3(nb), dim3(NSP * 64), 0, st, geo, sa);
+    hipLaunchKernelGGL((fr2d_kernel<NSP, FLUX, EPI, ADDR_BUFFER, GEO_RECT>), dim3(nb), dim3(NT * NSP * 64), 0, st, geo, sa);
   else if (c.geom == 0)
-    hipLaunchKernelGGL((fr2d_kernel<NSP, FLUX, EPI, ADDR_FLAT, GEO_RECT>), dim3(nb), dim3(NSP * 64), 0, st, geo, sa);
+    hipLaunchKernelGGL((fr2d_kernel<NSP, FLUX, EPI, ADDR_FLAT, GEO_RECT>), dim3(nb), dim3(NT * NSP * 64), 0, st, geo, sa);
   else if (c.geom == 1 && buf)
-    hipLaunchKernelGGL((fr2d_kernel<NSP, FLUX, EPI, ADDR_BUFFER, GEO_AFFINE>), dim3(nb), dim3(NSP * 64), 0, st, geo, sa);
+    hipLaunchKernelGGL((fr2d_kernel<NSP, FLUX, EPI, ADDR_BUFFER, GEO_AFFINE>), dim3(nb), dim3(NT * NSP * 64), 0, st, geo, sa);
   else if (c.geom == 1)
-    hipLaunchKernelGGL((fr2d_kernel<NSP, FLUX, EPI, ADDR_FLAT, GEO_AFFINE>), dim3(nb), dim3(NSP * 64), 0, st, geo, sa);
+    hipLaunchKernelGGL((fr2d_kernel<NSP, FLUX, EPI, ADDR_FLAT, GEO_AFFINE>), dim3(nb), dim3(NT * NSP * 64), 0, st, geo, sa);
   else if (buf)
-    hipLaunchKernelGGL((fr2d_kernel<NSP, FLUX, EPI, ADDR_BUFFER, GEO_POINT>), dim3(nb), dim3(NSP * 64), 0, st, geo, sa);
+    hipLaunchKernelGGL((fr2d_kernel<NSP, FLUX, EPI, ADDR_BUFFER, GEO_POINT>), dim3(nb), dim3(NT * NSP * 64), 0, st, geo, sa);
   else
-    hipLaunchKernelGGL((fr2d_kernel<NSP, FLUX, EPI, ADDR_FLAT, GEO_POINT>), dim3(nb), dim3(NSP * 64), 0, st, geo, sa);
+    hipLaunchKernelGGL((fr2d_kernel<NSP, FLUX, EPI, ADDR_FLAT, GEO_POINT>), dim3(nb), dim3(NT * NSP * 64), 0, st, geo, sa);
   FR_LAUNCHED("fr2d_kernel");
   return FR_OK;
 }
