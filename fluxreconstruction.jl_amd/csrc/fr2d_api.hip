@@ -209,7 +209,11 @@ static int prepare_step(Fr2dCtx &c, int scheme, hipStream_t st) {
   // the stage buffers take the state's ghost layer inside the first stage of every step
   (void)st;
   int rc = ensure_stage_buffers(c, scheme == FR_RK_RK4, scheme == FR_RK_TSIT5);
-  if (!rc && c.stagger < 0) c.stagger = fr2d_default_stagger(c);
+  // No staggered start unless asked for: 20 SSP-RK3 steps in us with 0 / 2 / 3 / 5 / 7 units: Rusanov
+  // 256 x 256 periodic 1081 / 1082 / 1101 / 1097 / 1151, with ghosts 1156 / 1158 / 1175 / 1170 / 1223, 250 x 199
+  // 1075 / 1066 / 1063 / 1054 / 1131, parallelograms 300 x 200 with ghosts 1107 / 1100 / 1097 / 1078 / 1187;
+  // HLL 256 x 256 with ghosts 1207 / 1200 / 1233 / 1231 / 1268
+  if (!rc && c.stagger < 0) c.stagger = 0;
   return rc;
 }
 

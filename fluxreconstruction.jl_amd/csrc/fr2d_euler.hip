@@ -218,25 +218,25 @@ __global__ __launch_bounds__(kTilesPerWg<NSP> * NSP * 64, (fr2d_min_waves<NSP, F
   // byte offset of the own element inside a plane (pitch (ny+2) < 2^29 on the host)
   const unsigned ebo = 8u * ((unsigned)(i0 + ex) + nxg * (unsigned)(j0 + ey));
 
-  if constexpr (EPI == EPI_RESIDUAL) {
-    if (blockIdx.x == 0) {  // du vanishes on the four ghost corners (example/shock-vortex.jl:27)
-      constexpr int per = NSP * NSP * 4;
-      for (int v = tid; v < 4 * per; v += THREADS) {
-        const int c = v / per, o = v % per;
-        const long long ci = (c & 1) ? geo.nx + 1 : 0, cj = (c & 2) ? geo.ny + 1 : 0;
-        sa.out[ci + (long long)nxg * cj + ldp * o] = 0.0;
-      }
-    }
-  } else {
-    if (blockIdx.x == 0 && sa.gc0) {  // the four ghost corners, which no halo task loads
-      constexpr int per = NSP * NSP * 4;
-      for (int v = tid; v < 4 * per; v += THREADS) {
-        const int c = v / per, o = v % per;
-        const long long ci = (c & 1) ? geo.nx + 1 : 0, cj = (c & 2) ? geo.ny + 1 : 0;
-        const long long at = ci + (long long)nxg * cj + ldp * o;
-        sa.gc0[at] = u[at];
-        sa.gc1[at] = u[at];
-      }
+  // the four ghost corners, which no halo task loads: du vanishes there (example/shock-vortex.jl:27),
+  // a copied ghost layer takes them (loaded here, stored when the halo lines are in)
+  constexpr int per = NSP * NSP * 4, NC = (4 * per + THREADS - 1) / THREADS;
+  auto corner = [&](int v) -> long long {
+    const int c = v / per, o = v % per;
+    const long long ci = (c & 1) ? geo.nx + 1 : 0, cj = (c & 2) ? geo.ny + 1 : 0;
+    return ci + (long long)nxg * cj + ldp * o;
+  };
+  const bool corners = blockIdx.x == 0 && (EPI == EPI_RESIDUAL || sa.gc0 != nullptr);
+  double cv[NC];
+  if (corners) {
+#pragma unroll
+    for (int n = 0; n < NC; ++n) {
+      const int v = tid + n * THREADS;
+      if (v >= 4 * per) break;
+      if constexpr (EPI == EPI_RESIDUAL)
+        sa.out[corner(v)] = 0.0;
+      else
+        cv[n] = u[corner(v)];
     }
   }
 
@@ -310,19 +310,30 @@ __global__ __launch_bounds__(kTilesPerWg<NSP> * NSP * 64, (fr2d_min_waves<NSP, F
     // the ghost element's line is copied to gc0, gc1 when asked (then hi, hj = si, sj)
     const bool ghost = hi == 0 || hi == geo.nx + 1 || hj == 0 || hj == geo.ny + 1;
     const bool gcopy = EPI != EPI_RESIDUAL && ghost && sa.gc0 != nullptr;
+    // every value is loaded before the first is stored: with a copy after each load the tiles along
+    // the boundary took a round trip per value (100 x 50, p = 2: 11.0 us for the copying stage, 6.7
+    // for one without).  10 SSP-RK3 steps: polar cells 256 x 256 849 -> 793 us, 201 x 133, p = 4 576 -> 544;
+    // 20 steps at 256 x 256, HLL with ghosts 1297 -> 1200, Rusanov periodic 1070 -> 1073
+    double hv[4][NSP];
+#pragma unroll
+    for (int m = 0; m < 4; ++m)
+#pragma unroll
+      for (int q = 0; q < NSP; ++q) hv[m][q] = LDL(u, pb + ps * q, m, hbo);
 #pragma unroll
     for (int m = 0; m < 4; ++m) {
       double s = 0.0;
 #pragma unroll
-      for (int q = 0; q < NSP; ++q) {
-        const double v = LDL(u, pb + ps * q, m, hbo);
-        s += v * w[q];
-        if (gcopy) {
-          STL(sa.gc0, pb + ps * q, m, hbo, v);
-          STL(sa.gc1, pb + ps * q, m, hbo, v);
-        }
-      }
+      for (int q = 0; q < NSP; ++q) s += hv[m][q] * w[q];
       htr[m] = s;
+    }
+    if (gcopy) {
+#pragma unroll
+      for (int m = 0; m < 4; ++m)
+#pragma unroll
+        for (int q = 0; q < NSP; ++q) {
+          STL(sa.gc0, pb + ps * q, m, hbo, hv[m][q]);
+          STL(sa.gc1, pb + ps * q, m, hbo, hv[m][q]);
+        }
     }
     if constexpr (EPI == EPI_RESIDUAL) {
       // du vanishes on the ghost layer (example/shock-vortex.jl:27)
@@ -333,6 +344,16 @@ __global__ __launch_bounds__(kTilesPerWg<NSP> * NSP * 64, (fr2d_min_waves<NSP, F
 #pragma unroll
           for (int q = 0; q < NSP; ++q) STL(sa.out, pb + ps * q, m, gbo, 0.0);
       }
+    }
+  }
+
+  if (EPI != EPI_RESIDUAL && corners) {
+#pragma unroll
+    for (int n = 0; n < NC; ++n) {
+      const int v = tid + n * THREADS;
+      if (v >= 4 * per) break;
+      sa.gc0[corner(v)] = cv[n];
+      sa.gc1[corner(v)] = cv[n];
     }
   }
 
@@ -781,16 +802,6 @@ bool fr2d_single_round(const Fr2dCtx &c) {
   const long long nb = (long long)((c.nx + TX - 1) / TX) * ((c.ny + TY - 1) / TY);
   return c.nsp == 4 && c.flux != FR_FLUX_ROE && c.geom != 2 && c.num_cu > 0 && nb > c.num_cu &&
          nb <= 4LL * c.num_cu;
-}
-
-// Delay of the staggered start for a context that has none set.  20 SSP-RK3 steps in us with 0 / 3 / 5 / 7
-// units: Rusanov 256 x 256 periodic 1103 / 1052 / 1056 / 1188, with ghosts 1228 / 1167 / 1178 / 1314,
-// 256 x 240 1173 / 1138 / 1154 / 1262, parallelograms 300 x 200 1114 / 1106 / 1115 / 1243, 250 x 199
-// 1117 / 1104 / 1112 / 1139, 200 x 150 (two workgroups per CU) 679 / 676 / 676 / 676; HLL 256 x 256
-// 1296 / 1297 / 1294 / 1293 and 180 x 180 968 / 973 / 972 / 974.  Timing the candidates on the device
-// in a context's first call chose no better and cost that call 34 ms.
-int fr2d_default_stagger(const Fr2dCtx &c) {
-  return fr2d_single_round(c) && c.flux == FR_FLUX_RUSANOV ? 3 : 0;
 }
 
 int fr2d_launch_fill_ghost(const Fr2dCtx &c, double *d_u, int rule, hipStream_t st) {

@@ -32,7 +32,7 @@ struct Fr2dCtx {
   // Staggered start of the RK stage launches whose tiles are all resident at once (at most four
   // workgroups per CU): workgroup slot s of a CU (s = block / num_cu) first sleeps s * stagger
   // units of 64 x 8 clocks, so the load phases of the workgroups sharing a CU do not coincide.
-  // -1: not set yet (the first stepping call takes fr2d_default_stagger), 0: off.  Only the timing
+  // -1: not set yet (the first stepping call sets 0), 0: off.  Only the timing
   // changes, never the arithmetic.
   int stagger = -1;
   // the caller's stream (caller_stream: any hipStream_t, NULL being HIP's null stream) or the
@@ -75,10 +75,8 @@ int fr2d_launch_stage(const Fr2dCtx &c, const double *d_u0, const double *d_us, 
                       double a1, double b, const double *acc_in, double *acc_out, double b2, hipStream_t st,
                       double *ghost_copy0 = nullptr, double *ghost_copy1 = nullptr);
 int fr2d_launch_fill_ghost(const Fr2dCtx &c, double *d_u, int rule, hipStream_t st);
-// whether the RK stage launches of c have every tile resident at once (the staggered start
-// applies), and the delay it takes unless the caller sets one
+// whether the RK stage launches of c have every tile resident at once (a staggered start applies)
 bool fr2d_single_round(const Fr2dCtx &c);
-int fr2d_default_stagger(const Fr2dCtx &c);
 // eval_out != nullptr: write the per-cell strength multiplier (modal: 0/1, learned: MLP output)
 // instead of filtering
 int fr2d_launch_sensor_filter(const Fr2dCtx &c, double *d_u, int mode, double lambda, double S0, double kappa,
