@@ -305,7 +305,7 @@ __device__ __forceinline__ bool shock_switch(double Se, double S0, double kappa)
 // -0.98.  NaN when it is out of the range in which shock_flagged may compare against it.
 inline double shock_cut(double S0, double kappa) {
   const double q = std::pow(10.0, S0 - kappa * (2.0 / M_PI) * std::asin(0.98));
-  return q > 1e-100 && q < 1e100 ? q : std::nan("");
+  return kappa >= 0.0 && q > 1e-100 && q < 1e100 ? q : std::nan("");
 }
 
 // shock_switch(log10(top / all), S0, kappa) with q = shock_cut(S0, kappa): the logarithm and the sine
