@@ -5,7 +5,7 @@
 // and, in stage mode, the explicit RK update out = a0*u0 + a1*u + b*L(u) in its epilogue.
 //
 // Mapping: a tile of TX x TY = 16 x 4 elements is worked on by NSP wavefronts, a workgroup owns one
-// tile (two at nsp = 5, kTilesPerWg).  Lane =
+// tile (at nsp = 5 two, kTilesPerWg).  Lane =
 // element of the tile (16 consecutive elements along x per row, so every global access of a
 // wavefront covers four 128-byte segments of the element-fastest SoA layout), wave index = one
 // line of solution points.  Each thread first holds row `line` of its element and finishes the
@@ -24,6 +24,7 @@
 #include <algorithm>
 #include <cstring>
 #include <new>
+#include <type_traits>
 
 #include "fr_common.h"
 #include "fr2d_internal.h"
@@ -117,13 +118,15 @@ __device__ __forceinline__ double row_shift(double x) {
 // 168 VGPRs of nsp = 5 hold three each, and one such workgroup was resident per CU (5.06 waves by the
 // counters) where LDS and registers allow two; with two tiles in a workgroup of ten (3, 3, 2, 2) ten are.
 // Per SSP-RK3 stage: 201 x 133, HLL 24.9 -> 19.1 us, 560 x 500, Rusanov 201 -> 176 us, Roe 223 -> 187, polar
-// cells 268 -> 231.  At nsp = 6 two tiles have to fit 168 VGPRs and spill: 466 x 500 239 -> 249 us, polar
-// cells 289 -> 387.
-template <int NSP>
-constexpr int kTilesPerWg = NSP == 5 ? 2 : 1;
+// cells 268 -> 231.  Grids of no more tiles than CUs keep one (every tile has a CU to itself: 20 x 14, seven
+// steps 305 us with one, 336 with two), and so does the RK4 form on point metrics, which would spill 50
+// values.  At nsp = 6 two tiles have to fit 168 VGPRs and spill: 466 x 500 239 -> 249 us, polar cells
+// 289 -> 387.
+template <int NSP, int EPI, int GEO>
+constexpr int kTilesPerWg = NSP == 5 && !(EPI == EPI_ACC && GEO == GEO_POINT) ? 2 : 1;
 
-template <int NSP, int FLUX, int EPI, int ADDR, int GEO>
-__global__ __launch_bounds__(kTilesPerWg<NSP> * NSP * 64, (fr2d_min_waves<NSP, FLUX, EPI, GEO>())) void fr2d_kernel(
+template <int NSP, int FLUX, int EPI, int ADDR, int GEO, int NT>
+__global__ __launch_bounds__(NT * NSP * 64, (fr2d_min_waves<NSP, FLUX, EPI, GEO>())) void fr2d_kernel(
     const Geo2D geo, const StageArgs sa) {
   // operators are compile-time constants (Gauss-Legendre points, Radau correction), so they
   // occupy no scalar registers for the length of the kernel
@@ -131,7 +134,7 @@ __global__ __launch_bounds__(kTilesPerWg<NSP> * NSP * 64, (fr2d_min_waves<NSP, F
   // LDS: the tile transpose sU (rows -> columns, then the y contributions columns -> rows) and
   // the tile's right x-faces (sX).  The y faces of a line live in that line's own column block
   // of sU between the column read and the write-back of the y contributions.
-  constexpr int NT = kTilesPerWg<NSP>, THREADS = NT * NSP * 64;
+  constexpr int THREADS = NT * NSP * 64;
   __shared__ double sUt[NT][NSP * NSP * 4 * TE];
   __shared__ double sXt[NT][4 * NSP * TY];
 
@@ -718,24 +721,33 @@ static int launch_nsp(const Fr2dCtx &c, const StageArgs &sa, hipStream_t st) {
   // reference-layout one when the padded pitch is nx + 2)
   geo.mj = geo.pitch == c.nx + 2 ? c.d_mj_ref : c.d_mj_pad;
   if (c.geom == 2 && !geo.mj) return fail(FR_E_INVALID, "fr2d: point metrics missing on the device");
-  constexpr int NT = kTilesPerWg<NSP>;
-  const unsigned nb = (unsigned)((geo.ntx * geo.nty + NT - 1) / NT);
+  const long long tiles = (long long)geo.ntx * geo.nty;
   const bool stag = !caller && c.stagger > 0 && fr2d_single_round(c);
   geo.stag_cu = stag ? c.num_cu : 0;
   geo.stag = stag ? c.stagger : 0;
   const bool buf = (caller ? c.len : c.lenp) * sizeof(double) < (size_t)0xFFFFFFFFu;
-  if (c.geom == 0 && buf)
-    hipLaunchKernelGGL((fr2d_kernel<NSP, FLUX, EPI, ADDR_BUFFER, GEO_RECT>), dim3(nb), dim3(NT * NSP * 64), 0, st, geo, sa);
-  else if (c.geom == 0)
-    hipLaunchKernelGGL((fr2d_kernel<NSP, FLUX, EPI, ADDR_FLAT, GEO_RECT>), dim3(nb), dim3(NT * NSP * 64), 0, st, geo, sa);
-  else if (c.geom == 1 && buf)
-    hipLaunchKernelGGL((fr2d_kernel<NSP, FLUX, EPI, ADDR_BUFFER, GEO_AFFINE>), dim3(nb), dim3(NT * NSP * 64), 0, st, geo, sa);
+  auto go = [&](auto kernel, int nt) {
+    hipLaunchKernelGGL(kernel, dim3((unsigned)((tiles + nt - 1) / nt)), dim3(nt * NSP * 64), 0, st, geo, sa);
+  };
+  auto pick = [&](auto addr, auto geom) {
+    constexpr int A = decltype(addr)::value, G = decltype(geom)::value, NT = kTilesPerWg<NSP, EPI, G>;
+    if (NT > 1 && tiles > c.num_cu)
+      go(fr2d_kernel<NSP, FLUX, EPI, A, G, NT>, NT);
+    else
+      go(fr2d_kernel<NSP, FLUX, EPI, A, G, 1>, 1);
+  };
+  auto by_addr = [&](auto geom) {
+    if (buf)
+      pick(std::integral_constant<int, ADDR_BUFFER>{}, geom);
+    else
+      pick(std::integral_constant<int, ADDR_FLAT>{}, geom);
+  };
+  if (c.geom == 0)
+    by_addr(std::integral_constant<int, GEO_RECT>{});
   else if (c.geom == 1)
-    hipLaunchKernelGGL((fr2d_kernel<NSP, FLUX, EPI, ADDR_FLAT, GEO_AFFINE>), dim3(nb), dim3(NT * NSP * 64), 0, st, geo, sa);
-  else if (buf)
-    hipLaunchKernelGGL((fr2d_kernel<NSP, FLUX, EPI, ADDR_BUFFER, GEO_POINT>), dim3(nb), dim3(NT * NSP * 64), 0, st, geo, sa);
+    by_addr(std::integral_constant<int, GEO_AFFINE>{});
   else
-    hipLaunchKernelGGL((fr2d_kernel<NSP, FLUX, EPI, ADDR_FLAT, GEO_POINT>), dim3(nb), dim3(NT * NSP * 64), 0, st, geo, sa);
+    by_addr(std::integral_constant<int, GEO_POINT>{});
   FR_LAUNCHED("fr2d_kernel");
   return FR_OK;
 }
