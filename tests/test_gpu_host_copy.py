@@ -21,3 +21,34 @@ def test_large_host_state_round_trip(nbytes):
         pr.set_state(u)
         assert np.array_equal(pr.get_state(), u)
         u = -u[::-1]
+
+
+@pytest.mark.parametrize("stream", ["own", "null", "per_thread", "torch"])
+def test_large_host_state_behind_queued_steps(stream):
+    """Steps are queued and not waited for: a state read back holds them, a state put in comes after them
+    (hipStreamPerThread is handle 2, another stream in every thread)."""
+    import ctypes as C
+
+    torch = pytest.importorskip("torch")
+    ncell = FROM // 16 + 3 * CHUNK // 16 + 5
+    pr = frhip.FRAdvectionProblem(frhip.FRPSpace1D(0.0, 1.0, ncell, 1), 1.0, "period")
+    u = np.asfortranarray(np.random.default_rng(0).standard_normal((ncell, 2)))
+    steps = (0.1 / ncell, 400, "ssprk3")
+    pr.set_state(u)
+    pr.step(*steps)
+    torch.cuda.synchronize()
+    ref = pr.get_state()
+    side = torch.cuda.Stream()
+    if stream != "own":
+        handle = {"null": 0, "per_thread": 2, "torch": side.cuda_stream}[stream]
+        assert frhip.lib().fr1d_set_stream(pr.h, C.c_void_p(handle)) == 0
+    for _ in range(2):
+        pr.set_state(u)
+        pr.step(*steps)
+        assert np.array_equal(pr.get_state(), ref)
+        pr.step(*steps)
+        pr.set_state(u)
+        torch.cuda.synchronize()
+        pr.step(0.1 / ncell, 0)
+        assert np.array_equal(pr.get_state(), u)
+    pr.close()
