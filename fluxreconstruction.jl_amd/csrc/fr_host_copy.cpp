@@ -100,16 +100,25 @@ static int staged(HostStaging &s, char *dev, char *host, size_t bytes, bool up, 
   return FR_OK;
 }
 
+// Whether the runtime knows the array: pinned, managed or on a device.
+static bool registered(const void *host) {
+  hipPointerAttribute_t at{};
+  if (hipPointerGetAttributes(&at, host) == hipSuccess) return at.type != hipMemoryTypeUnregistered;
+  (void)hipGetLastError();
+  return false;
+}
+
 // Whether the chunks serve a copy.  The workers all name the caller's stream, so its handle has to mean one
 // stream in every thread: hipStreamPerThread is another stream in each of them, whose copies would not
-// wait for the work that the caller has queued.
-static bool staging_serves(size_t bytes, hipStream_t st) {
-  return bytes >= HostStaging::kFrom && st != hipStreamPerThread;
+// wait for the work that the caller has queued.  An array that the runtime knows goes over the bus as it
+// is: 40 MB pinned 739 us in and 745 us out, by way of the chunks 1128 and 1140.
+static bool staging_serves(const void *host, size_t bytes, hipStream_t st) {
+  return bytes >= HostStaging::kFrom && st != hipStreamPerThread && !registered(host);
 }
 
 int copy_to_device(HostStaging &s, double *dev, const double *host, size_t n, hipStream_t st) {
   const size_t bytes = n * sizeof(double);
-  if (staging_serves(bytes, st) && s.ensure(st) == FR_OK)
+  if (staging_serves(host, bytes, st) && s.ensure(st) == FR_OK)
     return staged(s, (char *)dev, (char *)const_cast<double *>(host), bytes, true, st);
   FR_HIP(hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, st));
   FR_HIP(hipStreamSynchronize(st));
@@ -118,7 +127,7 @@ int copy_to_device(HostStaging &s, double *dev, const double *host, size_t n, hi
 
 int copy_to_host(HostStaging &s, double *host, const double *dev, size_t n, hipStream_t st) {
   const size_t bytes = n * sizeof(double);
-  if (staging_serves(bytes, st) && s.ensure(st) == FR_OK)
+  if (staging_serves(host, bytes, st) && s.ensure(st) == FR_OK)
     return staged(s, (char *)const_cast<double *>(dev), (char *)host, bytes, false, st);
   FR_HIP(hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, st));
   FR_HIP(hipStreamSynchronize(st));

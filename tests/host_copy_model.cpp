@@ -34,6 +34,9 @@ std::mutex mu;  // of the maps
 std::map<std::pair<hipStream_t, std::thread::id>, Queue> queues;
 std::map<hipEvent_t, Queue *> events;
 
+const void *pinned = nullptr;  // the one array that the runtime knows
+int copies = 0;
+
 Queue &queue(hipStream_t s) {
   std::lock_guard<std::mutex> l(mu);
   return queues[{s, s == hipStreamPerThread ? std::this_thread::get_id() : std::thread::id()}];
@@ -49,6 +52,10 @@ hipError_t hipHostMalloc(void **p, size_t n, unsigned) { return *p = std::malloc
 hipError_t hipHostFree(void *p) { return std::free(p), hipSuccess; }
 hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned) { return *e = (hipEvent_t) new char, hipSuccess; }
 hipError_t hipEventDestroy(hipEvent_t e) { return delete (char *)e, hipSuccess; }
+hipError_t hipPointerGetAttributes(hipPointerAttribute_t *a, const void *p) {
+  if (p != pinned) return hipErrorInvalidValue;
+  return a->type = hipMemoryTypeHost, hipSuccess;
+}
 hipError_t hipEventRecord(hipEvent_t e, hipStream_t s) {
   Queue &q = queue(s);
   std::lock_guard<std::mutex> l(mu);
@@ -65,7 +72,10 @@ hipError_t hipEventSynchronize(hipEvent_t e) {
 }
 hipError_t hipStreamSynchronize(hipStream_t s) { return queue(s).drain(), hipSuccess; }
 hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind, hipStream_t st) {
-  queue(st).push([=] { std::memcpy(d, s, n); });
+  queue(st).push([=] {
+    ++copies;
+    std::memcpy(d, s, n);
+  });
   return hipSuccess;
 }
 }
@@ -103,10 +113,27 @@ static void ordered(const char *what, hipStream_t st) {
   s.release();
 }
 
+// arrays that the runtime knows are copied as they are, by one copy each way
+static void straight(hipStream_t st) {
+  const size_t n = fr::HostStaging::kFrom / 8 + 1;
+  std::vector<double> dev(n, 1.0), host(n, 2.0);
+  pinned = host.data();
+  copies = 0;
+  fr::HostStaging s;
+  int rc = fr::copy_to_device(s, dev.data(), host.data(), n, st);
+  check("pinned array: one copy in", rc == 0 && copies == 1 && !s.buf && dev == host);
+  dev.assign(n, 3.0);
+  rc = fr::copy_to_host(s, host.data(), dev.data(), n, st);
+  check("pinned array: one copy out", rc == 0 && copies == 2 && !s.buf && dev == host);
+  s.release();
+  pinned = nullptr;
+}
+
 int main() {
   int own = 0;
   ordered("own stream", (hipStream_t)&own);
   ordered("null stream", nullptr);
   ordered("per-thread stream", hipStreamPerThread);
+  straight((hipStream_t)&own);
   return failed;
 }

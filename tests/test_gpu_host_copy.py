@@ -52,3 +52,20 @@ def test_large_host_state_behind_queued_steps(stream):
         pr.step(0.1 / ncell, 0)
         assert np.array_equal(pr.get_state(), u)
     pr.close()
+
+
+def test_large_pinned_state_round_trip():
+    import ctypes as C
+
+    torch = pytest.importorskip("torch")
+    ncell = FROM // 16 + 77
+    pr = frhip.FRAdvectionProblem(frhip.FRPSpace1D(0.0, 1.0, ncell, 1), 1.0, "period")
+    u = torch.empty(2 * ncell, dtype=torch.float64, pin_memory=True)
+    out = torch.zeros(2 * ncell, dtype=torch.float64, pin_memory=True)
+    u.copy_(torch.from_numpy(np.random.default_rng(1).standard_normal(2 * ncell)))
+    ptr = lambda t: C.cast(t.data_ptr(), C.POINTER(C.c_double))  # noqa: E731
+    assert frhip.lib().fr1d_set_state(pr.h, ptr(u)) == 0
+    assert frhip.lib().fr1d_get_state(pr.h, ptr(out)) == 0
+    assert torch.equal(out, u)
+    assert np.array_equal(pr.get_state().ravel(order="F"), u.numpy())
+    pr.close()

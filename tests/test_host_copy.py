@@ -1,5 +1,6 @@
 """csrc/fr_host_copy.cpp against a model of the HIP runtime (host_copy_model.cpp): copies between host
-arrays and the device come after the work queued on the caller's stream, whatever stream that is."""
+arrays and the device come after the work queued on the caller's stream, whatever stream that is, and
+arrays that the runtime knows are not copied twice."""
 import os
 import shutil
 import subprocess
