@@ -37,7 +37,8 @@ int hip_fail(hipError_t e, const char *what, const char *file, int line);
 struct HostStaging {
   static constexpr int kWorkers = 4;
   static constexpr size_t kChunk = 2u << 20;
-  static constexpr size_t kFrom = 24u << 20;  // bytes of a copy from which on it pays, its first one too
+  // bytes of a copy to the host and to the device from which on it pays, a context's first one too
+  static constexpr size_t kFromOut = 24u << 20, kFromIn = 30u << 20;
   char *buf = nullptr;
   hipEvent_t ev[2 * kWorkers] = {};
   int device = 0;

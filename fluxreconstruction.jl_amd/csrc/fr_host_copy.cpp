@@ -3,10 +3,11 @@
 // One hipMemcpyAsync on a pageable array pins and copies piece by piece in the calling thread, and a
 // fresh result array takes its page faults there too.  Large copies go through pinned chunks instead:
 // a few worker threads, each with two chunks, move the caller's pages while the other chunk is on the
-// bus.  Plain and staged, into a fresh array: 8 MB 474 / 328 us, 16 MB 916 / 512, 32 MB 3.13 / 1.43 ms,
-// 53 MB 5.27 / 1.74 ms; from one: 16 MB 445 / 508 us, 32 MB 1020 / 931, 53 MB 1849 / 1514.  The chunks
-// (16 MB) take about 0.7 ms to pin, once per context, hence HostStaging::kFrom.  Chunks of 1 MB took 2.0
-// and 1.87 ms at 53 MB, of 4 MB 1.74 and 1.34.
+// bus.  Plain and staged, into a fresh array: 8 MB 474 / 328 us, 16 MB 916 / 512, 24 MB 1742 / 1080, 32 MB
+// 2234 / 1273, 53 MB 5.27 / 1.74 ms; from one: 24 MB 668 / 714 us, 28 MB 798 / 815, 30 MB 864 / 864, 32 MB
+// 931 / 907, 40 MB 1350 / 1131, 53 MB 1849 / 1514.  The chunks (16 MB) take about 0.7 ms to pin, once per
+// context, hence HostStaging::kFromOut and kFromIn.  Chunks of 1 MB took 2.0 and 1.87 ms at 53 MB, of 4 MB
+// 1.74 and 1.34.
 #include <algorithm>
 #include <cstring>
 #include <exception>
@@ -112,13 +113,13 @@ static bool registered(const void *host) {
 // stream in every thread: hipStreamPerThread is another stream in each of them, whose copies would not
 // wait for the work that the caller has queued.  An array that the runtime knows goes over the bus as it
 // is: 40 MB pinned 739 us in and 745 us out, by way of the chunks 1128 and 1140.
-static bool staging_serves(const void *host, size_t bytes, hipStream_t st) {
-  return bytes >= HostStaging::kFrom && st != hipStreamPerThread && !registered(host);
+static bool staging_serves(const void *host, size_t bytes, size_t from, hipStream_t st) {
+  return bytes >= from && st != hipStreamPerThread && !registered(host);
 }
 
 int copy_to_device(HostStaging &s, double *dev, const double *host, size_t n, hipStream_t st) {
   const size_t bytes = n * sizeof(double);
-  if (staging_serves(host, bytes, st) && s.ensure(st) == FR_OK)
+  if (staging_serves(host, bytes, HostStaging::kFromIn, st) && s.ensure(st) == FR_OK)
     return staged(s, (char *)dev, (char *)const_cast<double *>(host), bytes, true, st);
   FR_HIP(hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, st));
   FR_HIP(hipStreamSynchronize(st));
@@ -127,7 +128,7 @@ int copy_to_device(HostStaging &s, double *dev, const double *host, size_t n, hi
 
 int copy_to_host(HostStaging &s, double *host, const double *dev, size_t n, hipStream_t st) {
   const size_t bytes = n * sizeof(double);
-  if (staging_serves(host, bytes, st) && s.ensure(st) == FR_OK)
+  if (staging_serves(host, bytes, HostStaging::kFromOut, st) && s.ensure(st) == FR_OK)
     return staged(s, (char *)const_cast<double *>(dev), (char *)host, bytes, false, st);
   FR_HIP(hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, st));
   FR_HIP(hipStreamSynchronize(st));

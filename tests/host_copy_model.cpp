@@ -93,7 +93,7 @@ static void check(const char *what, bool ok) {
 
 // a copy each way behind queued work on the same stream: the work adds one to every device value
 static void ordered(const char *what, hipStream_t st) {
-  const size_t n = fr::HostStaging::kFrom / 8 + 3 * fr::HostStaging::kChunk / 8 + 1;
+  const size_t n = fr::HostStaging::kFromIn / 8 + 3 * fr::HostStaging::kChunk / 8 + 1;
   std::vector<double> dev(n, 1.0), host(n, 0.0);
   auto step = [&] {
     queue(st).push([&] {
@@ -115,7 +115,7 @@ static void ordered(const char *what, hipStream_t st) {
 
 // arrays that the runtime knows are copied as they are, by one copy each way
 static void straight(hipStream_t st) {
-  const size_t n = fr::HostStaging::kFrom / 8 + 1;
+  const size_t n = fr::HostStaging::kFromIn / 8 + 1;
   std::vector<double> dev(n, 1.0), host(n, 2.0);
   pinned = host.data();
   copies = 0;
@@ -129,11 +129,26 @@ static void straight(hipStream_t st) {
   pinned = nullptr;
 }
 
+// 28 MiB: one copy in, which the chunks would make slower, and chunks out
+static void lines(hipStream_t st) {
+  const size_t n = (28u << 20) / 8;
+  std::vector<double> dev(n, 1.0), host(n, 2.0);
+  copies = 0;
+  fr::HostStaging s;
+  int rc = fr::copy_to_device(s, dev.data(), host.data(), n, st);
+  check("28 MiB: one copy in", rc == 0 && copies == 1 && dev == host);
+  dev.assign(n, 3.0);
+  rc = fr::copy_to_host(s, host.data(), dev.data(), n, st);
+  check("28 MiB: chunks out", rc == 0 && copies == 1 + 14 && dev == host);
+  s.release();
+}
+
 int main() {
   int own = 0;
   ordered("own stream", (hipStream_t)&own);
   ordered("null stream", nullptr);
   ordered("per-thread stream", hipStreamPerThread);
   straight((hipStream_t)&own);
+  lines((hipStream_t)&own);
   return failed;
 }
