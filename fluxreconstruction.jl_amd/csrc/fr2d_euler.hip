@@ -169,11 +169,15 @@ __global__ __launch_bounds__(NT * NSP * 64, (fr2d_min_waves<NSP, FLUX, EPI, GEO>
   auto SY = [&](int m, int fy, int x) -> double & { return sYl[(m * (TY + 1) + fy) * TX + x]; };
   // value of plane (k, l, m) at the element with byte offset bo inside the plane
   const unsigned ldp8 = (unsigned)(ldp * 8);
+  // byte offset of a plane, said to be uniform once more where it is used: where the compiler loses sight of
+  // it, a loop over the lanes' values goes around the access (residual, p = 3, per call: 560 x 500 94 us with
+  // such loops around the stores, 87 without; 1000 x 600 223 and 193; polar cells 300 x 200 25.4 and 24.5)
+  auto plane_off = [&](int plane) { return __builtin_amdgcn_readfirstlane((int)(ldp8 * (unsigned)plane)); };
   auto LD = [&](const double *base, int k, int l, int m, unsigned bo) -> double {
     const int plane = k + NSP * (l + NSP * m);
     if constexpr (ADDR == ADDR_BUFFER)
       return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(plane_rsrc(base, 0xFFFFFFFFu), bo,
-                                                                             (int)(ldp8 * (unsigned)plane), 0));
+                                                                             plane_off(plane), 0));
     else
       return *reinterpret_cast<const double *>(reinterpret_cast<const char *>(base + ldp * plane) + bo);
   };
@@ -184,7 +188,7 @@ __global__ __launch_bounds__(NT * NSP * 64, (fr2d_min_waves<NSP, FLUX, EPI, GEO>
     const int plane = k + NSP * (l + NSP * m);
     if constexpr (ADDR == ADDR_BUFFER)
       __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(fr_u2, v), plane_rsrc(base, 0xFFFFFFFFu), bo,
-                                            (int)(ldp8 * (unsigned)plane), kStAux);
+                                            plane_off(plane), kStAux);
     else
       *reinterpret_cast<double *>(reinterpret_cast<char *>(base + ldp * plane) + bo) = v;
   };
