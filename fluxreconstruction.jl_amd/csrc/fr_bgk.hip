@@ -294,6 +294,17 @@ constexpr bool kBgkSums = NSP < 5;
 // 8 MB (20 x 33, p = 2, 16 x 11 velocities) 225 / 271 us, 32 MB 328 / 342, 68 MB 620 / 517, 97 MB
 // (57 x 43, p = 2, 24 x 24) 1207 / 727.
 constexpr size_t kBgkStream = 64u << 20;
+// Grids inside one 16 x 16 tile with up to kBgkFewVel velocities are then many members, and a workgroup per
+// member and velocity range leaves most lanes without a cell: the line rises as the share of lanes with
+// one falls, kBgkFill of bytes per share.  One step, cached path / this one, 70 and 300 MB, 12 x 12
+// velocities: 1 x 1 cells, p = 2, 1.78 and 1.63 times as long here, 4 x 4 1.65 and 1.29, 6 x 6 1.36 and 1.02, 8 x 8
+// 1.20 and 0.89, 12 x 12 0.99 and 0.80; p = 3: 4 x 4 1.06 and 1.00, 6 x 6 0.85 and 0.65, 10 x 10 (two of its tiles)
+// 1.16 and 0.98; p = 4 0.2 to 0.7 everywhere.  With more velocities (few points, whose sums the cached path forms one after
+// another) 0.1 to 0.7: 1 x 1 cells, p = 2, 1079 x 1079 velocities 0.24, 8 x 8, p = 1, 202 x 202 0.24.
+constexpr int kBgkFewVel = 48 * 48;
+constexpr size_t bgk_fill(int nsp, long long tiles) {
+  return nsp >= 5 ? 0 : nsp == 4 && tiles == 1 ? 32u << 20 : 48u << 20;
+}
 
 // Operators by the sign of the velocity component (0: positive, 1: otherwise).  Upwind, only the face
 // towards the neighbour has a correction: D carries its own-trace part, D = dl - dhl ll' (positive) or
@@ -716,7 +727,15 @@ struct BgkCtx {
     return FR_OK;
   }
 
-  bool large() const { return len * sizeof(double) > kBgkStream; }
+  // whether the stage kernel serves (kBgkStream, bgk_fill)
+  bool large() const {
+    const size_t bytes = len * sizeof(double);
+    if (bytes <= kBgkStream) return false;
+    if (nx > BT || ny > BT || (long long)nu * nv > kBgkFewVel) return true;
+    const int bc = nsp <= 3 ? kBgkCells<3> : nsp == 4 ? kBgkCells<4> : kBgkCells<5>;
+    const long long tiles = bgk_tiles(bc, geom.tsh);
+    return (double)bytes * (double)geom.cells > (double)bgk_fill(nsp, tiles) * (double)(tiles * bc);
+  }
 
   int stage_cached(const BgkStage &sa, hipStream_t st) const {
     const int rc = launch_moments(sa.u, st);

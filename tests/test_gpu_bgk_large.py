@@ -55,3 +55,28 @@ def test_steps_of_one_call_and_of_several(nx, ny, deg, nv):
         g.set_state(f0)
         g.step(dt, n)
         assert np.array_equal(g.get_state(), outs[n - 1])
+
+
+@pytest.mark.parametrize("nx,ny,deg,nv,nmem", [(1, 1, 2, 12, 7000), (3, 5, 1, 16, 600), (4, 4, 3, 16, 170), (6, 6, 3, 16, 115),
+                                               (14, 14, 2, 16, 20), (2, 2, 1, 49, 230)])
+def test_many_members_of_few_cells(nx, ny, deg, nv, nmem):
+    """States above 64 MiB on either side of the line that the share of lanes with a cell draws: the first
+    and the last members against the oracle."""
+    u, wu = bgk.velocity_grid(nv)
+    taus = np.geomspace(1e-2, 1e-1, nmem)
+    one = bgk.maxwellian_state(nx, ny, deg, u, u, amp=0.1)
+    rng = np.random.default_rng(nmem)
+    f0 = (one[None, :] * (1.0 + 0.02 * rng.uniform(-1, 1, (nmem, 1)))).ravel()
+    assert f0.nbytes > 64 << 20
+    dt = 0.1 / (deg + 1) / max(nx, ny) / np.abs(u).max()
+    g = bgk.BGK2D(nx, ny, deg, u, wu, u, wu, taus)
+    g.set_state(f0)
+    g.step(dt, 1)
+    out = g.get_state().reshape(nmem, -1)
+    for b in (0, 1, nmem // 2, nmem - 1):
+        f = f0.reshape(nmem, -1)[b]
+        L = lambda x: O.bgk2d_rhs(x, nx, ny, deg, u, wu, u, wu, taus[b]).ravel()  # noqa: B023, E731
+        a = f + dt * L(f)
+        c = 0.75 * f + 0.25 * a + 0.25 * dt * L(a)
+        ref = f / 3 + 2 / 3 * c + 2 / 3 * dt * L(c)
+        assert np.linalg.norm(out[b] - ref) <= 1e-12 * np.linalg.norm(ref)
