@@ -396,14 +396,13 @@ __global__ __launch_bounds__(64 * MQ) void bgk_close_kernel(BgkGeo g, const doub
 // in flight, and each thread forms its x sums from its registers and its y sums from LDS.
 // No branch lies around a load or a store, so the waits count them exactly and a wavefront never
 // waits for its own stores: places outside the grid repeat the last cell of their row and column
-// (and store its values again).  COMBINE: with the a0 u0 term.  BUF: buffer access with 32-bit offsets
-// inside one velocity's plane of points (below 4 GiB), which spends no vector instruction on
-// addresses; flat addresses above.
+// (and store its values again).  COMBINE: with the a0 u0 term.  Buffer access with 32-bit offsets inside one
+// velocity's plane of points (below 4 GiB, large()) spends no vector instruction on addresses.
 // 128 x 128, p = 2, 24 x 24 velocities (679 MB a state): 317 us for the first stage, 423 us with u0 (4.6
 // and 5.0 TB/s; a plain copy of 1 GB reaches 5.0), against 135 us of moments and 360 / 578 us of the
 // cached path's transport.  64-cell tiles 357 / 491 us; waits for every load and store 570 us; stores
 // without the streaming hint 4-5 % slower; 128 registers (34 spilled) 1085 us.
-template <int NSP, bool COMBINE, bool BUF>
+template <int NSP, bool COMBINE>
 __global__ __launch_bounds__(kBgkCells<NSP> *NSP) void bgk_stage_kernel(BgkGeo g, BgkOps<NSP> ops,
                                                             const BgkVel *__restrict__ vt,
                                                             const double *__restrict__ tau,
@@ -423,24 +422,18 @@ __global__ __launch_bounds__(kBgkCells<NSP> *NSP) void bgk_stage_kernel(BgkGeo g
   const int i0 = (tile % tiles_x) * BTX, j0 = (tile / tiles_x) * BTY;
   const int ncx = min(BTX, g.nx - i0), ncy = min(BTY, g.ny - j0);
   const int tx = min(c & (BTX - 1), ncx - 1), ty = min(c >> g.tsh, ncy - 1);
-  using OFF = std::conditional_t<BUF, unsigned, unsigned long long>;  // bytes
+  using OFF = unsigned;  // bytes
   auto at_cell = [&](int i, int j) { return (OFF)8 * ((OFF)i + (OFF)g.nx * (OFF)j); };
   const OFF kb = (OFF)(8 * g.cells);  // from one point's cells to the next one's
   // value at byte offset o of point k (uniform) of the plane at base
   auto get = [&](const double *base, OFF o, int k) {
-    if constexpr (BUF)
-      return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(plane_rsrc(base, 0xFFFFFFFFu), o,
-                                                                             (int)(kb * (OFF)k), 0));
-    else
-      return *reinterpret_cast<const double *>(reinterpret_cast<const char *>(base) + kb * (OFF)k + o);
+    return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(plane_rsrc(base, 0xFFFFFFFFu), o,
+                                                                           (int)(kb * (OFF)k), 0));
   };
   constexpr int kAuxNt = 2;
   auto put = [&](double *base, OFF o, int k, double v, auto nt) {
-    if constexpr (BUF)
-      __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(fr_u2, v), plane_rsrc(base, 0xFFFFFFFFu), o,
-                                            (int)(kb * (OFF)k), decltype(nt)::value ? kAuxNt : 0);
-    else
-      *reinterpret_cast<double *>(reinterpret_cast<char *>(base) + kb * (OFF)k + o) = v;
+    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(fr_u2, v), plane_rsrc(base, 0xFFFFFFFFu), o,
+                                          (int)(kb * (OFF)k), decltype(nt)::value ? kAuxNt : 0);
   };
   const OFF own = at_cell(i0 + tx, j0 + ty);
 
@@ -650,15 +643,14 @@ struct BgkCtx {
     }
     const BgkGeo &g = geo();
     const long long tiles = bgk_tiles(kBgkCells<NSP>, g.tsh);
-    const bool buf = g.npts < (1LL << 29);
     auto go = [&](auto kernel) {
       hipLaunchKernelGGL(kernel, dim3((unsigned)(tiles * g.ngrp * nmem)), dim3(kBgkCells<NSP> * NSP), 0, st, g, o, d_vt, d_tau,
                          d_tab, sa, d_part);
     };
     if (sa.a0 == 0.0)
-      buf ? go(bgk_stage_kernel<NSP, false, true>) : go(bgk_stage_kernel<NSP, false, false>);
+      go(bgk_stage_kernel<NSP, false>);
     else
-      buf ? go(bgk_stage_kernel<NSP, true, true>) : go(bgk_stage_kernel<NSP, true, false>);
+      go(bgk_stage_kernel<NSP, true>);
     FR_LAUNCHED("bgk_stage_kernel");
     return FR_OK;
   }
@@ -727,10 +719,11 @@ struct BgkCtx {
     return FR_OK;
   }
 
-  // whether the stage kernel serves (kBgkStream, bgk_fill)
+  // whether the stage kernel serves: kBgkStream, bgk_fill, and a velocity's plane of points below the 4 GiB
+  // that its offsets reach
   bool large() const {
     const size_t bytes = len * sizeof(double);
-    if (bytes <= kBgkStream) return false;
+    if (bytes <= kBgkStream || geom.npts >= (1LL << 29)) return false;
     if (nx > BT || ny > BT || (long long)nu * nv > kBgkFewVel) return true;
     const int bc = nsp <= 3 ? kBgkCells<3> : nsp == 4 ? kBgkCells<4> : kBgkCells<5>;
     const long long tiles = bgk_tiles(bc, geom.tsh);
