@@ -583,7 +583,8 @@ struct BgkCtx {
   BgkVel *d_vt = nullptr;
   double *d_tau = nullptr;
   double *d_cons = nullptr;  // moments of the last moments launch
-  double *d_part = nullptr;  // sums of the velocity groups (large states)
+  // sums of the velocity groups (large states): starts at d_cons, since a call forms them anew where it steps
+  double *d_part = nullptr;
   double *d_tab = nullptr;  // Maxwellian factors Ea | Eb per member
   double *d_u = nullptr, *d_s1 = nullptr, *d_s2 = nullptr, *d_in = nullptr, *d_out = nullptr;
 
@@ -744,7 +745,7 @@ struct BgkCtx {
   void release() {
     if (stream) (void)hipStreamSynchronize(stream);
     staging.release();
-    double *bufs[] = {d_vel, d_tau, d_cons, d_part, d_tab, d_u, d_s1, d_s2, d_in, d_out};
+    double *bufs[] = {d_vel, d_tau, d_cons, d_tab, d_u, d_s1, d_s2, d_in, d_out};
     for (double *b : bufs)
       if (b) (void)hipFree(b);
     if (d_vt) (void)hipFree(d_vt);
@@ -819,9 +820,9 @@ int fr_bgk_create(fr_bgk_ctx **out, const fr_bgk_desc *d) {
     e = hipMemcpy(c->d_vt, vt.data(), vt.size() * sizeof(BgkVel), hipMemcpyHostToDevice);
   if (e == hipSuccess) e = hipMalloc(&c->d_tau, d->nmem * sizeof(double));
   if (e == hipSuccess) e = hipMemcpy(c->d_tau, d->tau, d->nmem * sizeof(double), hipMemcpyHostToDevice);
-  if (e == hipSuccess) e = hipMalloc(&c->d_cons, (size_t)g.npts * 4 * d->nmem * sizeof(double));
-  if (e == hipSuccess && c->large())
-    e = hipMalloc(&c->d_part, (size_t)g.npts * 4 * g.ngrp * d->nmem * sizeof(double));
+  if (e == hipSuccess)
+    e = hipMalloc(&c->d_cons, (size_t)g.npts * 4 * (c->large() ? g.ngrp : 1) * d->nmem * sizeof(double));
+  c->d_part = c->d_cons;
   if (e == hipSuccess) e = hipMalloc(&c->d_tab, (size_t)g.npts * (d->nu + d->nv) * d->nmem * sizeof(double));
   if (e == hipSuccess) e = hipMalloc(&c->d_u, c->len * sizeof(double));
   if (e != hipSuccess) {

@@ -80,3 +80,31 @@ def test_many_members_of_few_cells(nx, ny, deg, nv, nmem):
         c = 0.75 * f + 0.25 * a + 0.25 * dt * L(a)
         ref = f / 3 + 2 / 3 * c + 2 / 3 * dt * L(c)
         assert np.linalg.norm(out[b] - ref) <= 1e-12 * np.linalg.norm(ref)
+
+
+def test_sums_and_moments_share_their_memory():
+    """A new context holds the state, the moments (four per point, or per velocity group: here one) and the
+    Maxwellian factors; moments and right-hand sides between steps leave no trace in them."""
+    torch = pytest.importorskip("torch")
+    u, wu = bgk.velocity_grid(2)
+    torch.zeros(1, device="cuda")
+    g = bgk.BGK2D(8, 8, 1, u, wu, u, wu, [1e-2])  # the library's code is on the device
+    free = torch.cuda.mem_get_info()[0]
+    big = bgk.BGK2D(2048, 2048, 1, u, wu, u, wu, [1e-2])
+    state = 2048 * 2048 * 4 * 4 * 8
+    assert big.len * 8 == state
+    assert free - torch.cuda.mem_get_info()[0] <= 3 * state + (64 << 20)
+    big.close()
+    g.close()
+    u, wu = bgk.velocity_grid(24)
+    f0 = bgk.maxwellian_state(57, 43, 2, u, u, amp=0.1)
+    g = bgk.BGK2D(57, 43, 2, u, wu, u, wu, [1e-2])
+    out = []
+    for between in (lambda: None, lambda: (g.moments(), g.rhs(f0))):
+        g.set_state(f0)
+        g.step(1e-4, 1)
+        between()
+        g.step(1e-4, 1)
+        out.append((g.get_state(), g.moments()))
+    assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1])
+    g.close()
