@@ -143,18 +143,25 @@ __global__ __launch_bounds__(S * P) void bgk1d_moments_kernel(Bgk1dGeo g, const 
   bgk1d_close(m0, m1, m2, g.gamma, pr[g.npts], pr[2 * g.npts], pr[3 * g.npts]);
 }
 
-// x / d with r = 1 / d at hand (d = 0 for an infinite divisor): the quotient by the reciprocal and one
-// correction by its exact remainder, the division's result but for the rarest of last bits (three
-// operations, not ten)
-__device__ __forceinline__ double div_by(double x, double d, double r) {
-  const double q = x * r;
-  return fma(fma(-q, d, x), r, q);
-}
+// Relaxation times below which a context's kernels divide by tau (DIVIDE): the reciprocal of a subnormal one
+// overflows, and a quotient by one below this line may where M - u is far from it.
+constexpr double kTauDivide = 0x1p-500;
 
-// Relaxation time of a member as div_by takes it.
+// Relaxation time of a member: x over it as the quotient by the reciprocal and one correction by its exact
+// remainder, the division's result but for the rarest of last bits (three operations, not ten; d = 0 for an
+// infinite tau).  With tau >= kTauDivide such a quotient overflows, to NaN and not to the division's
+// infinity, only from |x| = 5e157 on, where the moments' squares have overflowed before.  Telling these
+// quotients apart in every kernel took 2 to 40 registers and up to 9 % of a step; DIVIDE divides.
+template <bool DIVIDE>
 struct Bgk1dTau {
   double d, r;
-  __device__ __forceinline__ explicit Bgk1dTau(double tau) : d(isinf(tau) ? 0.0 : tau), r(1.0 / tau) {}
+  __device__ __forceinline__ explicit Bgk1dTau(double tau)
+      : d(!DIVIDE && isinf(tau) ? 0.0 : tau), r(DIVIDE ? 0.0 : 1.0 / tau) {}
+  __device__ __forceinline__ double under(double x) const {
+    if constexpr (DIVIDE) return x / d;
+    const double q = x * r;
+    return fma(fma(-q, d, x), r, q);
+  }
 };
 
 // res[k] of the transport/relaxation operator (bgk_wave.jl:84-128) at one cell and velocity vel,
@@ -162,10 +169,10 @@ struct Bgk1dTau {
 // right trace for vel > 0, the right cell's left trace otherwise), derivative and Radau
 // corrections, plus (M - u) / tau with M = c0 exp(-lambda (vel - U)^2).  w: the cell's values, un: the
 // upwind neighbour's.  Shared by the streaming and the LDS-resident kernels, so both give the same bits.
-template <int NSP>
+template <int NSP, bool DIVIDE>
 __device__ __forceinline__ void bgk1d_cell_velocity(const Bgk1dOps &ops, double iJ, const double *w, const double *un,
                                                     double vel, bool pos, const double *U, const double *lam,
-                                                    const double *c0, const Bgk1dTau &tau, double *res) {
+                                                    const double *c0, const Bgk1dTau<DIVIDE> &tau, double *res) {
   double f[NSP];
 #pragma unroll
   for (int k = 0; k < NSP; ++k) f[k] = vel * w[k] * iJ;
@@ -186,7 +193,7 @@ __device__ __forceinline__ void bgk1d_cell_velocity(const Bgk1dOps &ops, double 
     for (int q = 0; q < NSP; ++q) r1 += f[q] * ops.dl[k + NSP * q];
     const double c = vel - U[k];
     const double M = c0[k] * exp(-lam[k] * (c * c));
-    res[k] = -(r1 + (iL - tl) * ops.dhl[k] + (iR - tr) * ops.dhr[k]) + div_by(M - w[k], tau.d, tau.r);
+    res[k] = -(r1 + (iL - tl) * ops.dhl[k] + (iR - tr) * ops.dhr[k]) + tau.under(M - w[k]);
   }
 }
 
@@ -209,7 +216,7 @@ __device__ __forceinline__ double bgk1d_combine(double a0, double a1, double b, 
 constexpr int kVelMax = 8;
 constexpr long long kVelThreads = 65536;
 
-template <int NSP, bool WITH_U0>
+template <int NSP, bool WITH_U0, bool DIVIDE>
 __global__ __launch_bounds__(256) void bgk1d_rhs_kernel(Bgk1dGeo g, Bgk1dOps ops, const double *__restrict__ uv,
                                                         const double *__restrict__ tau,
                                                         const double *__restrict__ prim, Bgk1dStage sa,
@@ -221,7 +228,7 @@ __global__ __launch_bounds__(256) void bgk1d_rhs_kernel(Bgk1dGeo g, Bgk1dOps ops
   const long long mem = t / per, r = t % per;
   const int i = (int)(r % g.nx), j0 = (int)(r / g.nx) * vpt;
   const long long kst = (long long)g.nx * g.nu;  // stride of the point index
-  const Bgk1dTau tv(tau[mem]);
+  const Bgk1dTau<DIVIDE> tv(tau[mem]);
   const double *pr = prim + mem * 4 * g.npts + i;
   double U[NSP], lam[NSP], c0[NSP];
 #pragma unroll
@@ -316,10 +323,10 @@ struct Div16 {
 
 // One stage C = a0 B + a1 A + b L(A) of the member held in LDS; every thread of the workgroup
 // calls it (it ends with a barrier).  C may be B (written at the value each thread read), never A.
-template <int NSP>
+template <int NSP, bool DIVIDE>
 __device__ __forceinline__ void resident_stage(const Bgk1dGeo &g, const Bgk1dOps &ops, const Div16 &by_pts,
                                                const Div16 &by_nx, const double *uv,
-                                               const double *wv, const Bgk1dTau &tv, const double *A,
+                                               const double *wv, const Bgk1dTau<DIVIDE> &tv, const double *A,
                                                const double *B, double *C, double a0, double a1, double b,
                                                double *part, double *pt) {
   const int tid = threadIdx.x;
@@ -380,7 +387,7 @@ __device__ __forceinline__ void resident_stage(const Bgk1dGeo &g, const Bgk1dOps
 }
 
 // nsteps steps of member blockIdx.x of `state` (read once, written once), the member held in LDS
-template <int NSP>
+template <int NSP, bool DIVIDE>
 __global__ __launch_bounds__(kResidentThreads) void bgk1d_resident_kernel(Bgk1dGeo g, Bgk1dOps ops,
                                                                           const double *__restrict__ uvg,
                                                                           const double *__restrict__ wvg,
@@ -393,7 +400,7 @@ __global__ __launch_bounds__(kResidentThreads) void bgk1d_resident_kernel(Bgk1dG
   double *pt = part + (long long)3 * kMomSlices * g.npts;
   double *uv = pt + 3 * g.npts, *wv = uv + g.nu;
   double *gs = state + (long long)blockIdx.x * ms;
-  const Bgk1dTau tv(tau[blockIdx.x]);
+  const Bgk1dTau<DIVIDE> tv(tau[blockIdx.x]);
   const Div16 by_pts((unsigned)g.npts), by_nx((unsigned)g.nx);
   for (long long v = threadIdx.x; v < ms; v += (int)blockDim.x) X[v] = gs[v];
   for (int j = threadIdx.x; j < g.nu; j += (int)blockDim.x) {
@@ -434,6 +441,7 @@ struct Bgk1dCtx {
   size_t len = 0;
   hipStream_t stream = nullptr;
   HostStaging staging;
+  bool divide = false;  // a member's tau lies below kTauDivide
   hipEvent_t ev = nullptr;  // orders work on a caller stream against the context's stream
   double *d_vel = nullptr;  // u | w
   double *d_tau = nullptr, *d_prim = nullptr;
@@ -478,7 +486,8 @@ struct Bgk1dCtx {
   template <int NSP>
   int launch_resident_n(const Bgk1dSteps &sc, int n, hipStream_t st) const {
     const Bgk1dGeo g = geo();
-    hipLaunchKernelGGL(bgk1d_resident_kernel<NSP>, dim3((unsigned)nmem), dim3((unsigned)resident_threads(g)),
+    hipLaunchKernelGGL((divide ? bgk1d_resident_kernel<NSP, true> : bgk1d_resident_kernel<NSP, false>),
+                       dim3((unsigned)nmem), dim3((unsigned)resident_threads(g)),
                        (unsigned)resident_lds_bytes(g, sc.scheme), st, g, dev_ops(), d_vel, d_vel + nu, d_tau, d_u,
                        sc, n);
     FR_LAUNCHED("bgk1d_resident_kernel");
@@ -504,8 +513,9 @@ struct Bgk1dCtx {
     int dev = 0, v = 0;
     if (hipGetDevice(&dev) != hipSuccess) return 0;
     if (hipDeviceGetAttribute(&v, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess || v <= 0) return 0;
-    if (hipFuncSetAttribute((const void *)bgk1d_resident_kernel<NSP>, hipFuncAttributeMaxDynamicSharedMemorySize, v) !=
-        hipSuccess) {
+    const void *kernel = divide ? (const void *)bgk1d_resident_kernel<NSP, true>
+                                : (const void *)bgk1d_resident_kernel<NSP, false>;
+    if (hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, v) != hipSuccess) {
       (void)hipGetLastError();
       return 0;
     }
@@ -534,7 +544,9 @@ struct Bgk1dCtx {
     while (vpt > 1 && threads() < kVelThreads) vpt /= 2;
     const long long n = threads();
     const bool u0 = !sa.residual && sa.a0 != 0.0;
-    hipLaunchKernelGGL((u0 ? bgk1d_rhs_kernel<NSP, true> : bgk1d_rhs_kernel<NSP, false>),
+    auto kernel = u0 ? (divide ? bgk1d_rhs_kernel<NSP, true, true> : bgk1d_rhs_kernel<NSP, true, false>)
+                     : (divide ? bgk1d_rhs_kernel<NSP, false, true> : bgk1d_rhs_kernel<NSP, false, false>);
+    hipLaunchKernelGGL(kernel,
                        dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, g, o, d_vel, d_tau, d_prim, sa, vpt);
     FR_LAUNCHED("bgk1d_rhs_kernel");
     return FR_OK;
@@ -669,6 +681,7 @@ int fr_bgk1d_create(fr_bgk1d_ctx **out, const fr_bgk1d_desc *d) {
   c->nmem = d->nmem;
   c->dx = d->dx;
   c->gamma = d->gamma;
+  for (int m = 0; m < d->nmem; ++m) c->divide = c->divide || d->tau[m] < kTauDivide;
   if (!build_ops(d->deg, FR_CORR_RADAU, c->ops)) {
     delete c;
     return fail(FR_E_INVALID, "fr_bgk1d_create: operator construction failed");

@@ -290,3 +290,38 @@ def test_create_rejects_bad_input():
     with pytest.raises(ValueError):
         g.set_state(np.zeros(7))
     g.close()
+
+
+@pytest.mark.parametrize("path", ["rhs", "stream", "resident"])
+@pytest.mark.parametrize("tau,scale", [(1e-310, 1.0), (1e-307, 1e3), (1e-301, 1e9), (1e-2, 1.0), (np.inf, 1.0),
+                                       (1.5e308, 1.0)])
+def test_relaxation_is_divided_as_ieee_divides(path, tau, scale):
+    """Quotients that overflow are infinite, not NaN, and a subnormal or infinite relaxation time divides
+    too.  The state is uniform in space, so du = (M - f) / tau but for the rounding of the derivative."""
+    ps = frhip.FRPSpace1D(0.0, 1.0, 8, 2)
+    vs = bgk.VSpace1D(-5.0, 5.0, 30)
+    f = np.zeros((8, 30, 3), order="F")
+    f[...] = (scale * np.exp(-(vs.u - 0.5) ** 2) * (1.0 + 0.5 * np.cos(2.0 * vs.u)))[None, :, None]
+    one, g = bgk.BGK1D(ps, vs, tau=1.0), bgk.BGK1D(ps, vs, tau=tau)
+    ref = one.rhs(f)  # M - f and the derivative's rounding
+    with np.errstate(over="ignore"):
+        want = ref / tau
+    if path == "rhs":
+        got = g.rhs(f)
+    else:  # u + dt du with u lost in dt du wherever that is infinite
+        g.set_path(path)
+        g.set_state(f)
+        g.step(1.0, 1, "euler")
+        with np.errstate(over="ignore"):
+            want = f + want
+        got = g.get_state()
+    assert not np.isnan(got).any()
+    # the derivative of a constant: some 30 roundings of values of at most 5 scale 2 / dx = 80 scale
+    slack = 1e-12 * scale
+    most = np.finfo(float).max * min(tau, 1.0)
+    big, small = np.abs(ref) > 1.01 * most, np.abs(ref) < 0.99 * most
+    assert big.any() == (tau < 1e-300) and small.any()
+    assert np.array_equal(got[big], want[big])
+    clear = small & (np.abs(ref) > 1e-6 * scale)  # M - f itself to 1e-6
+    assert clear.sum() > 100
+    assert np.all(np.abs(got - want)[clear] <= 1e-5 * np.abs(want[clear]) + slack)
