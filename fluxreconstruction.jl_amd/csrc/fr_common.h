@@ -303,16 +303,17 @@ __device__ __forceinline__ bool shock_switch(double Se, double S0, double kappa)
 }
 
 // The energy ratio at which the switch flips: sigma falls with Se, and is 0.99 where the sine is
-// -0.98.  NaN when it is out of the range in which shock_flagged may compare against it.
+// -0.98.  NaN when it is out of the range in which shock_flagged may compare against it: the long form
+// rounds Se - S0 and the sine, at |S0| or kappa = 1e4 by a relative 1e-11 of the ratio and at 1e8 by 1e-8.
 inline double shock_cut(double S0, double kappa) {
   const double q = std::pow(10.0, S0 - kappa * (2.0 / M_PI) * std::asin(0.98));
-  return kappa >= 0.0 && q > 1e-100 && q < 1e100 ? q : std::nan("");
+  return std::fabs(S0) <= 1e4 && kappa >= 0.0 && kappa <= 1e4 && q > 1e-100 && q < 1e100 ? q : std::nan("");
 }
 
 // shock_switch(log10(top / all), S0, kappa) with q = shock_cut(S0, kappa): the logarithm and the sine
 // are evaluated only within a relative 1e-9 of the cut, a margin far above the rounding errors of
-// the long form (a relative 1e-14 of the ratio), and for values out of range (all not above 1e-150,
-// NaN).  So the outcome is the long form's on every input.
+// the long form, and for values out of range (all not above 1e-150, NaN).  So the outcome is the long
+// form's on every input.
 __device__ __forceinline__ bool shock_flagged(double top, double all, double q, double S0, double kappa) {
   if (all > 1e-150) {
     if (top < q * (1.0 - 1e-9) * all) return false;

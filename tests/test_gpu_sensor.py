@@ -174,3 +174,36 @@ def test_fused_pass_with_active_limiter(deg, mode, rule):
     assert np.all(np.isfinite(out["fused"]))
     assert not np.array_equal(out["unfused"], out["no_limiter"])  # the limiter corrected cells
     assert np.array_equal(out["fused"], out["unfused"])
+
+
+@pytest.mark.parametrize("deg", [2, 3, 4])
+@pytest.mark.parametrize("kappa", [9.0, 100.0, 1e4, 1e6, 1e8])
+def test_switch_by_the_cut_is_the_long_form(deg, kappa):
+    """Cells whose top mode lies a relative 1e-11 ... 1e-3 of the energy ratio on either side of the cut: the
+    filter passes (which compare the ratio with the cut) flag as many as the evaluation (which takes the
+    logarithm and the sine), and with the script's S0 and kappa those above the cut.  For the larger kappa
+    S0 is shifted so that the cut is where the cells are."""
+    c = 2.0 / np.pi * np.arcsin(0.98)
+    S0 = -3.0 * np.log10(deg) if kappa == 9.0 else kappa * c - 4.0
+    cut = 10.0 ** (S0 - kappa * c)
+    delta = np.geomspace(1e-11, 1e-3, 300)
+    r, _ = np.polynomial.legendre.leggauss(deg + 1)
+    P = np.polynomial.legendre.legvander(r, deg) * np.sqrt((2 * np.arange(deg + 1) + 1) / 2)
+    low, high = np.outer(P[:, 0], P[:, 0]), np.outer(P[:, deg], P[:, deg])
+    for sign in (1.0, -1.0):
+        q = cut * (1 + sign * delta)
+        ps = frhip.FRPSpace2D(0.0, 1.0, delta.size, 0.0, 1.0, 1, deg, 1, 1)
+        u = np.zeros((delta.size + 2, 3, deg + 1, deg + 1, 4), order="F")
+        u[..., 0] = 1.3 * low
+        u[1:-1, 1, :, :, 0] += 1.3 * np.sqrt(q / (1 - q))[:, None, None] * high
+        u[..., 3] = 2.5
+        sol = frhip.FREuler2D(ps, 1.4, "hll", "ghost")
+        sol.set_state(u)
+        want = int((S.sensor_eval(sol, "modal", S0=S0, kappa=kappa) > 0).sum())
+        n = [sol.sensor_filter("modal", 1e-4, S0, kappa)]
+        sol.set_state(u)
+        n.append(sol.filter_refresh_limit("modal", 1e-4, S0, kappa))
+        sol.close()
+        assert n == [want, want], (sign, n, want)
+        if kappa == 9.0:
+            assert want == (delta.size if sign > 0 else 0)
