@@ -1036,8 +1036,10 @@ int fr1d_create(fr1d_ctx **out, const fr1d_desc *d) {
   c->gamma = d->gamma;
   c->a = d->a;
   c->correction = d->correction;
-  c->probs.push_back(Prob1D{0, d->ncell, d->deg + 1, 2.0 / d->dx, member_cut(d->deg)});
-  int rc = c->build(d->flux, d->equation);
+  int rc = no_throw("fr1d_create", [&] {
+    c->probs.push_back(Prob1D{0, d->ncell, d->deg + 1, 2.0 / d->dx, member_cut(d->deg)});
+    return c->build(d->flux, d->equation);
+  });
   if (rc) {
     c->release();
     delete c;
@@ -1133,8 +1135,11 @@ int fr_ens_create(fr_ens_ctx **out, int nprob, const int *ncell, const int *deg,
   FR_REQUIRE(c, FR_E_NOMEM, "fr_ens_create: out of host memory");
   c->bc = bc;
   c->gamma = gamma;
-  for (int b = 0; b < nprob; ++b) c->probs.push_back(Prob1D{0, ncell[b], deg[b] + 1, 2.0 / dx[b], member_cut(deg[b])});
-  int rc = c->build(flux, FR_EQ_EULER);
+  int rc = no_throw("fr_ens_create", [&] {
+    for (int b = 0; b < nprob; ++b)
+      c->probs.push_back(Prob1D{0, ncell[b], deg[b] + 1, 2.0 / dx[b], member_cut(deg[b])});
+    return c->build(flux, FR_EQ_EULER);
+  });
   if (rc) {
     c->release();
     delete c;

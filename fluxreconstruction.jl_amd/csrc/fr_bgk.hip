@@ -18,7 +18,6 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
-#include <exception>
 #include <new>
 #include <type_traits>
 #include <utility>
@@ -783,9 +782,14 @@ int fr_bgk_create(fr_bgk_ctx **out, const fr_bgk_desc *d) {
   c->dx = d->dx;
   c->dy = d->dy;
   c->gamma = d->gamma;
-  if (!build_ops(d->deg, FR_CORR_RADAU, c->ops)) {
+  int rc = no_throw("fr_bgk_create", [&] {
+    return build_ops(d->deg, FR_CORR_RADAU, c->ops)
+               ? (int)FR_OK
+               : fail(FR_E_INVALID, "fr_bgk_create: operator construction failed");
+  });
+  if (rc) {
     delete c;
-    return fail(FR_E_INVALID, "fr_bgk_create: operator construction failed");
+    return rc;
   }
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess ||
@@ -795,16 +799,18 @@ int fr_bgk_create(fr_bgk_ctx **out, const fr_bgk_desc *d) {
   const BgkGeo &g = c->geom;
   c->len = (size_t)g.mstride * d->nmem;
   std::vector<double> vel;
-  vel.insert(vel.end(), d->u, d->u + d->nu);
-  vel.insert(vel.end(), d->v, d->v + d->nv);
-  vel.insert(vel.end(), d->wu, d->wu + d->nu);
-  vel.insert(vel.end(), d->wv, d->wv + d->nv);
   std::vector<BgkVel> vt;  // of the stage kernel alone
-  try {
+  rc = no_throw("fr_bgk_create", [&] {
+    vel.insert(vel.end(), d->u, d->u + d->nu);
+    vel.insert(vel.end(), d->v, d->v + d->nv);
+    vel.insert(vel.end(), d->wu, d->wu + d->nu);
+    vel.insert(vel.end(), d->wv, d->wv + d->nv);
     if (c->large()) vt.reserve((size_t)d->nu * d->nv);
-  } catch (const std::exception &) {
+    return (int)FR_OK;
+  });
+  if (rc) {
     delete c;
-    return fail(FR_E_NOMEM, "fr_bgk_create: out of host memory");
+    return rc;
   }
   for (int b = 0; c->large() && b < d->nv; ++b)
     for (int a = 0; a < d->nu; ++a) {
@@ -826,7 +832,7 @@ int fr_bgk_create(fr_bgk_ctx **out, const fr_bgk_desc *d) {
   if (e == hipSuccess) e = hipMalloc(&c->d_tab, (size_t)g.npts * (d->nu + d->nv) * d->nmem * sizeof(double));
   if (e == hipSuccess) e = hipMalloc(&c->d_u, c->len * sizeof(double));
   if (e != hipSuccess) {
-    int rc = hip_fail(e, "fr_bgk_create", __FILE__, __LINE__);
+    rc = hip_fail(e, "fr_bgk_create", __FILE__, __LINE__);
     c->release();
     delete c;
     return rc;

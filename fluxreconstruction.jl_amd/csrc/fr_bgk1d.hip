@@ -682,14 +682,27 @@ int fr_bgk1d_create(fr_bgk1d_ctx **out, const fr_bgk1d_desc *d) {
   c->dx = d->dx;
   c->gamma = d->gamma;
   for (int m = 0; m < d->nmem; ++m) c->divide = c->divide || d->tau[m] < kTauDivide;
-  if (!build_ops(d->deg, FR_CORR_RADAU, c->ops)) {
+  int rc = no_throw("fr_bgk1d_create", [&] {
+    return build_ops(d->deg, FR_CORR_RADAU, c->ops)
+               ? (int)FR_OK
+               : fail(FR_E_INVALID, "fr_bgk1d_create: operator construction failed");
+  });
+  if (rc) {
     delete c;
-    return fail(FR_E_INVALID, "fr_bgk1d_create: operator construction failed");
+    return rc;
   }
   const Bgk1dGeo g = c->geo();
   c->len = (size_t)g.mstride * d->nmem;
-  std::vector<double> vel(d->u, d->u + d->nu);
-  vel.insert(vel.end(), d->w, d->w + d->nu);
+  std::vector<double> vel;
+  rc = no_throw("fr_bgk1d_create", [&] {
+    vel.insert(vel.end(), d->u, d->u + d->nu);
+    vel.insert(vel.end(), d->w, d->w + d->nu);
+    return (int)FR_OK;
+  });
+  if (rc) {
+    delete c;
+    return rc;
+  }
   hipError_t e = hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking);
   if (e == hipSuccess) e = hipEventCreateWithFlags(&c->ev, hipEventDisableTiming);
   if (e == hipSuccess) e = hipMalloc(&c->d_vel, vel.size() * sizeof(double));
@@ -699,7 +712,7 @@ int fr_bgk1d_create(fr_bgk1d_ctx **out, const fr_bgk1d_desc *d) {
   if (e == hipSuccess) e = hipMalloc(&c->d_prim, (size_t)g.npts * 4 * d->nmem * sizeof(double));
   if (e == hipSuccess) e = hipMalloc(&c->d_u, c->len * sizeof(double));
   if (e != hipSuccess) {
-    int rc = hip_fail(e, "fr_bgk1d_create", __FILE__, __LINE__);
+    rc = hip_fail(e, "fr_bgk1d_create", __FILE__, __LINE__);
     c->release();
     delete c;
     return rc;
@@ -839,7 +852,12 @@ int fr_bgk1d_moments(fr_bgk1d_ctx *c, double *w) {
   const Bgk1dGeo g = c->geo();
   int rc = c->launch_moments(c->d_u, c->stream);
   if (rc) return rc;
-  std::vector<double> prim((size_t)g.npts * 4 * c->nmem);
+  std::vector<double> prim;
+  rc = no_throw("fr_bgk1d_moments", [&] {
+    prim.resize((size_t)g.npts * 4 * c->nmem);
+    return (int)FR_OK;
+  });
+  if (rc) return rc;
   FR_HIP(hipMemcpyAsync(prim.data(), c->d_prim, prim.size() * sizeof(double), hipMemcpyDeviceToHost, c->stream));
   FR_HIP(hipStreamSynchronize(c->stream));
   for (long long mem = 0; mem < c->nmem; ++mem)

@@ -6,6 +6,7 @@
 #include <cmath>
 #include <cstddef>
 #include <cstdint>
+#include <exception>
 #include <string>
 
 #include "../../include/fr.h"
@@ -30,6 +31,16 @@ int hip_fail(hipError_t e, const char *what, const char *file, int line);
 
 // A kernel launch is checked with hipGetLastError right after it.
 #define FR_LAUNCHED(name) FR_HIP(hipGetLastError())
+
+// f() with an exception of its host allocations as FR_E_NOMEM: none leaves a C entry
+template <class F>
+int no_throw(const char *who, F &&f) {
+  try {
+    return f();
+  } catch (const std::exception &) {
+    return fail(FR_E_NOMEM, std::string(who) + ": out of host memory");
+  }
+}
 
 // ------------------------------------------------------------------ host arrays
 // Pinned chunks that a context's large copies to and from pageable host arrays go through
