@@ -1228,9 +1228,11 @@ int fr_ens_run_graph(fr_ens_ctx *c, int opts, double dt, int nsteps, int nrep, i
   if (rc) return rc;
   if (!c->d_count) FR_HIP(hipMalloc(&c->d_count, 2 * sizeof(int)));
   // The graph holds the context's own buffers and work lists, which never move once allocated, so a
-  // capture stays valid while the options, dt, the step count and the work mapping are unchanged.
-  if (!(c->gexec && c->g_opts == opts && c->g_dt == dt && c->g_nsteps == nsteps && c->g_threads == c->threads &&
-        c->g_grid == c->grid && c->g_path == c->path)) {
+  // capture stays valid while the options, dt, the step count, the path and, where a launch per stage is
+  // captured, the work mapping are unchanged.
+  const int scheme = (opts & FR_ENS_MIDPOINT) ? FR_RK_MIDPOINT : FR_RK_SSPRK3;
+  const bool same_map = c->use_blocks(scheme, 0) || (c->g_threads == c->threads && c->g_grid == c->grid);
+  if (!(c->gexec && c->g_opts == opts && c->g_dt == dt && c->g_nsteps == nsteps && same_map && c->g_path == c->path)) {
     if (c->gexec) {
       FR_HIP(hipStreamSynchronize(c->stream));
       (void)hipGraphExecDestroy(c->gexec);
@@ -1238,7 +1240,7 @@ int fr_ens_run_graph(fr_ens_ctx *c, int opts, double dt, int nsteps, int nrep, i
     }
     hipGraph_t graph = nullptr;
     FR_HIP(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
-    rc = c->run_steps((opts & FR_ENS_MIDPOINT) ? FR_RK_MIDPOINT : FR_RK_SSPRK3, 0, dt, nsteps, c->stream, opts);
+    rc = c->run_steps(scheme, 0, dt, nsteps, c->stream, opts);
     hipError_t e = hipStreamEndCapture(c->stream, &graph);
     if (rc) {
       if (graph) (void)hipGraphDestroy(graph);
@@ -1269,8 +1271,8 @@ int fr_ens_step_graph(fr_ens_ctx *c, double dt, int nsteps, int nrep) {
   return fr_ens_run_graph(c, 0, dt, nsteps, nrep, nullptr, nullptr);
 }
 
-// Times candidate (threads per workgroup, grid) mappings with HIP events over a few SSP-RK3
-// steps on a scratch copy of the state, keeps the fastest, and restores the state.
+// Times candidate (threads per workgroup, grid) mappings of the launches per stage with HIP events over a
+// few SSP-RK3 steps on a scratch copy of the state, keeps the fastest, and restores the state.
 int fr_ens_autotune(fr_ens_ctx *c, double dt, int *chosen) {
   FR_REQUIRE(c && std::isfinite(dt), FR_E_INVALID, "fr_ens_autotune: bad arguments");
   int rc = c->ensure_stage_buffers(false);

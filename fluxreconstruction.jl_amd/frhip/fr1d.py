@@ -290,6 +290,9 @@ class Ensemble1D:
         return n.value
 
     def autotune(self, dt: float) -> int:
+        """Times the work mappings of the launches per stage (set_path('batched'); looped steps take
+        their threads), keeps the fastest and returns its index; the register-resident steps of the other
+        paths have one mapping."""
         c = C.c_int(-1)
         check(_lib.lib().fr_ens_autotune(self.h, float(dt), C.byref(c)))
         return c.value

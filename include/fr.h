@@ -396,10 +396,12 @@ int fr_ens_step_graph(fr_ens_ctx *ctx, double dt, int nsteps, int nrep);
  * mean density is not positive is left unchanged and reported as FR_E_LIMITER after the loop. */
 enum { FR_ENS_FILTER = 1, FR_ENS_LIMIT = 2, FR_ENS_MIDPOINT = 4 };
 int fr_ens_run(fr_ens_ctx *ctx, int mode, int opts, double dt, int nsteps, int *n_flagged, int *n_limited);
-/* the batched loop of nsteps steps captured in a hipGraph (kept while opts, dt, nsteps and the
- * work mapping are unchanged, so later calls only replay it) and replayed nrep times */
+/* the loop of nsteps steps captured in a hipGraph (kept while opts, dt, nsteps, the path and, on
+ * FR1D_PATH_BATCHED, the work mapping are unchanged, so later calls only replay it) and replayed nrep times */
 int fr_ens_run_graph(fr_ens_ctx *ctx, int opts, double dt, int nsteps, int nrep, int *n_flagged, int *n_limited);
-/* time candidate work mappings on the device and keep the fastest; returns its index */
+/* time candidate work mappings of the launches per stage (FR1D_PATH_BATCHED; mode 1 takes their threads) on
+ * the device, keep the fastest and return its index, 0..14.  The register-resident steps that
+ * FR1D_PATH_AUTO and _MEMBER take have one mapping, which it does not touch. */
 int fr_ens_autotune(fr_ens_ctx *ctx, double dt, int *chosen);
 /* fr1d_sensor_filter / fr1d_positivity over every member (each with its own degree) */
 int fr_ens_sensor_filter(fr_ens_ctx *ctx, double dt, int *n_flagged);

@@ -1,5 +1,6 @@
 // The create calls of the 1D and BGK contexts against host allocations that fail one after another: every
-// failure is FR_E_NOMEM, no exception leaves the C entry.  The HIP runtime is a stand-in that succeeds.
+// failure is FR_E_NOMEM, no exception leaves the C entry; and when the ensemble's loop is captured anew.  The
+// HIP runtime is a stand-in that succeeds.
 #include <cstdio>
 #include <cstdlib>
 #include <new>
@@ -28,7 +29,8 @@ int hipStreamWaitEvent(P, P, unsigned) { return 0; }
 int hipStreamGetDevice(P, int *d) { return *d = 0, 0; }
 int hipStreamBeginCapture(P, int) { return 0; }
 int hipStreamEndCapture(P, P *) { return 0; }
-int hipGraphInstantiate(P *, P, P *, char *, size_t) { return 0; }
+int captures = 0;
+int hipGraphInstantiate(P *g, P, P *, char *, size_t) { return ++captures, *g = &captures, 0; }
 int hipGraphExecDestroy(P) { return 0; }
 int hipGraphDestroy(P) { return 0; }
 int hipGraphLaunch(P, P) { return 0; }
@@ -37,7 +39,8 @@ int hipEventCreateWithFlags(P *e, unsigned) { return *e = std::malloc(8), 0; }
 int hipEventDestroy(P e) { return std::free(e), 0; }
 int hipEventRecord(P, P) { return 0; }
 int hipEventSynchronize(P) { return 0; }
-int hipEventElapsedTime(float *ms, P, P) { return *ms = 1.0f, 0; }
+float elapsed = 1e6f;  // every timing beats the last one
+int hipEventElapsedTime(float *ms, P, P) { return *ms = --elapsed, 0; }
 int hipPointerGetAttributes(P, const void *) { return 1; }
 int hipFuncSetAttribute(const void *, int, int) { return 0; }
 int hipGetLastError(void) { return 0; }
@@ -101,6 +104,20 @@ int main() {
     fr_ens_destroy(c);
     return rc;
   });
+  // a captured loop of register-resident steps outlives a new mapping of the launches per stage
+  for (int path : {FR1D_PATH_AUTO, FR1D_PATH_BATCHED}) {
+    fr_ens_ctx *c = nullptr;
+    int choice = -1;
+    bool ok = fr_ens_create(&c, 300, n.data(), deg.data(), dx.data(), 1.4, FR_FLUX_HLL, FR_BC1_PERIOD) == FR_OK;
+    ok = ok && fr_ens_set_path(c, path) == FR_OK;
+    captures = 0;
+    for (int r = 0; r < 2; ++r) ok = ok && fr_ens_run_graph(c, FR_ENS_FILTER, 1e-3, 3, 1, nullptr, nullptr) == FR_OK;
+    ok = ok && captures == 1 && fr_ens_autotune(c, 1e-3, &choice) == FR_OK && choice == 14;
+    ok = ok && fr_ens_run_graph(c, FR_ENS_FILTER, 1e-3, 3, 1, nullptr, nullptr) == FR_OK;
+    ok = ok && captures == (path == FR1D_PATH_AUTO ? 1 : 2);
+    fr_ens_destroy(c);
+    if (!ok) std::printf("FAIL path %d: %d captures\n", path, captures), ++bad;
+  }
   std::vector<double> v(64, 1.0), tau(2, 0.1);
   for (int cells : {8, 80}) {  // 80 x 80 x 64 x 64 velocities: the path of large states
     fr_bgk_desc d{};
