@@ -719,11 +719,11 @@ struct BgkCtx {
     return FR_OK;
   }
 
-  // whether the stage kernel serves: kBgkStream, bgk_fill, and a velocity's plane of points below the 4 GiB
-  // that its offsets reach
+  // whether the stage kernel serves: kBgkStream, bgk_fill, a velocity's plane of points below the 4 GiB that
+  // its offsets reach, and points that the closure, with four threads for each, can launch (2^32 threads)
   bool large() const {
     const size_t bytes = len * sizeof(double);
-    if (bytes <= kBgkStream || geom.npts >= (1LL << 29)) return false;
+    if (bytes <= kBgkStream || geom.npts >= (1LL << 29) || geom.npts * nmem >= (1LL << 30)) return false;
     if (nx > BT || ny > BT || (long long)nu * nv > kBgkFewVel) return true;
     const int bc = nsp <= 3 ? kBgkCells<3> : nsp == 4 ? kBgkCells<4> : kBgkCells<5>;
     const long long tiles = bgk_tiles(bc, geom.tsh);

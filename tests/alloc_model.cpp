@@ -1,6 +1,6 @@
 // The create calls of the 1D and BGK contexts against host allocations that fail one after another: every
-// failure is FR_E_NOMEM, no exception leaves the C entry; and when the ensemble's loop is captured anew.  The
-// HIP runtime is a stand-in that succeeds.
+// failure is FR_E_NOMEM, no exception leaves the C entry; when the ensemble's loop is captured anew; and the
+// sizes of launches.  The HIP runtime is a stand-in that succeeds.
 #include <cstdio>
 #include <cstdlib>
 #include <new>
@@ -43,12 +43,20 @@ float elapsed = 1e6f;  // every timing beats the last one
 int hipEventElapsedTime(float *ms, P, P) { return *ms = --elapsed, 0; }
 int hipPointerGetAttributes(P, const void *) { return 1; }
 int hipFuncSetAttribute(const void *, int, int) { return 0; }
-int hipGetLastError(void) { return 0; }
+int last_error = 0;
+int hipGetLastError(void) {
+  const int e = last_error;
+  return last_error = 0, e;
+}
 const char *hipGetErrorString(int) { return ""; }
 struct Dim { unsigned x, y, z; };
-int hipLaunchKernel(const void *, Dim, Dim, P *, size_t, P) { return 0; }
-unsigned __hipPushCallConfiguration(Dim, Dim, size_t, P) { return 0; }
-int __hipPopCallConfiguration(Dim *, Dim *, size_t *, P *) { return 0; }
+// a launch has fewer than 2^32 threads
+int hipLaunchKernel(const void *, Dim g, Dim b, P *, size_t, P) {
+  return last_error = (unsigned long long)g.x * b.x < 1ull << 32 ? 0 : 9;
+}
+Dim grid, block;
+unsigned __hipPushCallConfiguration(Dim g, Dim b, size_t, P) { return grid = g, block = b, 0; }
+int __hipPopCallConfiguration(Dim *g, Dim *b, size_t *lds, P *st) { return *g = grid, *b = block, *lds = 0, *st = nullptr, 0; }
 P *__hipRegisterFatBinary(const void *) { return nullptr; }
 void __hipUnregisterFatBinary(P *) {}
 void __hipRegisterFunction(P *, const void *, char *, const char *, int, P, P, P, P, int *) {}
@@ -129,6 +137,16 @@ int main() {
       fr_bgk_destroy(c);
       return rc;
     });
+  }
+  {  // 2^30 points in planes of 2^27, four velocities: every launch of a step within the runtime's limit
+    fr_bgk_desc d{};
+    d.nx = 8192, d.ny = 4096, d.deg = 1, d.nu = d.nv = 2, d.nmem = 8, d.dx = d.dy = 0.1, d.gamma = 2.0;
+    std::vector<double> taus(8, 0.1);
+    d.u = d.v = d.wu = d.wv = v.data(), d.tau = taus.data();
+    fr_bgk_ctx *c = nullptr;
+    const bool ok = fr_bgk_create(&c, &d) == FR_OK && fr_bgk_step(c, 1e-3, 1) == FR_OK;
+    fr_bgk_destroy(c);
+    if (!ok) std::printf("FAIL fr_bgk_step of 2^30 points\n"), ++bad;
   }
   fr_bgk1d_desc d{};
   d.nx = 20, d.deg = 2, d.nu = 64, d.nmem = 2, d.dx = 0.1, d.gamma = 3.0;

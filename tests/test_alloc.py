@@ -1,5 +1,6 @@
-"""Host allocations that fail inside the create calls, one after another (alloc_model.cpp: the library's host
-code, compiled for the host alone, on a stand-in of the HIP runtime): FR_E_NOMEM, no exception."""
+"""The library's host code, compiled for the host alone, on a stand-in of the HIP runtime (alloc_model.cpp): host
+allocations that fail inside the create calls, one after another (FR_E_NOMEM, no exception), captures that
+are kept, launch sizes."""
 import os
 import subprocess
 
