@@ -101,7 +101,7 @@ static __global__ __launch_bounds__(256) void fr2d_pitch_copy_kernel(double *__r
                                                                      int w, long long nrow) {
   constexpr int U = 8;
   const int lane = threadIdx.x & 63;
-  const long long r = blockIdx.x * 4LL + (threadIdx.x >> 6);
+  const long long r = (blockIdx.y * (long long)gridDim.x + blockIdx.x) * 4 + (threadIdx.x >> 6);
   if (r >= nrow) return;
   const double *s = src + sp * r;
   double *d = dst + dp * r;
@@ -118,7 +118,9 @@ static __global__ __launch_bounds__(256) void fr2d_pitch_copy_kernel(double *__r
 
 static int pitch_copy(const Fr2dCtx &c, double *dst, long long dp, const double *src, long long sp, hipStream_t st) {
   const long long nrow = (long long)(c.ny + 2) * c.nsp * c.nsp * 4;
-  hipLaunchKernelGGL(fr2d_pitch_copy_kernel, dim3((unsigned)((nrow + 3) / 4)), dim3(256), 0, st, dst, dp, src, sp,
+  // one direction of a launch has fewer than 2^32 threads
+  const long long blocks = (nrow + 3) / 4, bx = std::min(blocks, 1LL << 23), by = (blocks + bx - 1) / bx;
+  hipLaunchKernelGGL(fr2d_pitch_copy_kernel, dim3((unsigned)bx, (unsigned)by), dim3(256), 0, st, dst, dp, src, sp,
                      c.nx + 2, nrow);
   FR_LAUNCHED("fr2d_pitch_copy_kernel");
   return FR_OK;

@@ -42,6 +42,8 @@ int hipEventSynchronize(P) { return 0; }
 float elapsed = 1e6f;  // every timing beats the last one
 int hipEventElapsedTime(float *ms, P, P) { return *ms = --elapsed, 0; }
 int hipPointerGetAttributes(P, const void *) { return 1; }
+int hipGetSymbolAddress(P *p, const void *) { return *p = std::malloc(8), 0; }
+void __hipRegisterVar(P *, P, char *, char *, int, size_t, int, int) {}
 int hipFuncSetAttribute(const void *, int, int) { return 0; }
 int last_error = 0;
 int hipGetLastError(void) {
@@ -147,6 +149,16 @@ int main() {
     const bool ok = fr_bgk_create(&c, &d) == FR_OK && fr_bgk_step(c, 1e-3, 1) == FR_OK;
     fr_bgk_destroy(c);
     if (!ok) std::printf("FAIL fr_bgk_step of 2^30 points\n"), ++bad;
+  }
+  {  // a strip of two million rows of cells, p = 2: 72 million rows of values between the two layouts
+    fr2d_desc d{};
+    d.nx = 1, d.ny = 2000000, d.deg = 2, d.gamma = 1.4, d.iJ11 = d.iJ22 = 1.0;
+    fr2d_ctx *c = nullptr;
+    double u = 0.0;
+    const bool ok = fr2d_create(&c, &d) == FR_OK && fr2d_set_state_dev(c, &u) == FR_OK &&
+                    fr2d_get_state_dev(c, &u) == FR_OK;
+    fr2d_destroy(c);
+    if (!ok) std::printf("FAIL 2D state copies of 72 million rows\n"), ++bad;
   }
   fr_bgk1d_desc d{};
   d.nx = 20, d.deg = 2, d.nu = 64, d.nmem = 2, d.dx = 0.1, d.gamma = 3.0;
