@@ -116,12 +116,40 @@ static __global__ __launch_bounds__(256) void fr2d_pitch_copy_kernel(double *__r
   }
 }
 
+// The same for rows of at most 32 values: 64 / L of them side by side in a wavefront, L the power of two that
+// holds one, and eight such groups in flight.  With a wavefront per row / here / hipMemcpy2DAsync: 50000 rows
+// of cells, rows of 3 values, p = 3 400 / 143 / 138 us; of 7, p = 2 232 / 81 / 81; 30000 of 16, p = 3 270 / 89 /
+// 181; 20000 of 32 203 / 117 / 237.  Rows of 33 to 63: 207 / - / 291.
+static __global__ __launch_bounds__(256) void fr2d_narrow_copy_kernel(double *__restrict__ dst, long long dp,
+                                                                      const double *__restrict__ src, long long sp,
+                                                                      int w, long long nrow, int log2l) {
+  constexpr int U = 8;
+  const int lane = threadIdx.x & 63, i = lane & ((1 << log2l) - 1), side = 64 >> log2l;
+  const long long wave = (blockIdx.y * (long long)gridDim.x + blockIdx.x) * 4 + (threadIdx.x >> 6);
+  const long long r = wave * (U * side) + (lane >> log2l);
+  if (i >= w) return;
+  double v[U];
+#pragma unroll
+  for (int q = 0; q < U; ++q)
+    if (r + q * side < nrow) v[q] = src[sp * (r + q * side) + i];
+#pragma unroll
+  for (int q = 0; q < U; ++q)
+    if (r + q * side < nrow) dst[dp * (r + q * side) + i] = v[q];
+}
+
 static int pitch_copy(const Fr2dCtx &c, double *dst, long long dp, const double *src, long long sp, hipStream_t st) {
   const long long nrow = (long long)(c.ny + 2) * c.nsp * c.nsp * 4;
+  const int w = c.nx + 2;
+  int log2l = 2;
+  while (log2l < 6 && (1 << log2l) < w) ++log2l;
+  const long long per = log2l < 6 ? 4 * 8 * (64 >> log2l) : 4;  // rows per workgroup
   // one direction of a launch has fewer than 2^32 threads
-  const long long blocks = (nrow + 3) / 4, bx = std::min(blocks, 1LL << 23), by = (blocks + bx - 1) / bx;
-  hipLaunchKernelGGL(fr2d_pitch_copy_kernel, dim3((unsigned)bx, (unsigned)by), dim3(256), 0, st, dst, dp, src, sp,
-                     c.nx + 2, nrow);
+  const long long blocks = (nrow + per - 1) / per, bx = std::min(blocks, 1LL << 23), by = (blocks + bx - 1) / bx;
+  const dim3 grid((unsigned)bx, (unsigned)by);
+  if (log2l < 6)
+    hipLaunchKernelGGL(fr2d_narrow_copy_kernel, grid, dim3(256), 0, st, dst, dp, src, sp, w, nrow, log2l);
+  else
+    hipLaunchKernelGGL(fr2d_pitch_copy_kernel, grid, dim3(256), 0, st, dst, dp, src, sp, w, nrow);
   FR_LAUNCHED("fr2d_pitch_copy_kernel");
   return FR_OK;
 }

@@ -25,3 +25,11 @@ def test_state_device_round_trip(nx, ny, deg):
     assert frhip.lib().fr2d_get_state_dev(s.h, out.data_ptr()) == 0
     assert torch.equal(out, u + 1.0)
     s.close()
+
+
+# rows of 3 to 33 values: 16, 8, 4 and 2 of them side by side in a wavefront, and the first that has one to
+# itself; row counts that end inside a group
+@pytest.mark.parametrize("nx,ny,deg", [(1, 77, 1), (2, 1, 1), (3, 130, 2), (6, 41, 1), (7, 9, 3), (14, 33, 2), (15, 5, 1),
+                                       (30, 18, 1), (31, 6, 2), (1, 3000, 5)])
+def test_narrow_state_device_round_trip(nx, ny, deg):
+    test_state_device_round_trip(nx, ny, deg)
