@@ -197,6 +197,13 @@ __global__ __launch_bounds__(256, 4) void fr2d_filter_refresh_limit_kernel(
         for (int a = 0; a < NP; ++a) ss += mod[a] * mod[a];
         top = mod[NP - 1] * mod[NP - 1];
       }
+      // From nsp = 5 on every lane forms its modes: left to itself the compiler moves them into the density
+      // lanes' branch, which took 83 us for 69 at p = 5, 1 x 3000, 45 for 40 at 37 x 41 and 33.7 for 32.3 at p = 4,
+      // 37 x 41; at p = 3 10 loop iterations at 512 x 256 take 1503 us so and 1518 with the modes kept out.
+      if constexpr (NSP >= 5) {
+        fr_pin(top);
+        fr_pin(ss);
+      }
       // the density lane decides for the quad; with the logarithm and the sine in every cell 10 loop
       // iterations took 308 us for 303 at 100 x 50, p = 2, and 1502 for 1491 at 512 x 256, p = 3
       lam = __shfl(r == 0 && shock_flagged(top, ss, cut, S0, kappa) ? 1 : 0, 0, 4) ? lambda : 0.0;
