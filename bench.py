@@ -117,7 +117,7 @@ def bench_bgk1d():
 
 def bench_fr1d_small():
     """The reference's small 1D runs (100 cells, p = 2, 1000 steps: advection RK4, Sod Midpoint)
-    with a launch per stage and on the per-member path (frhip.workloads)."""
+    with a launch per stage and register-resident (frhip.workloads)."""
     from frhip import workloads
 
     return {"workload": "1D FR 100 cells p=2, 1000 steps", "unit": "ms per run", **workloads.fr1d_small()}

@@ -119,8 +119,11 @@ __device__ __forceinline__ double row_shift(double x) {
 // counters) where LDS and registers allow two; with two tiles in a workgroup of ten (3, 3, 2, 2) ten are.
 // Per SSP-RK3 stage: 201 x 133, HLL 24.9 -> 19.1 us, 560 x 500, Rusanov 201 -> 176 us, Roe 223 -> 187, polar
 // cells 268 -> 231.  Grids of no more tiles than CUs keep one (every tile has a CU to itself: 20 x 14, seven
-// steps 305 us with one, 336 with two), and so does the RK4 form on point metrics, which would spill 50
-// values.  At nsp = 6 two tiles have to fit 168 VGPRs and spill: 466 x 500 239 -> 249 us, polar cells
+// steps 305 us with one, 336 with two), and so does the RK4 form on point metrics.  Two tiles spill there and
+// in the other RK4 forms (22 to 66 values) alike, but the others are faster with them all the same: ten RK4
+// steps, one / two tiles, 250 x 199, rectangles, HLL 2310 / 2017 us, Roe 2428 / 2288, parallelograms, HLL
+// 2386 / 2008; 560 x 500, rectangles, Rusanov 14362 / 13048, parallelograms, Roe 15232 / 14235; polar cells
+// 250 x 199 2582 / 2648, 300 x 200 2650 / 2976, 201 x 133 1367 / 1346.  At nsp = 6 two tiles have to fit 168 VGPRs and spill: 466 x 500 239 -> 249 us, polar cells
 // 289 -> 387.
 template <int NSP, int EPI, int GEO>
 constexpr int kTilesPerWg = NSP == 5 && !(EPI == EPI_ACC && GEO == GEO_POINT) ? 2 : 1;

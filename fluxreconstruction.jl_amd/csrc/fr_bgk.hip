@@ -8,8 +8,8 @@
 //
 // State f(i, j, k, l, a, b, member), column-major: the cell index is fastest, so a wavefront of
 // consecutive cells reads contiguous memory for a fixed (point, velocity).  Two paths:
-// - states that the caches serve (kBgkStream): moments (one thread per solution point, loop over the velocities, FP64
-//   sums; it also writes the separable Maxwellian factors of the point), then transport + relaxation +
+// - states that the caches serve, members of few cells, and points beyond what the other path's offsets and
+//   launches reach (BgkCtx::large): moments (one thread per solution point, loop over the velocities, FP64 sums; it also writes the separable Maxwellian factors of the point), then transport + relaxation +
 //   RK stage (one workgroup per (member, velocity, 16 x 16 cell tile), one thread per cell; the upwind
 //   traces of the neighbours come from LDS or from the halo threads);
 // - larger states: a stage kernel that walks a tile through a range of velocities and leaves partial

@@ -199,7 +199,7 @@ def FRAdvectionProblem(*args, **kwargs) -> FR1D:
 
 
 class Ensemble1D:
-    """Independent 1D Euler problems advanced together (one launch per SSP-RK3 stage).
+    """Independent 1D Euler problems advanced together (several steps of every member per launch).
     Member b: ncell[b] cells of degree deg[b] on a uniform grid of spacing dx[b]."""
 
     def __init__(self, ncell, deg, dx, gamma: float = 1.4, flux: str = "rusanov", bc: str = "dirichlet"):

@@ -373,7 +373,7 @@ int fr1d_positivity(fr1d_ctx *ctx, int *n_limited);
 typedef struct fr_ens_ctx fr_ens_ctx;
 /* nprob independent 1D Euler problems (layout of each member as fr1d); member b has ncell[b]
  * cells of degree deg[b] (1..8) and cell size dx[b].  No reference counterpart: the reference
- * runs one FREulerProblem per script; an ensemble advances many in one launch per stage. */
+ * runs one FREulerProblem per script; an ensemble advances many together. */
 int fr_ens_create(fr_ens_ctx **out, int nprob, const int *ncell, const int *deg, const double *dx,
                   double gamma, int flux, int bc);
 int fr_ens_destroy(fr_ens_ctx *ctx);
@@ -381,7 +381,7 @@ size_t fr_ens_state_len(const fr_ens_ctx *ctx);          /* total doubles over a
 size_t fr_ens_offset(const fr_ens_ctx *ctx, int member); /* first double of a member */
 int fr_ens_set_state(fr_ens_ctx *ctx, const double *u);  /* concatenated member states */
 int fr_ens_get_state(fr_ens_ctx *ctx, double *u);
-/* mode 0: one batched launch per stage; 1: one launch per member per stage (looped baseline) */
+/* mode 0: all members together (FR1D_PATH_*); 1: one launch per member per stage (looped baseline) */
 int fr_ens_step(fr_ens_ctx *ctx, int mode, double dt, int nsteps);
 /* the execution path of fr_ens_step / fr_ens_run (FR1D_PATH_*; see fr1d_set_path) */
 int fr_ens_set_path(fr_ens_ctx *ctx, int path);
@@ -391,7 +391,7 @@ int fr_ens_step_graph(fr_ens_ctx *ctx, double dt, int nsteps, int nrep);
  * or, with FR_ENS_MIDPOINT, the script's own Midpoint steps: FR_ENS_FILTER runs
  * fr1d_sensor_filter's sensor + filter (filter time step dt) on the state before every step;
  * FR_ENS_LIMIT runs positive_limiter (src/dissipation.jl:61-123) on the input of every stage.
- * mode 0: one batched launch per pass; 1: one launch per member per pass (looped baseline).
+ * mode 0: all members together (FR1D_PATH_*); 1: one launch per member per pass (looped baseline).
  * n_flagged / n_limited (optional) sum the filtered / limited cells over the loop.  A cell whose
  * mean density is not positive is left unchanged and reported as FR_E_LIMITER after the loop. */
 enum { FR_ENS_FILTER = 1, FR_ENS_LIMIT = 2, FR_ENS_MIDPOINT = 4 };
