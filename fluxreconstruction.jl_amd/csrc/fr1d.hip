@@ -568,9 +568,9 @@ __device__ __forceinline__ void block1d(const Prob1D &pb, const Blk1D &bk, const
 
 // Three wavefronts per SIMD in the plain form of degrees up to 4.  Roe, us with this bound / none, 512 members,
 // SSP-RK3: p = 1 476 / 504, p = 2 574 / 590, p = 3 676 / 701, p = 4, where it spills (93 registers), 766 / 745 and,
-// 2000 members of 257 to 600 cells with the filter, 1993 / 1436 (4580 with a launch per stage).  Degrees 5 to 8 run at
-// one or two wavefronts per SIMD and are ahead of a launch per stage as well: 1000 cells, SSP-RK3, p = 5, 7
-// and 8 0.23 to 0.24 of its time, 1024 members of 200 to 256 cells, p = 8 with the filter, 0.13.
+// 2000 members of 257 to 600 cells with the filter, 1993 / 1436 (4580 with a launch per stage).  Degrees 5 to
+// 8 run at one or two wavefronts per SIMD and are ahead of a launch per stage as well: 1000 cells, SSP-RK3,
+// p = 5, 7 and 8 0.23 to 0.24 of its time, 1024 members of 200 to 256 cells, p = 8 with the filter, 0.13.
 template <int EQ, int FLUX, int NMAX, int KIND>
 __global__ __launch_bounds__(kBlockT, (NMAX <= 5 && KIND == BLK_PLAIN ? 3 : 1)) void fr1d_block_kernel(const Prob1D *__restrict__ probs,
                                                              const Blk1D *__restrict__ blocks,

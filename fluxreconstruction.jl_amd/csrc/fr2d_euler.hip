@@ -123,8 +123,8 @@ __device__ __forceinline__ double row_shift(double x) {
 // in the other RK4 forms (22 to 66 values) alike, but the others are faster with them all the same: ten RK4
 // steps, one / two tiles, 250 x 199, rectangles, HLL 2310 / 2017 us, Roe 2428 / 2288, parallelograms, HLL
 // 2386 / 2008; 560 x 500, rectangles, Rusanov 14362 / 13048, parallelograms, Roe 15232 / 14235; polar cells
-// 250 x 199 2582 / 2648, 300 x 200 2650 / 2976, 201 x 133 1367 / 1346.  At nsp = 6 two tiles have to fit 168 VGPRs and spill: 466 x 500 239 -> 249 us, polar cells
-// 289 -> 387.
+// 250 x 199 2582 / 2648, 300 x 200 2650 / 2976, 201 x 133 1367 / 1346.  At nsp = 6 two tiles have to fit
+// 168 VGPRs and spill: 466 x 500 239 -> 249 us, polar cells 289 -> 387.
 template <int NSP, int EPI, int GEO>
 constexpr int kTilesPerWg = NSP == 5 && !(EPI == EPI_ACC && GEO == GEO_POINT) ? 2 : 1;
 

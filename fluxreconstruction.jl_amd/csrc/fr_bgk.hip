@@ -9,8 +9,8 @@
 // State f(i, j, k, l, a, b, member), column-major: the cell index is fastest, so a wavefront of
 // consecutive cells reads contiguous memory for a fixed (point, velocity).  Two paths:
 // - states that the caches serve, members of few cells, and points beyond what the other path's offsets and
-//   launches reach (BgkCtx::large): moments (one thread per solution point, loop over the velocities, FP64 sums; it also writes the separable Maxwellian factors of the point), then transport + relaxation +
-//   RK stage (one workgroup per (member, velocity, 16 x 16 cell tile), one thread per cell; the upwind
+//   launches reach (BgkCtx::large): moments (one thread per solution point, loop over the velocities, FP64 sums; it
+//   also writes the separable Maxwellian factors of the point), then transport + relaxation + RK stage (one workgroup per (member, velocity, 16 x 16 cell tile), one thread per cell; the upwind
 //   traces of the neighbours come from LDS or from the halo threads);
 // - larger states: a stage kernel that walks a tile through a range of velocities and leaves partial
 //   velocity sums of its result, and a closure that adds them per point and writes the factors, so no
@@ -295,11 +295,11 @@ constexpr bool kBgkSums = NSP < 5;
 constexpr size_t kBgkStream = 64u << 20;
 // Grids inside one 16 x 16 tile with up to kBgkFewVel velocities are then many members, and a workgroup per
 // member and velocity range leaves most lanes without a cell: the line rises as the share of lanes with
-// one falls, kBgkFill of bytes per share.  One step, cached path / this one, 70 and 300 MB, 12 x 12
+// one falls, bgk_fill of bytes per share.  One step, cached path / this one, 70 and 300 MB, 12 x 12
 // velocities: 1 x 1 cells, p = 2, 1.78 and 1.63 times as long here, 4 x 4 1.65 and 1.29, 6 x 6 1.36 and 1.02, 8 x 8
 // 1.20 and 0.89, 12 x 12 0.99 and 0.80; p = 3: 4 x 4 1.06 and 1.00, 6 x 6 0.85 and 0.65, 10 x 10 (two of its tiles)
-// 1.16 and 0.98; p = 4 0.2 to 0.7 everywhere.  With more velocities (few points, whose sums the cached path forms one after
-// another) 0.1 to 0.7: 1 x 1 cells, p = 2, 1079 x 1079 velocities 0.24, 8 x 8, p = 1, 202 x 202 0.24.
+// 1.16 and 0.98; p = 4 0.2 to 0.7 everywhere.  With more velocities (few points, whose sums the cached path forms
+// one after another) 0.1 to 0.7: 1 x 1 cells, p = 2, 1079 x 1079 velocities 0.24, 8 x 8, p = 1, 202 x 202 0.24.
 constexpr int kBgkFewVel = 48 * 48;
 constexpr size_t bgk_fill(int nsp, long long tiles) {
   return nsp >= 5 ? 0 : nsp == 4 && tiles == 1 ? 32u << 20 : 48u << 20;

@@ -29,10 +29,10 @@ from .space import CSpace2D, FRPSpace1D, FRPSpace2D
 def riemann_ensemble(steps=10, nprob=512, seed=2024):
     """nprob seeded 1D Euler Riemann problems (64..2048 cells, p in {2,3,4}, piecewise-constant
     data with the jump on a cell face), Rusanov, SSP-RK3, run as the reference's per-step loop
-    (example/euler_highlevel.jl:37-54: sensor + filter before every step): every
-    member stepped together (register-resident, several steps per launch; eager and as a hipGraph
-    captured during the warm-up; the tuner times launches per stage, whose threads looped takes) vs one
-    launch per member per pass."""
+    (example/euler_highlevel.jl:37-54: sensor + filter before every step): all members together
+    (register-resident, several steps per launch; eager and as a hipGraph captured during the
+    warm-up) vs one launch per member per pass (with the threads that the tuner of the launches per
+    stage picks)."""
     import torch
 
     ncell, deg, dx, members = ics.riemann_ensemble(nprob, seed=seed)
@@ -174,8 +174,7 @@ def bgk1d_script(steps=1000):
 
 def fr1d_small(steps=1000):
     """The reference's small 1D runs, wall time of the whole run on the batched path (a launch per
-    stage) and on the member path (register-resident: up to 4096 steps per launch), from
-    the same state; both end in the same bits:
+    stage) and on the member path (register-resident: up to 4096 steps per launch), from the same state; both end in the same bits:
     - advection, 100 cells, p = 2, RK4, dt = 0.1 dx (example/advection_lowlevel.jl's setup, 1000
       steps to t = 1);
     - Euler (HLL, Dirichlet), Sod's problem on 100 cells, p = 2, Midpoint, dt = 1e-4 (1000 steps)."""
